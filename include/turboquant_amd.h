@@ -293,7 +293,7 @@ int tq_mse_dequantize(const uint8_t* packed, const float* norms, int64_t num_vec
  * turboquant/quantizer.py:121-158, with turboquant/qjl.py:28-63): the MSE
  * quantizer at mse_bit_width = bit_width - 1 (1..3 here), then QJL on the unit
  * residual.  The two d x d QJL products (sign(S r) and S^T z) are plain GEMMs
- * left to the caller's BLAS; these two calls are the rest of the algorithm.
+ * left to the caller here; these two calls are the rest of the algorithm.
  *
  * tq_prod_quantize: tq_mse_quantize's outputs, plus the MSE read-back
  *   x_hat = tq_mse_dequantize(packed, norms) (same fp32 bits), the residual
@@ -343,6 +343,27 @@ int tq_prod_dequantize_qjl(const uint8_t* packed, const float* norms, const int8
                            int32_t padded_dim, int32_t mse_bit_width, const float* signs,
                            const float* centroids, const void* st_hi, const void* st_lo,
                            float* out, tq_stream_t stream);
+
+/*
+ * The same above padded_dim 128 (256, 512 or 1024), where S no longer fits a
+ * wave's registers: the row kernels of tq_prod_quantize / tq_prod_dequantize
+ * and the QJL product as a matrix-core kernel of its own.  Operands as above
+ * (halves [padded_dim, padded_dim]).  tq_prod_quantize_qjl_ws keeps the unit
+ * residual in `workspace` (16-byte aligned, tq_prod_workspace_bytes bytes) as
+ * fp16 halves; tq_prod_dequantize_qjl_ws forms z S in the rows of `out`.
+ */
+int64_t tq_prod_workspace_bytes(int64_t num_vectors, int32_t padded_dim);
+int tq_prod_quantize_qjl_ws(const float* x, int64_t num_vectors, int32_t dim, int32_t padded_dim,
+                            int32_t mse_bit_width, const float* signs, const float* boundaries,
+                            const float* centroids, const void* s_hi, const void* s_lo,
+                            uint8_t* packed, float* norms, int8_t* qjl_signs,
+                            float* residual_norms, void* workspace, int64_t workspace_bytes,
+                            tq_stream_t stream);
+int tq_prod_dequantize_qjl_ws(const uint8_t* packed, const float* norms, const int8_t* qjl_signs,
+                              const float* residual_norms, int64_t num_vectors, int32_t dim,
+                              int32_t padded_dim, int32_t mse_bit_width, const float* signs,
+                              const float* centroids, const void* st_hi, const void* st_lo,
+                              float* out, tq_stream_t stream);
 
 /*
  * Layer glue of the end-to-end harness, no counterpart in the

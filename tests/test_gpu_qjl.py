@@ -1,0 +1,111 @@
+"""The QJL products of TurboQuantProd above padded size 128 (tq_qjl.hip) at
+the edges of their tiles (128 vectors x 128 outputs, K steps of 32), odd row
+lengths and the smallest calls, against 64-bit products of the same operands;
+and the row kernels at row lengths off the float4 pieces."""
+import pytest
+import torch
+
+from turboquant_amd import algorithm as A
+from turboquant_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(129, 1), (200, 127), (256, 128), (257, 129), (384, 300), (513, 3), (512, 256),
+          (1000, 130), (1023, 129), (1024, 64)]
+
+
+def _prod(dim, bits, n):
+    q = A.TurboQuantProd(dim, bits, device="cuda:0", seed=5)
+    x = torch.randn((n, dim), generator=torch.Generator("cuda").manual_seed(dim + n),
+                    device="cuda") * 2.0
+    return q, x, q.mse.rotation.padded_dim, q.mse._host_tables()
+
+
+@pytest.mark.parametrize("dim,n", SHAPES)
+def test_quantize_signs_against_64_bits(dim, n):
+    bits = 2 + dim % 4
+    print(f"case: qjl quantize dim={dim} n={n} bits={bits}", flush=True)
+    q, x, pd, (bnd, cen) = _prod(dim, bits, n)
+    args = (x, pd, bits - 1, q.mse.rotation.signs, bnd, cen)
+    packed, norms, resid, rnorm = ops.prod_quantize(*args)
+    sh, sl, _, _ = q.qjl.halves(pd)
+    p2, n2, z, r2 = ops.prod_quantize_qjl_ws(*args, sh, sl)
+    assert torch.equal(p2, packed) and torch.equal(n2, norms) and torch.equal(r2, rnorm)
+    s64, r64 = q.qjl.S.double(), resid.double()
+    proj = r64 @ s64.t()
+    wrong = z != torch.where(proj >= 0, 1, -1)
+    # hi + lo holds S to 2^-23 and r to 2^-23, the product drops lo lo (2^-22),
+    # the sum of 3 K products rounds to 2^-24 each
+    bound = (r64.abs() @ s64.abs().t()) * (2.0 ** -21 + 3 * dim * 2.0 ** -24)
+    assert bool((proj.abs() <= bound)[wrong].all()), proj[wrong].abs().max().item()
+
+
+@pytest.mark.parametrize("dim,n", SHAPES)
+def test_dequantize_term_against_64_bits(dim, n):
+    """z S alone: norms of zero and a weight of 1, with signs and with any
+    other int8 values (the product is defined for them too)."""
+    print(f"case: qjl dequantize dim={dim} n={n}", flush=True)
+    q, x, pd, (bnd, cen) = _prod(dim, 4, n)
+    packed, _, _, _ = ops.prod_quantize(x, pd, 3, q.mse.rotation.signs, bnd, cen)
+    _, _, th, tl = q.qjl.halves(pd)
+    s64 = q.qjl.S.double()
+    zero = torch.zeros(n, device="cuda")
+    gamma = torch.full((n,), 1.0 / q.qjl.dequant_scale, device="cuda")
+    gen = torch.Generator("cuda").manual_seed(n)
+    for z in (torch.randint(0, 2, (n, dim), generator=gen, device="cuda", dtype=torch.int8) * 2 - 1,
+              torch.randint(-128, 128, (n, dim), generator=gen, device="cuda", dtype=torch.int8)):
+        got = ops.prod_dequantize_qjl_ws(packed, zero, z, gamma, dim, pd, 3,
+                                         q.mse.rotation.signs, cen, th, tl).double()
+        want = z.double() @ s64
+        bound = (z.double().abs() @ s64.abs()) * (2.0 ** -22 + (2 * dim + 4) * 2.0 ** -24)
+        assert bool(((got - want).abs() <= bound).all()), (got - want).abs().max().item()
+
+
+def test_dequantize_paths_agree_around_the_size_rule():
+    """One vector fewer than QJL_GEMM_MIN (the torch product) and that many:
+    the rows they share are within the roundings of both."""
+    q, x, pd, (bnd, cen) = _prod(200, 4, A.QJL_GEMM_MIN)
+    out = q.quantize(x)
+    many, few = q.dequantize(*out), q.dequantize(*[t[:-1] for t in out])
+    assert few.shape[0] == A.QJL_GEMM_MIN - 1
+    assert torch.allclose(many[:-1], few, rtol=1e-5, atol=1e-5 * few.abs().max().item())
+
+
+@pytest.mark.parametrize("dim", [50, 98, 130, 258, 514, 1002, 1023])
+def test_row_kernels_off_the_float4_pieces(dim):
+    n = 67
+    q, qc = (A.TurboQuantMSE(dim, 3, device=d, seed=2) for d in ("cuda:0", "cpu"))
+    x = torch.randn((n, dim), generator=torch.Generator().manual_seed(dim))
+    packed, norms = q.quantize(x.cuda())
+    pc, nc = qc.quantize(x)
+    same = (packed.cpu() == pc).all(-1)
+    assert same.float().mean().item() >= 0.95
+    assert torch.allclose(norms.cpu(), nc, rtol=1e-6)
+    assert torch.equal(q.dequantize(packed, norms).cpu(), qc.dequantize(packed.cpu(), norms.cpu()))
+
+
+def test_empty_batches_and_replaced_matrix():
+    q, x, pd, _ = _prod(300, 4, 40)
+    packed, norms, z, rnorm = q.quantize(x[:0])
+    assert packed.shape == (0, 256) and z.shape == (0, 300) and rnorm.shape == (0,)
+    before = q.quantize(x)[2]
+    q.qjl.S.neg_()  # written in place: the operand halves are made again
+    assert torch.equal(q.quantize(x)[2], -before)
+    q.qjl.S = -q.qjl.S
+    assert torch.equal(q.quantize(x)[2], before)
+
+
+def test_first_call_inside_a_graph():
+    """Operand halves made during a capture hold values only when the graph
+    runs: they are not kept for eager calls, and replays are right."""
+    q, x, _, _ = _prod(400, 3, 70)
+    q.mse._host_tables()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        z = q.quantize(x)[2]
+    eager = q.quantize(x)[2].clone()
+    for _ in range(3):
+        z.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(z, eager)

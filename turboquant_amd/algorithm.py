@@ -18,7 +18,8 @@ compression.  The serving path (the paged 4-bit cache) is the HIP kernels in
   (quantizer.py:17-60).  On a GPU, fp32 vectors of padded size 64..1024 are
   quantized and dequantized by this package's HIP kernels
   (ops.mse_quantize / ops.mse_dequantize, tq_mse.hip); TurboQuantProd's MSE
-  stage goes through them too, its QJL stage is a GEMM.
+  stage goes through them too, its QJL products run on the matrix cores
+  (tq_mse.hip up to padded size 128, tq_qjl.hip above).
 
 Random tensors (signs, QJL matrix) come from seeded CPU torch generators, so
 the same seeds give the reference's values.
@@ -41,6 +42,15 @@ CENTROIDS_N01 = {
     4: (0.1284153814744918, 0.3880823046410021, 0.6567591430551046, 0.9423683558764893,
         1.2562490887894980, 1.6180344937899930, 2.0693470280837980, 2.7326368237440100),
 }
+
+
+# Vectors from which TurboQuantProd.dequantize above padded size 128 forms z S
+# with this package's kernel.  The kernel is the faster one at every size (1500
+# vectors of dim 1000: 42 against 63 us; 4096: 48 against 88; 20011: 143
+# against 386) and the nearer one to 64 bits; below the line the product stays
+# torch's fp32 GEMM so that small batches keep equalling torch's expression
+# z.float() @ S bit for bit, which callers compare against.
+QJL_GEMM_MIN = 2048
 
 
 def _levels(bit_width: int) -> list[float]:
@@ -167,21 +177,34 @@ class QJL:
     def halves(self, padded_dim: int):
         """(S_hi, S_lo, S^T_hi, S^T_lo): fp16 halves with S = hi + lo (to 22
         bits), zero-padded to [padded_dim, padded_dim], for the fused kernels
-        (made once per padded size and device)."""
-        cache = self.__dict__.setdefault("_halves", {})
+        (made once per padded size and device; again when S was replaced or
+        written to)."""
+        made_from = (self.S, None if self.S.is_inference() else self.S._version)
+        kept_of = self.__dict__.get("_halves_of", (None, None))
+        cache = self.__dict__.get("_halves", {})
         key = (padded_dim, str(self.S.device))
-        if key not in cache:
-            out = []
-            for m in (self.S, self.S.t()):
-                hi = m.half()
-                lo = (m - hi.float()).half()
-                for h in (hi, lo):
-                    pad = torch.zeros((padded_dim, padded_dim), dtype=torch.float16,
-                                      device=self.S.device)
-                    pad[:self.dim, :self.dim] = h
-                    out.append(pad)
-            cache[key] = (out[0], out[1], out[2], out[3])
-        return cache[key]
+        if kept_of[0] is not made_from[0] or kept_of[1] != made_from[1]:
+            if cache and self.S.is_cuda:
+                torch.cuda.synchronize(self.S.device)  # kernels on any stream that read the old ones
+            cache = {}
+        if key in cache:
+            return cache[key]
+        out = []
+        for m in (self.S, self.S.t()):
+            hi = m.half()
+            lo = (m - hi.float()).half()
+            for h in (hi, lo):
+                pad = torch.zeros((padded_dim, padded_dim), dtype=torch.float16,
+                                  device=self.S.device)
+                pad[:self.dim, :self.dim] = h
+                out.append(pad)
+        if self.S.is_cuda:
+            if torch.cuda.is_current_stream_capturing():
+                return tuple(out)  # they hold values only once the graph runs: not kept
+            # later calls may come from other streams
+            torch.cuda.current_stream(self.S.device).synchronize()
+        self._halves, self._halves_of = {**cache, key: tuple(out)}, made_from
+        return self._halves[key]
 
     @torch.no_grad()
     def quantize(self, x: torch.Tensor) -> torch.Tensor:
@@ -257,10 +280,11 @@ class TurboQuantProd:
     @torch.no_grad()
     def quantize(self, x: torch.Tensor):
         """-> (mse_packed, mse_norms, qjl_signs int8 {-1, +1}, residual_norms).
-        fp32 vectors on a GPU take one HIP kernel: up to padded size 128 the
-        whole algorithm with the QJL product on the matrix cores
-        (tq_prod_quantize_qjl), above it the MSE stage, its read-back and the
-        unit residual (tq_prod_quantize) followed by the QJL GEMM."""
+        fp32 vectors on a GPU take HIP kernels: up to padded size 128 the
+        whole algorithm in one, with the QJL product on the matrix cores
+        (tq_prod_quantize_qjl); above it the MSE stage, its read-back and the
+        unit residual, followed by the QJL product on the matrix cores
+        (tq_prod_quantize_qjl_ws)."""
         if x.dtype == torch.float32 and self.mse._hip(x):
             from . import ops
             bnd, cen = self.mse._host_tables()
@@ -269,10 +293,9 @@ class TurboQuantProd:
                 sh, sl, _, _ = self.qjl.halves(pd)
                 return ops.prod_quantize_qjl(x, pd, self.mse.bit_width, self.mse.rotation.signs,
                                              bnd, cen, sh, sl)
-            packed, norms, ru, rn = ops.prod_quantize(x, self.mse.rotation.padded_dim,
-                                                      self.mse.bit_width,
-                                                      self.mse.rotation.signs, bnd, cen)
-            return packed, norms, self.qjl.quantize(ru), rn
+            sh, sl, _, _ = self.qjl.halves(pd)
+            return ops.prod_quantize_qjl_ws(x, pd, self.mse.bit_width, self.mse.rotation.signs,
+                                            bnd, cen, sh, sl)
         packed, norms = self.mse.quantize(x)
         r = x - self.mse.dequantize(packed, norms)
         rn = torch.linalg.vector_norm(r, dim=-1).clamp_min(1e-8)
@@ -289,6 +312,12 @@ class TurboQuantProd:
                                                self.dim, pd, self.mse.bit_width,
                                                self.mse.rotation.signs,
                                                self.mse._host_tables()[1], th, tl)
+            if qjl_signs.dtype == torch.int8 and mse_norms.numel() >= QJL_GEMM_MIN:
+                _, _, th, tl = self.qjl.halves(pd)
+                return ops.prod_dequantize_qjl_ws(mse_packed, mse_norms, qjl_signs,
+                                                  residual_norms, self.dim, pd,
+                                                  self.mse.bit_width, self.mse.rotation.signs,
+                                                  self.mse._host_tables()[1], th, tl)
             return ops.prod_dequantize(mse_packed, mse_norms, qjl_signs.float() @ self.qjl.S,
                                        residual_norms, self.dim, self.mse.rotation.padded_dim,
                                        self.mse.bit_width, self.mse.rotation.signs,

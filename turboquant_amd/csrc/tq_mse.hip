@@ -34,11 +34,15 @@
 #include <cstring>
 
 #include "tq_common.h"
+#include "tq_qjl.h"
 
 namespace tq {
 namespace {
 
 constexpr int kMseThreads = 256;
+
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 struct MseParams {
   const float* x;      // quantize in: [n, dim]
@@ -48,6 +52,8 @@ struct MseParams {
   const float* signs;  // [pd]
   float* resid;        // prod quantize out: unit residual [n, dim] (null: MSE only)
   float* rnorm;        // prod quantize out: residual norms [n]
+  _Float16* rhi;       // or, instead of resid: the unit residual times kQjlScale as
+  _Float16* rlo;       // fp16 hi + lo halves [n][pd], zeros past dim
   const float* add;    // prod dequantize in: S^T z rows [n, dim] (null: MSE only)
   const float* gamma;  // prod dequantize in: residual norms [n]
   float add_scale;     // sqrt(pi / 2) / dim
@@ -112,18 +118,56 @@ __device__ __forceinline__ void fmac_xor8(float* x, float sg) {
 #endif
 }
 
-// one cross-lane stage over E registers: v += sg * v of lane l ^ m
+// the butterfly with lane l ^ 4 for 8 registers: a + b on the lower lane, a - b
+// on the upper one, as two DPP instructions writing disjoint banks (lanes 0-3
+// and 8-11 of a row take lane + 4, the others lane - 4); 2 instructions per
+// register where moves and an fma take 3
+__device__ __forceinline__ void butterfly4(float* x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  float y[8];
+#define TQ_B(I, J)                                                              \
+  "v_add_f32_dpp %" #I ", %" #J ", %" #J " row_shl:4 row_mask:0xf bank_mask:0x5\n\t" \
+  "v_sub_f32_dpp %" #I ", %" #J ", %" #J " row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
+  asm volatile("s_nop 1\n\t" TQ_B(0, 8) TQ_B(1, 9) TQ_B(2, 10) TQ_B(3, 11) TQ_B(4, 12)
+                   TQ_B(5, 13) TQ_B(6, 14) TQ_B(7, 15)
+               : "=&v"(y[0]), "=&v"(y[1]), "=&v"(y[2]), "=&v"(y[3]), "=&v"(y[4]), "=&v"(y[5]),
+                 "=&v"(y[6]), "=&v"(y[7])
+               : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]), "v"(x[5]), "v"(x[6]),
+                 "v"(x[7]));
+#undef TQ_B
+  for (int k = 0; k < 8; k++) x[k] = y[k];
+#else
+  (void)x;
+#endif
+}
+
+// the butterfly with lane l ^ 16 for a register pair: the swap brings row 2k
+// of both registers into a and row 2k + 1 into b, a second one puts the sums
+// and differences back
+__device__ __forceinline__ void butterfly16(float& a, float& b) {
+  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  const float lo = __uint_as_float(r[0]), hi = __uint_as_float(r[1]);
+  r = __builtin_amdgcn_permlane16_swap(__float_as_uint(lo + hi), __float_as_uint(lo - hi), false,
+                                       false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+
+// one cross-lane stage over E registers, partner lane l ^ m: lane distances 1,
+// 2 and 8 keep own + sg * partner (the upper lane then holds the difference
+// negated, see tau_scale), 4 and 16 the reference's values
 template <int E>
-__device__ __forceinline__ void fmac_xor(float (&v)[E], int m, float sg) {
+__device__ __forceinline__ void cross_stage(float (&v)[E], int m, float sg) {
   static_assert(E % 8 == 0, "registers in batches of 8");
 #pragma unroll
   for (int b = 0; b < E; b += 8) {
     if (m == 1) fmac_xor8<1>(v + b, sg);
     else if (m == 2) fmac_xor8<2>(v + b, sg);
     else if (m == 8) fmac_xor8<8>(v + b, sg);
+    else if (m == 4) butterfly4(v + b);
     else {
 #pragma unroll
-      for (int k = 0; k < 8; k++) v[b + k] = __builtin_fmaf(lane_xor(v[b + k], m), sg, v[b + k]);
+      for (int k = 0; k < 8; k += 2) butterfly16(v[b + k], v[b + k + 1]);
     }
   }
 }
@@ -144,7 +188,7 @@ __device__ __forceinline__ void fwht_group(float (&v)[E], int p) {
 #pragma unroll
   for (int m = 1; m < P; m <<= 1) {
     const float sg = (p & m) ? -1.0f : 1.0f;  // own + sg * partner: one v_fmac with DPP
-    fmac_xor<E>(v, m, sg);
+    cross_stage<E>(v, m, sg);
   }
 #pragma unroll
   for (int h = 8; h < E; h <<= 1)  // chunk index bits: stride 8 P h / 8
@@ -174,19 +218,20 @@ __device__ __forceinline__ void fwht_contig(float (&v)[E], int p) {
 #pragma unroll
   for (int m = 1; m < P; m <<= 1) {
     const float sg = (p & m) ? -1.0f : 1.0f;
-    fmac_xor<E>(v, m, sg);
+    cross_stage<E>(v, m, sg);
   }
 }
 
 // Both transforms leave lane p with tau_p times the reference's values, tau_p
-// = (-1)^popcount(p): a cross-lane stage keeps own + sg * partner, which on
-// the upper lane is own - partner = -(partner - own), the reference's value
-// negated (exactly); lanes paired in a stage share tau from the earlier
-// stages, and negation commutes with the in-lane stages.  The scale 1/sqrt(pd)
-// then takes tau: (tau v) * (tau s) == v * s bit for bit.
+// = (-1)^popcount of p's bits 0, 1 and 3: those cross-lane stages keep own +
+// sg * partner, which on the upper lane is own - partner = -(partner - own),
+// the reference's value negated (exactly); lanes paired in a stage share tau
+// from the earlier stages (the stages 4 and 16 keep the sign: both operands
+// carry the same tau), and negation commutes with the in-lane stages.  The
+// scale 1/sqrt(pd) then takes tau: (tau v) * (tau s) == v * s bit for bit.
 template <int P>
 __device__ __forceinline__ float tau_scale(float inv_sqrt_pd, int p) {
-  return (__builtin_popcount(p & (P - 1)) & 1) ? -inv_sqrt_pd : inv_sqrt_pd;
+  return (__builtin_popcount(p & (P - 1) & 0xb) & 1) ? -inv_sqrt_pd : inv_sqrt_pd;
 }
 
 // fp32 value with the sign of a +-1 sign value folded in (exact: s * v)
@@ -240,6 +285,10 @@ __device__ __forceinline__ int bin_code(float y, const uint2* bins, int base) {
 // rn = max(||r||, 1e-8) (stored) and r / rn correctly rounded, left in v
 // (0 beyond dim).  Every lane of the workgroup runs this, live or not (the
 // lane exchanges need the whole vector group); only live rows store.
+//
+// Rows of a multiple of four dims come as float4 pieces also where dim is not
+// the padded size (60,000 x 1000: the kernel 202 -> 82 us against single
+// floats; 500,009 x 96: 108 -> 45 us).
 template <int PD>
 __device__ __forceinline__ void load_row(const MseParams& p, int64_t row, int sub,
                                          float (&v)[MseGeom<PD>::E]) {
@@ -251,6 +300,17 @@ __device__ __forceinline__ void load_row(const MseParams& p, int64_t row, int su
 #pragma unroll
     for (int i = 0; i < E / 4; i++) {
       const float4 f = src[i];
+      v[4 * i] = f.x;
+      v[4 * i + 1] = f.y;
+      v[4 * i + 2] = f.z;
+      v[4 * i + 3] = f.w;
+    }
+  } else if ((p.dim & 3) == 0) {  // rows 16-byte aligned, a float4 wholly inside or past the end
+    const float* src = p.x + (live ? row : 0) * p.dim + d0;
+#pragma unroll
+    for (int i = 0; i < E / 4; i++) {
+      float4 f = {0.0f, 0.0f, 0.0f, 0.0f};
+      if (live && d0 + 4 * i < p.dim) f = reinterpret_cast<const float4*>(src)[i];
       v[4 * i] = f.x;
       v[4 * i + 1] = f.y;
       v[4 * i + 2] = f.z;
@@ -381,12 +441,28 @@ __global__ __launch_bounds__(kMseThreads) void mse_quantize_kernel(MseParams p) 
   if constexpr (RES) {
     if (row >= p.n) return;
     const int d0 = sub * E;
+    if (p.rhi) {  // (v s - hi is exact in fp32)
+#pragma unroll
+      for (int c = 0; c < E / 8; c++) {
+        half8_t h, l;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          const float r = v[8 * c + e] * kQjlScale;
+          h[e] = (_Float16)r;
+          l[e] = (_Float16)(r - (float)h[e]);
+        }
+        *reinterpret_cast<half8_t*>(p.rhi + row * PD + d0 + 8 * c) = h;
+        *reinterpret_cast<half8_t*>(p.rlo + row * PD + d0 + 8 * c) = l;
+      }
+      return;
+    }
     float* rrow = p.resid + row * p.dim;
-    if (p.dim == PD) {
+    if ((p.dim & 3) == 0) {
 #pragma unroll
       for (int i = 0; i < E / 4; i++)
-        reinterpret_cast<float4*>(rrow + d0)[i] =
-            float4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+        if (d0 + 4 * i < p.dim)
+          reinterpret_cast<float4*>(rrow + d0)[i] =
+              float4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
     } else {
 #pragma unroll
       for (int i = 0; i < E; i++)
@@ -435,16 +511,14 @@ template <int PD, int BITS, bool ADD>
 __device__ __forceinline__ void dequantize_row(const MseParams& p, const float* cen, int64_t row,
                                                int sub, const float* arow,
                                                const RowCodes<PD, BITS>& rc,
-                                               float* stage = nullptr) {
+                                               float (&v)[MseGeom<PD>::E]) {
 #pragma clang fp contract(off)
   using MG = MseGeom<PD>;
-  constexpr int P = MG::P, E = MG::E, NC = E / 8;
+  constexpr int P = MG::P, E = MG::E;
   constexpr int PER = BITS == 3 ? 2 : 8 / BITS;
   constexpr uint32_t kMask = (1u << BITS) - 1u;
-  const bool live = row < p.n;
   const uint32_t* word = rc.word;
   const float nrm = rc.nrm;
-  float v[E];
 #pragma unroll
   for (int i = 0; i < E; i++) {
     const int k = i % 8;
@@ -452,52 +526,61 @@ __device__ __forceinline__ void dequantize_row(const MseParams& p, const float* 
   }
   fwht_group<E, P>(v, sub);
   const float ts = tau_scale<P>(p.inv_sqrt_pd, sub);  // v holds tau * FWHT
-  if (!live) return;
-  float* orow = p.out + row * p.dim;
+  if (row >= p.n) return;
   const float wq = ADD ? p.add_scale * p.gamma[row] : 0.0f;
-  // the signs of the lane's chunks, two float4 loads per chunk
-  float sg[E];
+  const bool full = (p.dim & 3) == 0;  // uniform
 #pragma unroll
-  for (int i = 0; i < NC; i++) {
-    const float4* sp = reinterpret_cast<const float4*>(p.signs + 8 * (sub + P * i));
-    const float4 a = sp[0], b = sp[1];
-    sg[8 * i] = a.x;
-    sg[8 * i + 1] = a.y;
-    sg[8 * i + 2] = a.z;
-    sg[8 * i + 3] = a.w;
-    sg[8 * i + 4] = b.x;
-    sg[8 * i + 5] = b.y;
-    sg[8 * i + 6] = b.z;
-    sg[8 * i + 7] = b.w;
-  }
-  auto val = [&](int i) {
+  for (int i = 0; i < E; i += 4) {
     const int d = 8 * (sub + P * (i / 8)) + i % 8;
-    const float xm = apply_sign(v[i] * ts, sg[i]) * nrm;
-    if constexpr (ADD) return xm + arow[d] * wq;
-    else return xm;
-  };
-  if (p.dim == PD) {
-    // into the row's LDS stage (the caller writes it out coalesced), or HBM
-    float* const dst = stage ? stage : orow;
-#pragma unroll
-    for (int i = 0; i < NC; i++) {
-      float4* o4 = reinterpret_cast<float4*>(dst + 8 * (sub + P * i));
-      o4[0] = float4{val(8 * i), val(8 * i + 1), val(8 * i + 2), val(8 * i + 3)};
-      o4[1] = float4{val(8 * i + 4), val(8 * i + 5), val(8 * i + 6), val(8 * i + 7)};
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < E; i++) {
-      const int d = 8 * (sub + P * (i / 8)) + i % 8;
-      if (d < p.dim) orow[d] = val(i);
+    const float4 s = *reinterpret_cast<const float4*>(p.signs + d);
+    v[i] = apply_sign(v[i] * ts, s.x) * nrm;
+    v[i + 1] = apply_sign(v[i + 1] * ts, s.y) * nrm;
+    v[i + 2] = apply_sign(v[i + 2] * ts, s.z) * nrm;
+    v[i + 3] = apply_sign(v[i + 3] * ts, s.w) * nrm;
+    if constexpr (ADD) {
+      float4 t = {0.0f, 0.0f, 0.0f, 0.0f};
+      if (full) {
+        if (d < p.dim) t = *reinterpret_cast<const float4*>(arow + d);
+      } else {
+        t.x = d < p.dim ? arow[d] : 0.0f;
+        t.y = d + 1 < p.dim ? arow[d + 1] : 0.0f;
+        t.z = d + 2 < p.dim ? arow[d + 2] : 0.0f;
+        t.w = d + 3 < p.dim ? arow[d + 3] : 0.0f;
+      }
+      v[i] = v[i] + t.x * wq;
+      v[i + 1] = v[i + 1] + t.y * wq;
+      v[i + 2] = v[i + 2] + t.z * wq;
+      v[i + 3] = v[i + 3] + t.w * wq;
     }
   }
 }
 
-// Full-width rows (dim == pd) go out through an LDS stage per wave: the
+// a lane's values of a row to dst (the row in LDS or HBM): whole float4 pieces
+// (VEC: dim is a multiple of four, so each lies inside the row or past its
+// end), or single floats
+template <int PD, bool VEC>
+__device__ __forceinline__ void store_chunks(float* dst, int sub, int dim,
+                                             const float (&v)[MseGeom<PD>::E]) {
+  constexpr int P = MseGeom<PD>::P, E = MseGeom<PD>::E;
+#pragma unroll
+  for (int i = 0; i < E; i += 4) {
+    const int d = 8 * (sub + P * (i / 8)) + i % 8;
+    if constexpr (VEC) {
+      if (d < dim)
+        *reinterpret_cast<float4*>(dst + d) = float4{v[i], v[i + 1], v[i + 2], v[i + 3]};
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        if (d + e < dim) dst[d + e] = v[i + e];
+    }
+  }
+}
+
+// Rows of a multiple of four dims go out through an LDS stage per wave: the
 // wave's 64 / P rows are consecutive in memory, so each store instruction
 // writes 1 KB of consecutive bytes (64 lanes x 16 B) instead of 16-byte
-// pieces at a 32-byte stride that leave every line half-written.
+// pieces at a 32-byte stride that leave every line half-written (1M x 128:
+// 149.5 -> 126.6 us; 60,000 x 1000, single floats before: 161 -> 48 us).
 template <int PD, int BITS, bool ADD>
 __global__ __launch_bounds__(kMseThreads) void mse_dequantize_kernel(MseParams p) {
   using MG = MseGeom<PD>;
@@ -509,12 +592,15 @@ __global__ __launch_bounds__(kMseThreads) void mse_dequantize_kernel(MseParams p
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int sub = lane % P, vw = lane / P;
   const int64_t row = (int64_t)blockIdx.x * MG::VPB + threadIdx.x / P;
-  const bool staged = p.dim == PD;  // uniform
+  float v[MG::E];
   dequantize_row<PD, BITS, ADD>(p, cen, row, sub,
                                 ADD && row < p.n ? p.add + row * p.dim : nullptr,
-                                load_codes<PD, BITS>(p, row, sub),
-                                staged ? &stg[w][vw * PD] : nullptr);
-  if (!staged) return;
+                                load_codes<PD, BITS>(p, row, sub), v);
+  if ((p.dim & 3) != 0) {  // uniform
+    if (row < p.n) store_chunks<PD, false>(p.out + row * p.dim, sub, p.dim, v);
+    return;
+  }
+  if (row < p.n) store_chunks<PD, true>(&stg[w][vw * p.dim], sub, p.dim, v);
   // LDS operations of one wave complete in order; the wave barrier keeps the
   // compiler from moving the reads above the writes
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -523,8 +609,8 @@ __global__ __launch_bounds__(kMseThreads) void mse_dequantize_kernel(MseParams p
   const int64_t row0 = (int64_t)blockIdx.x * MG::VPB + (int64_t)w * VW;
   const int64_t rows = p.n - row0 < VW ? p.n - row0 : VW;
   if (rows <= 0) return;
-  const int total = (int)rows * PD;  // floats of the wave's live rows
-  float* const dst = p.out + row0 * PD;
+  const int total = (int)rows * p.dim;  // floats of the wave's live rows
+  float* const dst = p.out + row0 * p.dim;
 #pragma unroll
   for (int k = 4 * lane; k < VW * PD; k += 256)
     if (k < total) *reinterpret_cast<float4*>(dst + k) = *reinterpret_cast<const float4*>(&stg[w][k]);
@@ -547,9 +633,6 @@ __global__ __launch_bounds__(kMseThreads) void mse_dequantize_kernel(MseParams p
 // vectors from LDS (lane: vector l % 16, the same dims), D = lane: vector
 // l % 16, outputs 4 (l / 16) + e.
 // --------------------------------------------------------------------------
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
 struct QjlParams {
   const _Float16* s_hi;  // [PD][PD] row-major: quantize S, dequantize S^T
   const _Float16* s_lo;
@@ -744,9 +827,10 @@ __global__ __launch_bounds__(kMseThreads) void prod_qjl_dequantize_kernel(MsePar
     // full-width rows: each lane overwrites its own dims of the term row with
     // the output, and the wave writes its 8 consecutive rows out coalesced
     const bool staged = p.dim == PD;  // uniform
-    dequantize_row<PD, BITS, true>(p, cen, row, sub, term + vl * TS, cc,
-                                   staged ? term + vl * TS : nullptr);
+    float v[MG::E];
+    dequantize_row<PD, BITS, true>(p, cen, row, sub, term + vl * TS, cc, v);
     if (staged) {
+      if (row < p.n) store_chunks<PD, true>(term + vl * TS, sub, PD, v);
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -762,6 +846,9 @@ __global__ __launch_bounds__(kMseThreads) void prod_qjl_dequantize_kernel(MsePar
             *reinterpret_cast<float4*>(dst + k) = *reinterpret_cast<const float4*>(
                 term + (w * VW + k / PD) * TS + k % PD);
       }
+    } else if (row < p.n) {
+      if ((p.dim & 3) == 0) store_chunks<PD, true>(p.out + row * p.dim, sub, p.dim, v);
+      else store_chunks<PD, false>(p.out + row * p.dim, sub, p.dim, v);
     }
     __syncthreads();  // the next batch rewrites the tile
   }
@@ -773,7 +860,7 @@ hipError_t launch_mse(bool quant, int bits, const MseParams& p, hipStream_t st) 
   const dim3 block(kMseThreads);
 #define TQ_MSE_CASE(B)                                                                   \
   case B:                                                                                \
-    if (quant && p.resid)                                                                \
+    if (quant && p.rnorm)                                                                \
       hipLaunchKernelGGL((mse_quantize_kernel<PD, B, true>), grid, block, 0, st, p);     \
     else if (quant)                                                                      \
       hipLaunchKernelGGL((mse_quantize_kernel<PD, B, false>), grid, block, 0, st, p);    \
@@ -851,6 +938,8 @@ bool build_bins(const float* b, int bits, MseParams& p) {
 struct ProdArgs {
   const float* centroids = nullptr;  // quantize: read-back table
   float* resid = nullptr;
+  _Float16* rhi = nullptr;  // or the residual as halves
+  _Float16* rlo = nullptr;
   float* rnorm = nullptr;
   const float* add = nullptr;  // dequantize
   const float* gamma = nullptr;
@@ -880,9 +969,9 @@ int mse_call(bool quant, const float* x, uint8_t* packed, float* norms, float* o
     set_error("%s: null pointer", what);
     return kEinval;
   }
-  const bool prod_q = pa.resid || pa.rnorm || pa.centroids;
+  const bool prod_q = pa.resid || pa.rhi || pa.rnorm || pa.centroids;
   const bool prod_d = pa.add || pa.gamma;
-  if ((prod_q && !(pa.resid && pa.rnorm && pa.centroids)) || (prod_d && !(pa.add && pa.gamma))) {
+  if ((prod_q && !((pa.resid || (pa.rhi && pa.rlo)) && pa.rnorm && pa.centroids)) || (prod_d && !(pa.add && pa.gamma))) {
     set_error("%s: null pointer", what);
     return kEinval;
   }
@@ -901,6 +990,8 @@ int mse_call(bool quant, const float* x, uint8_t* packed, float* norms, float* o
   p.out = out;
   p.signs = signs;
   p.resid = pa.resid;
+  p.rhi = pa.rhi;
+  p.rlo = pa.rlo;
   p.rnorm = pa.rnorm;
   p.add = pa.add;
   p.gamma = pa.gamma;
@@ -938,7 +1029,7 @@ int prod_qjl_call(bool quant, const float* x, uint8_t* packed, float* norms, flo
                   const float* gamma, tq_stream_t stream) {
   const char* what = quant ? "prod_quantize_qjl" : "prod_dequantize_qjl";
   if (padded_dim != 64 && padded_dim != 128) {
-    set_error("%s: padded_dim %d unsupported (64 or 128; larger sizes take the BLAS path)", what,
+    set_error("%s: padded_dim %d unsupported (64 or 128; larger sizes: the _ws entry point)", what,
               padded_dim);
     return kEinval;
   }
@@ -978,6 +1069,8 @@ int prod_qjl_call(bool quant, const float* x, uint8_t* packed, float* norms, flo
   p.out = out;
   p.signs = signs;
   p.resid = nullptr;
+  p.rhi = nullptr;
+  p.rlo = nullptr;
   p.rnorm = rnorm;
   p.add = nullptr;
   p.gamma = gamma;
@@ -1120,6 +1213,114 @@ extern "C" int tq_prod_dequantize_qjl(const uint8_t* packed, const float* norms,
                            mse_bit_width, signs, centroids, nullptr,
                            static_cast<const _Float16*>(st_hi), static_cast<const _Float16*>(st_lo),
                            nullptr, qjl_signs, nullptr, residual_norms, stream);
+}
+
+namespace tq {
+namespace {
+
+// operand checks of the entry points above padded size 128
+int qjl_ws_check(const char* what, int32_t padded_dim, const void* hi, const void* lo,
+                 const void* z, int64_t n, int32_t dim) {
+  if (padded_dim != 256 && padded_dim != 512 && padded_dim != 1024) {
+    set_error("%s: padded_dim %d unsupported (256, 512 or 1024)", what, padded_dim);
+    return kEinval;
+  }
+  if (dim < 1 || dim > padded_dim || 2 * dim <= padded_dim) {
+    set_error("%s: padded_dim %d must be the power of two next to dim %d", what, padded_dim, dim);
+    return kEinval;
+  }
+  if (n < 0 || n > ((int64_t)1 << 32)) {  // (also keeps the tile count in an int32)
+    set_error("%s: vector count %lld out of range", what, (long long)n);
+    return kEinval;
+  }
+  if (n == 0) return 0;
+  if (!hi || !lo || !z) {
+    set_error("%s: null pointer", what);
+    return kEinval;
+  }
+  if ((((uintptr_t)hi | (uintptr_t)lo) & 15) != 0 || ((uintptr_t)z & 7) != 0) {
+    set_error("%s: the S halves must be 16-byte and qjl_signs 8-byte aligned", what);
+    return kEinval;
+  }
+  return 0;
+}
+
+}  // namespace
+}  // namespace tq
+
+extern "C" int64_t tq_prod_workspace_bytes(int64_t num_vectors, int32_t padded_dim) {
+  if (num_vectors <= 0 || padded_dim < 256 || padded_dim > 1024) return 0;
+  return num_vectors * padded_dim * 4;
+}
+
+extern "C" int tq_prod_quantize_qjl_ws(const float* x, int64_t num_vectors, int32_t dim,
+                                       int32_t padded_dim, int32_t mse_bit_width,
+                                       const float* signs, const float* boundaries,
+                                       const float* centroids, const void* s_hi, const void* s_lo,
+                                       uint8_t* packed, float* norms, int8_t* qjl_signs,
+                                       float* residual_norms, void* workspace,
+                                       int64_t workspace_bytes, tq_stream_t stream) {
+  const char* what = "prod_quantize_qjl_ws";
+  int rc = tq::qjl_ws_check(what, padded_dim, s_hi, s_lo, qjl_signs, num_vectors, dim);
+  if (rc || num_vectors == 0) return rc;
+  if (!centroids || !residual_norms) {
+    tq::set_error("%s: null pointer", what);
+    return tq::kEinval;
+  }
+  if (!workspace || ((uintptr_t)workspace & 15) != 0 ||
+      workspace_bytes < tq_prod_workspace_bytes(num_vectors, padded_dim)) {
+    tq::set_error("%s: workspace must be 16-byte aligned and hold %lld bytes", what,
+                  (long long)tq_prod_workspace_bytes(num_vectors, padded_dim));
+    return tq::kEinval;
+  }
+  tq::ProdArgs pa;
+  pa.centroids = centroids;
+  pa.rhi = static_cast<_Float16*>(workspace);
+  pa.rlo = pa.rhi + num_vectors * padded_dim;
+  pa.rnorm = residual_norms;
+  rc = tq::mse_call(true, x, packed, norms, nullptr, num_vectors, dim, padded_dim, mse_bit_width,
+                    signs, boundaries, stream, what, pa);
+  if (rc) return rc;
+  const hipError_t e = tq::launch_qjl(
+      true, pa.rhi, pa.rlo, nullptr, static_cast<const _Float16*>(s_hi),
+      static_cast<const _Float16*>(s_lo), qjl_signs, nullptr, num_vectors, dim, padded_dim,
+      reinterpret_cast<hipStream_t>(stream));
+  if (e != hipSuccess) tq::set_error("%s: launch failed: %s", what, hipGetErrorString(e));
+  return (int)e;
+}
+
+extern "C" int tq_prod_dequantize_qjl_ws(const uint8_t* packed, const float* norms,
+                                         const int8_t* qjl_signs, const float* residual_norms,
+                                         int64_t num_vectors, int32_t dim, int32_t padded_dim,
+                                         int32_t mse_bit_width, const float* signs,
+                                         const float* centroids, const void* st_hi,
+                                         const void* st_lo, float* out, tq_stream_t stream) {
+  const char* what = "prod_dequantize_qjl_ws";
+  int rc = tq::qjl_ws_check(what, padded_dim, st_hi, st_lo, qjl_signs, num_vectors, dim);
+  if (rc || num_vectors == 0) return rc;
+  if (!packed || !norms || !residual_norms || !signs || !centroids || !out) {
+    tq::set_error("%s: null pointer", what);
+    return tq::kEinval;
+  }
+  if (mse_bit_width < 1 || mse_bit_width > 4) {
+    tq::set_error("%s: bit_width %d unsupported (1..4)", what, mse_bit_width);
+    return tq::kEinval;
+  }
+  if ((((uintptr_t)out | (uintptr_t)packed | (uintptr_t)signs) & 15) != 0) {
+    tq::set_error("%s: out, packed and signs must be 16-byte aligned", what);
+    return tq::kEinval;
+  }
+  // z S goes into the output rows, which the dequantize then completes in place
+  const hipError_t e = tq::launch_qjl(
+      false, nullptr, nullptr, qjl_signs, static_cast<const _Float16*>(st_hi),
+      static_cast<const _Float16*>(st_lo), nullptr, out, num_vectors, dim, padded_dim,
+      reinterpret_cast<hipStream_t>(stream));
+  if (e != hipSuccess) {
+    tq::set_error("%s: launch failed: %s", what, hipGetErrorString(e));
+    return (int)e;
+  }
+  return tq_prod_dequantize(packed, norms, out, residual_norms, num_vectors, dim, padded_dim,
+                            mse_bit_width, signs, centroids, out, stream);
 }
 
 extern "C" int tq_diag_mse_bucketize(int32_t force_search) {

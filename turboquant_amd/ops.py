@@ -436,6 +436,22 @@ def prod_quantize_qjl(x: torch.Tensor, padded_dim: int, mse_bit_width: int,
     padded_dim 64 or 128): x fp32 [..., dim] -> (packed, norms, qjl_signs int8
     [..., dim], residual_norms).  s_hi / s_lo: fp16 [padded_dim, padded_dim]
     halves of the QJL matrix."""
+    return _prod_quantize_qjl(x, padded_dim, mse_bit_width, signs, boundaries, centroids, s_hi,
+                              s_lo, False)
+
+
+def prod_quantize_qjl_ws(x: torch.Tensor, padded_dim: int, mse_bit_width: int,
+                         signs: torch.Tensor, boundaries, centroids, s_hi: torch.Tensor,
+                         s_lo: torch.Tensor):
+    """prod_quantize_qjl at padded_dim 256, 512 or 1024: the row kernel and
+    the QJL product on the matrix cores (tq_prod_quantize_qjl_ws), the unit
+    residual between them in a workspace from torch's allocator."""
+    return _prod_quantize_qjl(x, padded_dim, mse_bit_width, signs, boundaries, centroids, s_hi,
+                              s_lo, True)
+
+
+def _prod_quantize_qjl(x, padded_dim, mse_bit_width, signs, boundaries, centroids, s_hi, s_lo,
+                       large: bool):
     _require_gpu(x, signs, s_hi, s_lo)
     if x.dtype != torch.float32:
         raise RuntimeError("prod_quantize_qjl: x must be fp32")
@@ -457,12 +473,17 @@ def prod_quantize_qjl(x: torch.Tensor, padded_dim: int, mse_bit_width: int,
     rnorm = torch.empty(lead, dtype=torch.float32, device=x.device)
     signs = _aligned16(signs)
     lib = _lib.load()
+    args = (x.data_ptr(), n, dim, int(padded_dim), int(mse_bit_width), signs.data_ptr(),
+            _host_f32(boundaries), _host_f32(centroids), s_hi.data_ptr(), s_lo.data_ptr(),
+            packed.data_ptr(), norms.data_ptr(), z.data_ptr(), rnorm.data_ptr())
     with torch.cuda.device(x.device):
-        rc = lib.tq_prod_quantize_qjl(x.data_ptr(), n, dim, int(padded_dim), int(mse_bit_width),
-                                      signs.data_ptr(), _host_f32(boundaries),
-                                      _host_f32(centroids), s_hi.data_ptr(), s_lo.data_ptr(),
-                                      packed.data_ptr(), norms.data_ptr(), z.data_ptr(),
-                                      rnorm.data_ptr(), _stream_ptr(x.device))
+        if large:
+            ws = torch.empty(int(lib.tq_prod_workspace_bytes(n, int(padded_dim))),
+                             dtype=torch.uint8, device=x.device)
+            rc = lib.tq_prod_quantize_qjl_ws(*args, ws.data_ptr(), ws.numel(),
+                                             _stream_ptr(x.device))
+        else:
+            rc = lib.tq_prod_quantize_qjl(*args, _stream_ptr(x.device))
     _lib.check(rc, "prod_quantize_qjl")
     return packed, norms, z, rnorm
 
@@ -474,6 +495,22 @@ def prod_dequantize_qjl(packed: torch.Tensor, norms: torch.Tensor, qjl_signs: to
     """TurboQuantProd.dequantize with z S formed in-kernel
     (tq_prod_dequantize_qjl, padded_dim 64 or 128).  st_hi / st_lo: fp16
     halves of S^T."""
+    return _prod_dequantize_qjl(packed, norms, qjl_signs, residual_norms, dim, padded_dim,
+                                mse_bit_width, signs, centroids, st_hi, st_lo, False)
+
+
+def prod_dequantize_qjl_ws(packed: torch.Tensor, norms: torch.Tensor, qjl_signs: torch.Tensor,
+                           residual_norms: torch.Tensor, dim: int, padded_dim: int,
+                           mse_bit_width: int, signs: torch.Tensor, centroids,
+                           st_hi: torch.Tensor, st_lo: torch.Tensor) -> torch.Tensor:
+    """prod_dequantize_qjl at padded_dim 256, 512 or 1024
+    (tq_prod_dequantize_qjl_ws)."""
+    return _prod_dequantize_qjl(packed, norms, qjl_signs, residual_norms, dim, padded_dim,
+                                mse_bit_width, signs, centroids, st_hi, st_lo, True)
+
+
+def _prod_dequantize_qjl(packed, norms, qjl_signs, residual_norms, dim, padded_dim, mse_bit_width,
+                         signs, centroids, st_hi, st_lo, large: bool):
     _require_gpu(packed, norms, qjl_signs, residual_norms, signs, st_hi, st_lo)
     per = 2 if mse_bit_width == 3 else 8 // mse_bit_width
     if packed.dtype != torch.uint8 or packed.shape[-1] != padded_dim // per:
@@ -498,12 +535,11 @@ def prod_dequantize_qjl(packed: torch.Tensor, norms: torch.Tensor, qjl_signs: to
     signs = _aligned16(signs)
     lib = _lib.load()
     with torch.cuda.device(packed.device):
-        rc = lib.tq_prod_dequantize_qjl(packed.data_ptr(), nf.data_ptr(), z.data_ptr(),
-                                        rn.data_ptr(), nf.numel(), int(dim), int(padded_dim),
-                                        int(mse_bit_width), signs.data_ptr(),
-                                        _host_f32(centroids), st_hi.data_ptr(),
-                                        st_lo.data_ptr(), out.data_ptr(),
-                                        _stream_ptr(packed.device))
+        fn = lib.tq_prod_dequantize_qjl_ws if large else lib.tq_prod_dequantize_qjl
+        rc = fn(packed.data_ptr(), nf.data_ptr(), z.data_ptr(), rn.data_ptr(), nf.numel(),
+                int(dim), int(padded_dim), int(mse_bit_width), signs.data_ptr(),
+                _host_f32(centroids), st_hi.data_ptr(), st_lo.data_ptr(), out.data_ptr(),
+                _stream_ptr(packed.device))
     _lib.check(rc, "prod_dequantize_qjl")
     return out
 
