@@ -332,8 +332,8 @@ def bench_prefill_chunk(torch, w, steps, warmup, chunk=2048):
     a chunk of `chunk` new tokens at the end of a configs[2] sequence (32768
     tokens, so 30720 cached before it; the chunk's own K/V are in the cache
     too, written first as vLLM does), Qwen3-8B geometry.  The cached context
-    is read back by tq_dequant_paged and the chunk attends it plus its fresh
-    K/V in tq_prefill_attention (lower-right causal, grouped kv heads).  The
+    is read back by tq_prefill_gather and the chunk attends it plus its fresh
+    K/V in tq_prefill_attention_batch (lower-right causal, grouped kv heads).  The
     metadata carries host copies of the boundaries (as vLLM's does), so no
     device-to-host read happens; timed call by call with HIP events."""
     from types import SimpleNamespace
@@ -357,8 +357,8 @@ def bench_prefill_chunk(torch, w, steps, warmup, chunk=2048):
                        max(1, min(steps, 50)), max(1, min(warmup, 5)))
     return {"us": round(ms * 1e3, 1), "chunk_tokens": chunk, "cached_tokens": L - chunk,
             "config": "Qwen3-8B geometry 32q/8kv/128, one request, context read back from "
-                      "the quantized cache (tq_dequant_paged) + tq_prefill_attention "
-                      "(lower-right causal, GQA)"}
+                      "the quantized cache (tq_prefill_gather) + "
+                      "tq_prefill_attention_batch (lower-right causal, GQA)"}
 
 
 MFMA_F16_PEAK_TFLOPS = 2500.0

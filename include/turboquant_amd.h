@@ -220,6 +220,26 @@ int tq_dequant_paged(const uint8_t* k_slab, const uint8_t* v_slab,
                      tq_stream_t stream);
 
 /*
+ * Keys and values of the requests of a prefill step as fp16 rows
+ * [*, num_kv_heads, padded_dim] (rows contiguous, zero past head_dim) in one
+ * launch: request i's ctx_lens[i] cached tokens (page-table row table_rows[i],
+ * block_table_stride entries apart) read back as tq_dequant_paged does to the
+ * rows from out_starts[i] of out_k / out_v, then its fresh_lens[i] rows from
+ * fresh_starts[i] of key / value (in_dtype) converted to fp16.  The five index
+ * arrays are HOST arrays, read before the call returns.  The slabs and the
+ * table may be null when every ctx is 0.
+ */
+int tq_prefill_gather(const uint8_t* k_slab, const uint8_t* v_slab, const int32_t* block_table,
+                      int64_t block_table_stride, int32_t num_kv_heads, int32_t head_dim,
+                      int32_t padded_dim, int32_t block_size, int32_t ebs, int64_t num_blocks,
+                      const float* signs, const void* key, const void* value, int32_t in_dtype,
+                      int64_t k_stride_tok, int64_t k_stride_head, int64_t v_stride_tok,
+                      int64_t v_stride_head, const int32_t* table_rows, const int32_t* ctx_lens,
+                      const int32_t* fresh_starts, const int32_t* fresh_lens,
+                      const int32_t* out_starts, int32_t num_requests, void* out_k, void* out_v,
+                      tq_stream_t stream);
+
+/*
  * Causal GQA attention of a prefill chunk over fp16 K/V (head_dim 64, 128 or 256):
  * o[i, h] = softmax_j(q[i, h] . k[j, h / r] * sm_scale) v[j, h / r] over keys
  * j <= (kv_len - q_len) + i, r = num_qo_heads / num_kv_heads.  q, o: fp16
@@ -262,6 +282,31 @@ int tq_prefill_attention_ws(const void* q, int64_t q_stride_tok, int64_t q_strid
                             void* workspace, int64_t workspace_bytes, tq_stream_t stream);
 int64_t tq_prefill_workspace_bytes(int32_t q_len, int32_t kv_len, int32_t num_qo_heads,
                                    int32_t num_kv_heads, int32_t head_dim);
+
+/*
+ * The same attention for the requests of one scheduler step in one launch:
+ * request i has q_lens[i] query rows from row q_starts[i] of q (and o) and
+ * kv_lens[i] >= q_lens[i] keys from row kv_starts[i] of k / v (kv_sources[i]
+ * 0) or of k2 / v2 (kv_sources[i] != 0), the queries at the end of its keys.
+ * The five arrays are HOST arrays, read before the call returns.  q and o hold
+ * head_dim (a multiple of 8) elements per head, fp16 or bf16 (TQ_F16 /
+ * TQ_BF16); K and V are fp16 rows of padded_dim (64, 128 or 256) elements,
+ * zero past head_dim.  Query blocks whose keys would outlast the rest of the
+ * launch are split over workgroups and merged; the workspace (16-byte
+ * aligned) must hold tq_prefill_batch_workspace_bytes.
+ */
+int64_t tq_prefill_batch_workspace_bytes(const int32_t* q_lens, const int32_t* kv_lens,
+                                         int32_t num_requests, int32_t num_qo_heads,
+                                         int32_t padded_dim);
+int tq_prefill_attention_batch(
+    const void* q, int64_t q_stride_tok, int64_t q_stride_head, int32_t q_dtype, const void* k,
+    int64_t k_stride_tok, int64_t k_stride_head, const void* v, int64_t v_stride_tok,
+    int64_t v_stride_head, const void* k2, const void* v2, int64_t k2_stride_tok,
+    int64_t k2_stride_head, void* o, int64_t o_stride_tok, int64_t o_stride_head, int32_t o_dtype,
+    const int32_t* q_starts, const int32_t* q_lens, const int32_t* kv_starts,
+    const int32_t* kv_lens, const int32_t* kv_sources, int32_t num_requests, int32_t num_qo_heads,
+    int32_t num_kv_heads, int32_t head_dim, int32_t padded_dim, float sm_scale, void* workspace,
+    int64_t workspace_bytes, tq_stream_t stream);
 
 /*
  * The algorithm library's TurboQuantMSE quantizer (reference

@@ -49,6 +49,14 @@ SIGNATURES = {
                                        _I64, _I64, _I32, _I32, _I32, _I32, _I32, _F32, _P, _I64,
                                        _P]),
     "tq_prefill_workspace_bytes": (_I64, [_I32, _I32, _I32, _I32, _I32]),
+    "tq_prefill_gather": (_I32, [_P, _P, _P, _I64, _I32, _I32, _I32, _I32, _I32, _I64, _P, _P,
+                                 _P, _I32, _I64, _I64, _I64, _I64, _P, _P, _P, _P, _P, _I32, _P,
+                                 _P, _P]),
+    "tq_prefill_batch_workspace_bytes": (_I64, [_P, _P, _I32, _I32, _I32]),
+    "tq_prefill_attention_batch": (_I32, [_P, _I64, _I64, _I32, _P, _I64, _I64, _P, _I64, _I64,
+                                          _P, _P, _I64, _I64, _P, _I64, _I64, _I32, _P, _P, _P,
+                                          _P, _P, _I32, _I32, _I32, _I32, _I32, _F32, _P, _I64,
+                                          _P]),
     "tq_mse_quantize": (_I32, [_P, _I64, _I32, _I32, _I32, _P, _P, _P, _P, _P]),
     "tq_mse_dequantize": (_I32, [_P, _P, _I64, _I32, _I32, _I32, _P, _P, _P, _P]),
     "tq_prod_quantize": (_I32, [_P, _I64, _I32, _I32, _I32, _P, _P, _P, _P, _P, _P, _P, _P]),

@@ -36,6 +36,10 @@
 //    conflict-free.  Two buffers of each (distinct LDS arrays, so the
 //    compiler does not wait for the copies in flight into the other buffer),
 //    one barrier per tile.
+//  * The requests of a scheduler step run as one launch of work items (batch
+//    mode, tq_prefill_attention_batch): five prompts of 229 .. 1326 tokens at
+//    32 q heads take 52 us where five launches with their key splits and
+//    merges took 125 us, two chunks over 5000-token contexts 138 against 175.
 //  * Short chunks over long contexts (too few query blocks to fill the
 //    CUs): each query block's tiles are split over several workgroups
 //    (grid z), which leave their normalised O (fp16), reference max and row
@@ -44,7 +48,10 @@
 //    moves only when a tile exceeds it by more than 8 / scale); probabilities
 //    enter the PV MFMA as fp16 (round to nearest), accumulation is fp32;
 //    at head size 64 the row sum is taken from those fp16 values.
-#include <atomic>
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
+#include <vector>
 
 #include "tq_common.h"
 
@@ -84,6 +91,54 @@ struct PrefillParams {
   float* ws_ml;    // [nsplit][lq][Hq][2]
 };
 
+// Batch mode: the query blocks of several requests in one launch, as a list of
+// work items (a kernel argument, so no device copy of the plan is needed).
+// Item: query block qb (kBM rows) of request req over its key tiles [t0, t1);
+// slot >= 0: the tiles are a share of the block's, O and (max, sum) go to that
+// workspace slot for prefill_batch_merge_kernel.
+struct PrefillReq {
+  int q0, lq;  // first row in q and o, query rows
+  int k0, lk;  // first row in the K / V source, keys
+  int src;     // 0: k, v; 1: k2, v2
+};
+struct PrefillItem {
+  uint32_t req_qb;  // req | qb << 6
+  int t0, t1, slot;
+};
+constexpr int kBatchReqs = 64, kBatchItems = 160;
+struct PrefillBatch {
+  const void* q;
+  const _Float16* k;
+  const _Float16* v;
+  const _Float16* k2;
+  const _Float16* v2;
+  void* o;
+  int64_t q_st, q_sh, k_st, k_sh, v_st, v_sh, k2_st, k2_sh, o_st, o_sh;  // in elements
+  int ratio, hd;      // hd <= kD: dims of q and o rows (zero padded to kD here)
+  int q_bf16, o_bf16;  // q / o element type (else fp16)
+  float c;             // sm_scale * log2(e)
+  _Float16* ws_o;      // [slot][kBM 128][Hq][kD]
+  float* ws_ml;        // [slot][128][Hq][2]
+  PrefillReq reqs[kBatchReqs];
+  PrefillItem items[kBatchItems];
+};
+static_assert(sizeof(PrefillBatch) <= 4096, "kernel argument");
+
+// eight bf16 as eight fp16, round to nearest even (exact in fp16's range)
+__device__ __forceinline__ u32x4 bf16_to_f16(u32x4 x) {
+  u32x4 r;
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+    r[i] = pack_h2(__uint_as_float(x[i] << 16), __uint_as_float(x[i] & 0xffff0000u));
+  return r;
+}
+
+// two floats as a bf16 pair, round to nearest even
+__device__ __forceinline__ uint32_t pack_b2(float a, float b) {
+  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf2));
+}
+
 // max / sum of x over lanes l and l ^ 32: v_permlane32_swap of x with
 // itself returns (x, x of lane l ^ 32) in some order in every lane
 __device__ __forceinline__ float max32(float x) {
@@ -97,12 +152,72 @@ __device__ __forceinline__ float sum32(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// what one workgroup computes: rows qb kBM .. of a request (query rows from
+// q_row0) over its key tiles [t0, t1)
+struct PrefillWork {
+  int qb, q_row0, lq, lk, t0, t1, slot, hd;
+  const _Float16* k;
+  const _Float16* v;
+  int64_t k_st, k_sh, v_st, v_sh;
+};
+
+template <int kBM, int kBN, bool SPLIT>
+__device__ __forceinline__ PrefillWork prefill_work(const PrefillParams& p) {
+  PrefillWork r;
+  r.qb = p.nqb - 1 - (int)blockIdx.y;
+  r.q_row0 = 0;
+  r.lq = p.lq;
+  r.lk = p.lk;
+  r.slot = -1;
+  r.hd = 0;
+  r.k = p.k;
+  r.v = p.v;
+  r.k_st = p.k_st;
+  r.k_sh = p.k_sh;
+  r.v_st = p.v_st;
+  r.v_sh = p.v_sh;
+  const int q0 = r.qb * kBM;
+  const int kend = min(p.lk, p.lk - p.lq + min(q0 + kBM, p.lq));  // keys any row here sees
+  r.t0 = 0;
+  r.t1 = (kend + kBN - 1) / kBN;
+  if constexpr (SPLIT) {
+    r.t0 = (int)blockIdx.z * p.tps;
+    r.t1 = min(r.t1, r.t0 + p.tps);
+  }
+  return r;
+}
+
+template <int kBM, int kBN, bool SPLIT>
+__device__ __forceinline__ PrefillWork prefill_work(const PrefillBatch& p) {
+  const PrefillItem it = p.items[blockIdx.y];
+  const PrefillReq rq = p.reqs[it.req_qb & 63u];
+  PrefillWork r;
+  r.qb = (int)(it.req_qb >> 6);
+  r.q_row0 = rq.q0;
+  r.lq = rq.lq;
+  r.lk = rq.lk;
+  r.t0 = it.t0;
+  r.t1 = it.t1;
+  r.slot = it.slot;
+  r.hd = p.hd;
+  r.k_st = rq.src ? p.k2_st : p.k_st;
+  r.k_sh = rq.src ? p.k2_sh : p.k_sh;
+  r.v_st = rq.src ? p.k2_st : p.v_st;
+  r.v_sh = rq.src ? p.k2_sh : p.v_sh;
+  r.k = (rq.src ? p.k2 : p.k) + (int64_t)rq.k0 * r.k_st;
+  r.v = (rq.src ? p.v2 : p.v) + (int64_t)rq.k0 * r.v_st;
+  return r;
+}
+
 // WPE: waves per SIMD the register budget is sized for (2 at head size 64
 // and 128; 1 at 256, whose q operand and output accumulators alone take 192
 // registers per lane)
-template <int kD, int NW, int kBN, bool SPLIT, int WPE = 2>
+//
+// PP: PrefillParams (one request, SPLIT: its split-KV mode) or PrefillBatch.
+template <int kD, int NW, int kBN, bool SPLIT, int WPE = 2, class PP = PrefillParams>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
-void prefill_kernel(PrefillParams p) {
+void prefill_kernel(PP p) {
+  constexpr bool kBatch = std::is_same_v<PP, PrefillBatch>;
   constexpr int kKRow = kD * 2;       // bytes of one K row in LDS
   constexpr int kCH = kD / 8;         // 16-byte chunks per K row
   constexpr int kRPC = 1024 / kKRow;  // K rows per 1 KB copy
@@ -119,23 +234,25 @@ void prefill_kernel(PrefillParams p) {
   const int lane = threadIdx.x & 63;
   const int w = threadIdx.x >> 6;
   const int hh = lane >> 5, n = lane & 31;
-  const int qb = p.nqb - 1 - (int)blockIdx.y;
   const int head = blockIdx.x, g = head / p.ratio;
-  const int q0 = qb * kBM;
-  const int off = p.lk - p.lq;
-  const int qrow = q0 + 32 * w + n;  // this lane's query row
-  const int kend = min(p.lk, off + min(q0 + kBM, p.lq));  // keys any row here sees
-  const int ntiles = (kend + kBN - 1) / kBN;
+  const PrefillWork wk = prefill_work<kBM, kBN, SPLIT>(p);
+  const int q0 = wk.qb * kBM;
+  const int off = wk.lk - wk.lq;
+  const int qrow = q0 + 32 * w + n;  // this lane's query row (of its request)
 
   // q^T as the B operand of S^T = K Q^T: k-step s covers dims 16s .. 16s+15,
   // lane (hh, n) holds dims 16s + 8hh .. +7 of query row qrow
   half8_t qB[kD / 16];
   {
-    const _Float16* qp = p.q + (int64_t)qrow * p.q_st + (int64_t)head * p.q_sh + 8 * hh;
+    const int64_t qo = (int64_t)(wk.q_row0 + qrow) * p.q_st + (int64_t)head * p.q_sh + 8 * hh;
+    const _Float16* qp = static_cast<const _Float16*>(p.q) + qo;  // (bf16: the same size)
 #pragma unroll
     for (int s = 0; s < kD / 16; s++) {
       u32x4 x = {0u, 0u, 0u, 0u};
-      if (qrow < p.lq) x = *reinterpret_cast<const u32x4*>(qp + 16 * s);
+      if (qrow < wk.lq && (!kBatch || 16 * s + 8 * hh < wk.hd))
+        x = *reinterpret_cast<const u32x4*>(qp + 16 * s);
+      if constexpr (kBatch)
+        if (p.q_bf16) x = bf16_to_f16(x);
       qB[s] = __builtin_bit_cast(half8_t, x);
     }
   }
@@ -150,7 +267,7 @@ void prefill_kernel(PrefillParams p) {
   // lets their addresses be a per-lane base xor 64 d plus an immediate).
   // Wave w issues copies j = w + NW i of both.
   constexpr int kKC = (kBN / kRPC) / NW;  // copies per wave, tile and tensor
-  const int kst_b = (int)(p.k_st * 2), vst_b = (int)(p.v_st * 2);
+  const int kst_b = (int)(wk.k_st * 2), vst_b = (int)(wk.v_st * 2);
   uint32_t koff[kKC], voff[kKC];  // per-lane byte offsets of this wave's copies in a tile
 #pragma unroll
   for (int i = 0; i < kKC; i++) {
@@ -161,7 +278,7 @@ void prefill_kernel(PrefillParams p) {
   // buffer resource over rows [kb, Lk) of a K or V tile (wave-uniform base
   // and size; rows past Lk read as zeros)
   auto tile_rsrc = [&](const _Float16* base, int64_t st, int kb) {
-    const int rows = min(kBN, p.lk - kb);
+    const int rows = min(kBN, wk.lk - kb);
     const uint64_t a = (uint64_t)(uintptr_t)(base + (int64_t)kb * st);
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
     const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
@@ -169,12 +286,12 @@ void prefill_kernel(PrefillParams p) {
     return __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)(((uint64_t)hi << 32) | lo),
                                              (short)0, nrec, 0x00020000);
   };
-  const _Float16* const kbase = p.k + (int64_t)g * p.k_sh;
-  const _Float16* const vbase = p.v + (int64_t)g * p.v_sh;
+  const _Float16* const kbase = wk.k + (int64_t)g * wk.k_sh;
+  const _Float16* const vbase = wk.v + (int64_t)g * wk.v_sh;
   auto issue = [&](int kt, uint8_t* kb, uint8_t* vb) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the LDS-copy builtin has no host form
-    const __amdgpu_buffer_rsrc_t rk = tile_rsrc(kbase, p.k_st, kt * kBN);
-    const __amdgpu_buffer_rsrc_t rv = tile_rsrc(vbase, p.v_st, kt * kBN);
+    const __amdgpu_buffer_rsrc_t rk = tile_rsrc(kbase, wk.k_st, kt * kBN);
+    const __amdgpu_buffer_rsrc_t rv = tile_rsrc(vbase, wk.v_st, kt * kBN);
 #pragma unroll
     for (int i = 0; i < kKC; i++) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (void*)(kb + 1024 * (w + NW * i)), 16,
@@ -251,8 +368,8 @@ void prefill_kernel(PrefillParams p) {
     // score at tile key 4 hh + kk gets -inf (the sign bits of lim - kk spread
     // into 0xff800000) or +0 added; no compare masks, so no scalar registers
     // for them
-    if (kb + kBN - 1 > off + q0 + 32 * w || kb + kBN > p.lk) {
-      const int lim = min(qlim, p.lk - 1) - kb - 4 * hh;
+    if (kb + kBN - 1 > off + q0 + 32 * w || kb + kBN > wk.lk) {
+      const int lim = min(qlim, wk.lk - 1) - kb - 4 * hh;
 #pragma unroll
       for (int u = 0; u < kNU; u++)
 #pragma unroll
@@ -338,11 +455,7 @@ void prefill_kernel(PrefillParams p) {
   };
 
   // this workgroup's tiles: all of them, or split z's share
-  int t0 = 0, t1 = ntiles;
-  if constexpr (SPLIT) {
-    t0 = (int)blockIdx.z * p.tps;
-    t1 = min(ntiles, t0 + p.tps);
-  }
+  const int t0 = wk.t0, t1 = wk.t1;
   if (t0 < t1) issue(t0, kbuf0, vbuf0);
   for (int kt = t0; kt < t1; kt += 2) {
     // tile kt: buffers 0
@@ -358,14 +471,15 @@ void prefill_kernel(PrefillParams p) {
     tile(kt + 1, kbuf1, vbuf1);
   }
 
-  if constexpr (SPLIT) {
+  lsum = sum32(lsum);
+  const float inv = lsum > 0.0f ? 1.0f / lsum : 0.0f;
+  if (SPLIT || (kBatch && wk.slot >= 0)) {
     // this split's O / row sum (a convex combination of V rows: fp16 is
     // safe) and (mc, row sum); a split that held no visible key for a row
     // leaves mc = -inf, sum 0, O = 0
-    lsum = sum32(lsum);
-    if (qrow < p.lq) {
-      const int64_t r = ((int64_t)blockIdx.z * p.lq + qrow) * gridDim.x + head;
-      const float inv = lsum > 0.0f ? 1.0f / lsum : 0.0f;
+    if (qrow < wk.lq) {
+      const int64_t r = (kBatch ? (int64_t)wk.slot * kBM + 32 * w + n
+                                : (int64_t)blockIdx.z * wk.lq + qrow) * gridDim.x + head;
       _Float16* const wo = p.ws_o + r * kD + 4 * hh;
 #pragma unroll
       for (int d = 0; d < kD / 32; d++)
@@ -381,17 +495,20 @@ void prefill_kernel(PrefillParams p) {
   }
 
   // o = O / sum, lane (hh, n) holds dims 32d + 8jq + 4hh + 0..3 of row qrow
-  lsum = sum32(lsum);
-  if (qrow < p.lq) {
-    const float inv = lsum > 0.0f ? 1.0f / lsum : 0.0f;
-    _Float16* op = p.o + (int64_t)qrow * p.o_st + (int64_t)head * p.o_sh + 4 * hh;
+  if (qrow < wk.lq) {
+    _Float16* op = static_cast<_Float16*>(p.o) + (int64_t)(wk.q_row0 + qrow) * p.o_st +
+                   (int64_t)head * p.o_sh + 4 * hh;
 #pragma unroll
     for (int d = 0; d < kD / 32; d++)
 #pragma unroll
       for (int jq = 0; jq < 4; jq++) {
-        const uint32_t lo = pack_h2(oacc[d][4 * jq] * inv, oacc[d][4 * jq + 1] * inv);
-        const uint32_t hi = pack_h2(oacc[d][4 * jq + 2] * inv, oacc[d][4 * jq + 3] * inv);
-        *reinterpret_cast<u32x2*>(op + 32 * d + 8 * jq) = u32x2{lo, hi};
+        const float f0 = oacc[d][4 * jq] * inv, f1 = oacc[d][4 * jq + 1] * inv;
+        const float f2 = oacc[d][4 * jq + 2] * inv, f3 = oacc[d][4 * jq + 3] * inv;
+        if (kBatch && 32 * d + 8 * jq + 4 * hh >= wk.hd) continue;
+        u32x2 r = {pack_h2(f0, f1), pack_h2(f2, f3)};
+        if constexpr (kBatch)
+          if (p.o_bf16) r = u32x2{pack_b2(f0, f1), pack_b2(f2, f3)};
+        *reinterpret_cast<u32x2*>(op + 32 * d + 8 * jq) = r;
       }
   }
 }
@@ -403,9 +520,10 @@ void prefill_kernel(PrefillParams p) {
 // (RB 2, 64-key tiles: 217 VGPRs, two waves per SIMD), where the registers
 // of two row blocks fit; at head size 128 they do not (one wave per SIMD,
 // measured slower).
-template <int kD, int NW, int kBN, int RB, int WPE>
+template <int kD, int NW, int kBN, int RB, int WPE, class PP = PrefillParams>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
-void prefill_rb_kernel(PrefillParams p) {
+void prefill_rb_kernel(PP p) {
+  constexpr bool kBatch = std::is_same_v<PP, PrefillBatch>;
   constexpr int kKRow = kD * 2;
   constexpr int kCH = kD / 8;
   constexpr int kRPC = 1024 / kKRow;
@@ -420,29 +538,32 @@ void prefill_rb_kernel(PrefillParams p) {
   const int lane = threadIdx.x & 63;
   const int w = threadIdx.x >> 6;
   const int hh = lane >> 5, n = lane & 31;
-  const int qb = p.nqb - 1 - (int)blockIdx.y;
   const int head = blockIdx.x, g = head / p.ratio;
-  const int q0 = qb * kBM;
-  const int off = p.lk - p.lq;
+  const PrefillWork wk = prefill_work<kBM, kBN, false>(p);
+  const int q0 = wk.qb * kBM;
+  const int off = wk.lk - wk.lq;
   const int wrow0 = q0 + 32 * RB * w;  // the wave's first row
-  const int kend = min(p.lk, off + min(q0 + kBM, p.lq));
-  const int ntiles = (kend + kBN - 1) / kBN;
+  const int ntiles = wk.t1;
 
   half8_t qB[RB][kD / 16];
 #pragma unroll
   for (int rb = 0; rb < RB; rb++) {
     const int qrow = wrow0 + 32 * rb + n;
-    const _Float16* qp = p.q + (int64_t)qrow * p.q_st + (int64_t)head * p.q_sh + 8 * hh;
+    const int64_t qo = (int64_t)(wk.q_row0 + qrow) * p.q_st + (int64_t)head * p.q_sh + 8 * hh;
+    const _Float16* qp = static_cast<const _Float16*>(p.q) + qo;  // (bf16: the same size)
 #pragma unroll
     for (int s = 0; s < kD / 16; s++) {
       u32x4 x = {0u, 0u, 0u, 0u};
-      if (qrow < p.lq) x = *reinterpret_cast<const u32x4*>(qp + 16 * s);
+      if (qrow < wk.lq && (!kBatch || 16 * s + 8 * hh < wk.hd))
+        x = *reinterpret_cast<const u32x4*>(qp + 16 * s);
+      if constexpr (kBatch)
+        if (p.q_bf16) x = bf16_to_f16(x);
       qB[rb][s] = __builtin_bit_cast(half8_t, x);
     }
   }
 
   constexpr int kKC = (kBN / kRPC) / NW;
-  const int kst_b = (int)(p.k_st * 2), vst_b = (int)(p.v_st * 2);
+  const int kst_b = (int)(wk.k_st * 2), vst_b = (int)(wk.v_st * 2);
   uint32_t koff[kKC], voff[kKC];
 #pragma unroll
   for (int i = 0; i < kKC; i++) {
@@ -451,7 +572,7 @@ void prefill_rb_kernel(PrefillParams p) {
     voff[i] = (uint32_t)(row * vst_b + (((lane % kCH) ^ (4 * ((row & 3) >> kQS))) * 16));
   }
   auto tile_rsrc = [&](const _Float16* base, int64_t st, int kb) {
-    const int rows = min(kBN, p.lk - kb);
+    const int rows = min(kBN, wk.lk - kb);
     const uint64_t a = (uint64_t)(uintptr_t)(base + (int64_t)kb * st);
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
     const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
@@ -459,12 +580,12 @@ void prefill_rb_kernel(PrefillParams p) {
     return __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)(((uint64_t)hi << 32) | lo),
                                              (short)0, nrec, 0x00020000);
   };
-  const _Float16* const kbase = p.k + (int64_t)g * p.k_sh;
-  const _Float16* const vbase = p.v + (int64_t)g * p.v_sh;
+  const _Float16* const kbase = wk.k + (int64_t)g * wk.k_sh;
+  const _Float16* const vbase = wk.v + (int64_t)g * wk.v_sh;
   auto issue = [&](int kt, uint8_t* kb, uint8_t* vb) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    const __amdgpu_buffer_rsrc_t rk = tile_rsrc(kbase, p.k_st, kt * kBN);
-    const __amdgpu_buffer_rsrc_t rv = tile_rsrc(vbase, p.v_st, kt * kBN);
+    const __amdgpu_buffer_rsrc_t rk = tile_rsrc(kbase, wk.k_st, kt * kBN);
+    const __amdgpu_buffer_rsrc_t rv = tile_rsrc(vbase, wk.v_st, kt * kBN);
 #pragma unroll
     for (int i = 0; i < kKC; i++) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (void*)(kb + 1024 * (w + NW * i)), 16,
@@ -538,8 +659,8 @@ void prefill_rb_kernel(PrefillParams p) {
 #pragma unroll
     for (int rb = 0; rb < RB; rb++) {
       const int rfirst = wrow0 + 32 * rb;
-      if (kb + kBN - 1 > off + rfirst || kb + kBN > p.lk) {
-        const int lim = min(off + rfirst + n, p.lk - 1) - kb - 4 * hh;
+      if (kb + kBN - 1 > off + rfirst || kb + kBN > wk.lk) {
+        const int lim = min(off + rfirst + n, wk.lk - 1) - kb - 4 * hh;
 #pragma unroll
         for (int u = 0; u < kNU; u++)
 #pragma unroll
@@ -624,18 +745,21 @@ void prefill_rb_kernel(PrefillParams p) {
   for (int rb = 0; rb < RB; rb++) {
     const int qrow = wrow0 + 32 * rb + n;
     const float ls = sum32(lsum[rb]);
-    if (qrow < p.lq) {
+    if (qrow < wk.lq) {
       const float inv = ls > 0.0f ? 1.0f / ls : 0.0f;
-      _Float16* op = p.o + (int64_t)qrow * p.o_st + (int64_t)head * p.o_sh + 4 * hh;
+      _Float16* op = static_cast<_Float16*>(p.o) + (int64_t)(wk.q_row0 + qrow) * p.o_st +
+                     (int64_t)head * p.o_sh + 4 * hh;
 #pragma unroll
       for (int d = 0; d < kD / 32; d++)
 #pragma unroll
         for (int jq = 0; jq < 4; jq++) {
-          const uint32_t lo =
-              pack_h2(oacc[rb][d][4 * jq] * inv, oacc[rb][d][4 * jq + 1] * inv);
-          const uint32_t hi =
-              pack_h2(oacc[rb][d][4 * jq + 2] * inv, oacc[rb][d][4 * jq + 3] * inv);
-          *reinterpret_cast<u32x2*>(op + 32 * d + 8 * jq) = u32x2{lo, hi};
+          const float f0 = oacc[rb][d][4 * jq] * inv, f1 = oacc[rb][d][4 * jq + 1] * inv;
+          const float f2 = oacc[rb][d][4 * jq + 2] * inv, f3 = oacc[rb][d][4 * jq + 3] * inv;
+          if (kBatch && 32 * d + 8 * jq + 4 * hh >= wk.hd) continue;
+          u32x2 r = {pack_h2(f0, f1), pack_h2(f2, f3)};
+          if constexpr (kBatch)
+            if (p.o_bf16) r = u32x2{pack_b2(f0, f1), pack_b2(f2, f3)};
+          *reinterpret_cast<u32x2*>(op + 32 * d + 8 * jq) = r;
         }
     }
   }
@@ -671,6 +795,57 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p, int
   for (int i = 0; i < V; i++) op[i] = (_Float16)(acc[i] * inv);
 }
 
+// Merge of the split query blocks of a batch: D / 8 lanes per (row, q head), 8
+// dims (16 bytes) each, the same weights as above.
+struct PrefillGroup {
+  int q_row, slot0;  // the block's first row in o, its first slot
+  uint16_t nsplit, rows;
+};
+struct PrefillMerge {
+  void* o;
+  int64_t o_st, o_sh;
+  int hq, hd, o_bf16;
+  const _Float16* ws_o;
+  const float* ws_ml;
+  PrefillGroup groups[kBatchItems];
+};
+
+template <int kD>
+__global__ __launch_bounds__(256) void prefill_batch_merge_kernel(PrefillMerge p) {
+  constexpr int L = kD / 8, kVecs = 256 / L;
+  const PrefillGroup g = p.groups[blockIdx.y];
+  const int idx = (int)blockIdx.x * kVecs + (int)threadIdx.x / L;  // row * hq + head
+  const int c = 8 * ((int)threadIdx.x % L);
+  if (idx >= g.rows * p.hq) return;
+  const int row = idx / p.hq, head = idx % p.hq;
+  const int64_t zs = (int64_t)128 * p.hq;  // vectors of one slot
+  const int64_t v0 = g.slot0 * zs + idx;
+  float mx = -INFINITY;
+  for (int z = 0; z < g.nsplit; z++) mx = fmaxf(mx, p.ws_ml[2 * (v0 + z * zs)]);
+  float den = 0.0f, acc[8];
+#pragma unroll
+  for (int i = 0; i < 8; i++) acc[i] = 0.0f;
+#pragma unroll 4
+  for (int z = 0; z < g.nsplit; z++) {
+    const f32x2 ml = *reinterpret_cast<const f32x2*>(p.ws_ml + 2 * (v0 + z * zs));
+    const half8_t x = *reinterpret_cast<const half8_t*>(p.ws_o + (v0 + z * zs) * kD + c);
+    // a split without a visible key for the row has weight 0 (its O is 0)
+    const float wgt = ml[0] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml[0] - mx) * ml[1];
+    den += wgt;
+#pragma unroll
+    for (int i = 0; i < 8; i++) acc[i] = __builtin_fmaf(wgt, (float)x[i], acc[i]);
+  }
+  if (c >= p.hd) return;
+  const float inv = den > 0.0f ? 1.0f / den : 0.0f;
+  u32x4 r;
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+    r[i] = p.o_bf16 ? pack_b2(acc[2 * i] * inv, acc[2 * i + 1] * inv)
+                    : pack_h2(acc[2 * i] * inv, acc[2 * i + 1] * inv);
+  *reinterpret_cast<u32x4*>(static_cast<_Float16*>(p.o) + (int64_t)(g.q_row + row) * p.o_st +
+                            (int64_t)head * p.o_sh + c) = r;
+}
+
 // the workgroup shapes, at head size 64 or 128: 256 query rows (eight waves
 // with 128-key tiles at head size 128; four waves of two row blocks with
 // 64-key tiles at head size 64); four waves, 64-key tiles; four waves split
@@ -693,13 +868,13 @@ hipError_t launch_prefill(int nw, int heads, hipStream_t st, const PrefillParams
       hipLaunchKernelGGL((prefill_merge_kernel<D>), dim3((unsigned)((waves + 3) / 4)), dim3(256),
                          0, st, p, heads);
     }
-  } else if (nw == 8 && D == 64) {
-    // head size 64: four waves of 64 rows (two row blocks each), 64-key tiles
-    hipLaunchKernelGGL((prefill_rb_kernel<D, 4, 64, 2, 2>), dim3(heads, p.nqb), dim3(256), 0, st,
-                       p);
   } else if (nw == 8) {
-    hipLaunchKernelGGL((prefill_kernel<D, 8, 128, false>), dim3(heads, p.nqb), dim3(512), 0, st,
-                       p);
+    if constexpr (D == 64)  // four waves of 64 rows (two row blocks each), 64-key tiles
+      hipLaunchKernelGGL((prefill_rb_kernel<D, 4, 64, 2, 2>), dim3(heads, p.nqb), dim3(256), 0, st,
+                         p);
+    else
+      hipLaunchKernelGGL((prefill_kernel<D, 8, 128, false>), dim3(heads, p.nqb), dim3(512), 0, st,
+                         p);
   } else if (p.nsplit <= 1) {
     hipLaunchKernelGGL((prefill_kernel<D, 4, 64, false>), dim3(heads, p.nqb), dim3(256), 0, st,
                        p);
@@ -751,8 +926,340 @@ PrefillPlan plan_prefill(int q_len, int kv_len, int heads, int head_dim) {
   return sp;
 }
 
+// Plan of one batch of at most kBatchReqs requests: its items (longest first)
+// and the split query blocks.
+struct BatchPlan {
+  int nw = 4;
+  int slots = 0;
+  std::vector<PrefillItem> items;
+  std::vector<PrefillGroup> groups;  // q_row: of the request (group_req)
+  std::vector<int> group_req;
+};
+
+struct QueryBlock {
+  int req, qb, tiles;
+};
+
+// Time of a list of items (tiles each, longest first) in tiles: `groups` sets
+// of workgroup slots, one workgroup per q head in each, take the items in
+// turn as they fall free; an item costs its tiles and about one for its start.
+template <class Tiles>
+double batch_time(size_t n, double groups, Tiles tiles) {
+  if (groups < 1.0) groups = 1.0;
+  double total = 0.0;
+  if (n > 512 || n <= groups) {
+    for (size_t i = 0; i < n; i++) total += tiles(i) + 1.0;
+    return n == 0 ? 0.0 : std::max(tiles(0) + 1.0, total / groups);
+  }
+  std::vector<double> busy((size_t)groups, 0.0);  // a heap, the first to fall free on top
+  auto later = [](double x, double y) { return x > y; };
+  for (size_t i = 0; i < n; i++) {
+    std::pop_heap(busy.begin(), busy.end(), later);
+    busy.back() += tiles(i) + 1.0;
+    total = std::max(total, busy.back());
+    std::push_heap(busy.begin(), busy.end(), later);
+  }
+  return total;
+}
+
+std::vector<QueryBlock> query_blocks(const int32_t* q_lens, const int32_t* kv_lens, int nreq,
+                                     int bm, int bn) {
+  std::vector<QueryBlock> blocks;
+  for (int i = 0; i < nreq; i++)
+    for (int qb = 0; (int64_t)qb * bm < q_lens[i]; qb++) {
+      const int kend = kv_lens[i] - q_lens[i] + std::min((qb + 1) * bm, q_lens[i]);
+      blocks.push_back({i, qb, (kend + bn - 1) / bn});
+    }
+  std::stable_sort(blocks.begin(), blocks.end(),
+                   [](const QueryBlock& x, const QueryBlock& y) { return x.tiles > y.tiles; });
+  return blocks;
+}
+
+// Shape and splits by estimated time.  Measured at 32 q heads, head size 128
+// on 256 CUs: a 256-row, 128-key tile takes 3.84 us of a CU (one workgroup),
+// a 128-row, 64-key tile 2.1 us (two resident); at head size 64 both shapes
+// run two workgroups per CU, 2.15 and 1.15 us a tile.  So 256-row blocks win
+// where they waste few rows and fill whole rounds (2048 tokens over 30k: 947
+// against 1008 us; a 4096-token prompt 140 against 152 us) and 128-row blocks
+// elsewhere (five prompts of 229 .. 1326 tokens 55 against 61 us; six of 1300
+// 126 against 147 us).  Splitting the keys of 128-row blocks pays where few
+// blocks leave slots idle (256 tokens over 32k: 155 against 669 us) and costs
+// the merge, 4 .. 9 us.
+BatchPlan plan_batch(const int32_t* q_lens, const int32_t* kv_lens, int nreq, int heads,
+                     int head_dim) {
+  BatchPlan bp;
+  const double cus = device_cus() > 0 ? device_cus() : 256;
+  std::vector<QueryBlock> blocks = query_blocks(q_lens, kv_lens, nreq, 128, 64);
+  const double groups = (head_dim == 256 ? 1.0 : 2.0) * cus / heads;
+  int64_t total = 0;
+  for (const QueryBlock& b : blocks) total += b.tiles;
+  // the parts of a block of t tiles at most `unit` tiles each
+  auto parts = [](int t, double unit) {
+    return t > 1.25 * unit ? (int)std::ceil(t / unit) : 1;
+  };
+  double best = batch_time(blocks.size(), groups, [&](size_t i) { return blocks[i].tiles; });
+  double unit = 1e30;
+  if (!blocks.empty() && blocks.size() <= 4 * groups) {
+    const double even = std::max(8.0, total / groups);  // tiles per slot, at least 512 keys
+    for (const double f : {1.5, 1.05, 0.8, 0.5}) {
+      const double u = std::max(8.0, f * even);
+      int slots = 0;
+      std::vector<double> cost;
+      for (const QueryBlock& b : blocks) {
+        const int ns = parts(b.tiles, u);
+        if (ns > 1) slots += ns;
+        cost.insert(cost.end(), ns, (double)((b.tiles + ns - 1) / ns));
+      }
+      if (slots == 0) continue;
+      std::sort(cost.begin(), cost.end(), [](double x, double y) { return x > y; });
+      // the merge: its launch and the slots' rows written and read
+      const double t = batch_time(cost.size(), groups, [&](size_t i) { return cost[i]; }) + 2.0 +
+                       0.3 * slots * heads / 32.0;
+      if (t < best) {
+        best = t;
+        unit = u;
+      }
+    }
+  }
+  if (head_dim != 256) {
+    const std::vector<QueryBlock> wide =
+        query_blocks(q_lens, kv_lens, nreq, 256, head_dim == 128 ? 128 : 64);
+    const double t = batch_time(wide.size(), (head_dim == 128 ? 1.0 : 2.0) * cus / heads,
+                                [&](size_t i) { return wide[i].tiles; });
+    if (head_dim == 128 ? t * 3.84 <= best * 2.1 : t * 2.15 <= best * 1.15) {
+      bp.nw = 8;
+      unit = 1e30;
+      blocks = wide;
+    }
+  }
+  const int bm = bp.nw == 8 ? 256 : 128;
+  for (const QueryBlock& b : blocks) {
+    int ns = parts(b.tiles, unit);
+    const int per = (b.tiles + ns - 1) / ns;
+    ns = (b.tiles + per - 1) / per;
+    const int slot0 = bp.slots;
+    for (int z = 0; z < ns; z++)
+      bp.items.push_back({(uint32_t)b.req | (uint32_t)b.qb << 6, z * per,
+                          std::min(b.tiles, (z + 1) * per), ns > 1 ? slot0 + z : -1});
+    if (ns > 1) {
+      bp.slots += ns;
+      bp.groups.push_back({b.qb * bm, slot0, (uint16_t)ns,
+                           (uint16_t)std::min(bm, q_lens[b.req] - b.qb * bm)});
+      bp.group_req.push_back(b.req);
+    }
+  }
+  std::stable_sort(bp.items.begin(), bp.items.end(), [](const PrefillItem& x, const PrefillItem& y) {
+    return x.t1 - x.t0 > y.t1 - y.t0;
+  });
+  return bp;
+}
+
+template <int D>
+hipError_t launch_batch(const BatchPlan& bp, int heads, hipStream_t st, PrefillBatch& p) {
+  for (size_t a = 0; a < bp.items.size(); a += kBatchItems) {
+    const unsigned n = (unsigned)std::min<size_t>(kBatchItems, bp.items.size() - a);
+    std::copy_n(bp.items.begin() + a, n, p.items);
+    const dim3 grid(heads, n);
+    if (bp.nw == 8) {
+      if constexpr (D == 64)
+        hipLaunchKernelGGL((prefill_rb_kernel<D, 4, 64, 2, 2, PrefillBatch>), grid, dim3(256), 0,
+                           st, p);
+      else if constexpr (D == 128)
+        hipLaunchKernelGGL((prefill_kernel<D, 8, 128, false, 2, PrefillBatch>), grid, dim3(512), 0,
+                           st, p);
+    } else {
+      hipLaunchKernelGGL((prefill_kernel<D, 4, 64, false, D == 256 ? 1 : 2, PrefillBatch>), grid,
+                         dim3(256), 0, st, p);
+    }
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  PrefillMerge m;
+  m.o = p.o;
+  m.o_st = p.o_st;
+  m.o_sh = p.o_sh;
+  m.hq = heads;
+  m.hd = p.hd;
+  m.o_bf16 = p.o_bf16;
+  m.ws_o = p.ws_o;
+  m.ws_ml = p.ws_ml;
+  for (size_t a = 0; a < bp.groups.size(); a += kBatchItems) {
+    const unsigned n = (unsigned)std::min<size_t>(kBatchItems, bp.groups.size() - a);
+    int rows = 0;
+    for (unsigned i = 0; i < n; i++) {
+      m.groups[i] = bp.groups[a + i];
+      m.groups[i].q_row += p.reqs[bp.group_req[a + i]].q0;
+      rows = std::max<int>(rows, m.groups[i].rows);
+    }
+    constexpr int kVecs = 256 / (D / 8);
+    hipLaunchKernelGGL((prefill_batch_merge_kernel<D>), dim3((rows * heads + kVecs - 1) / kVecs, n),
+                       dim3(256), 0, st, m);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+// workspace of a plan: O rows, then (max, sum) pairs, of each slot's 128 rows
+int64_t batch_ws_bytes(const BatchPlan& bp, int heads, int head_dim) {
+  return (int64_t)bp.slots * 128 * heads * (head_dim * 2 + 8);
+}
+
+bool batch_sizes_ok(const int32_t* q_lens, const int32_t* kv_lens, int32_t nreq, int32_t heads,
+                    int32_t head_dim) {
+  if (nreq < 0 || heads <= 0 || (nreq > 0 && (!q_lens || !kv_lens)) ||
+      (head_dim != 64 && head_dim != 128 && head_dim != 256))
+    return false;
+  for (int i = 0; i < nreq; i++)
+    if (q_lens[i] < 0 || kv_lens[i] < q_lens[i] || q_lens[i] > (1 << 26)) return false;
+  return true;
+}
+
 }  // namespace
 }  // namespace tq
+
+extern "C" int64_t tq_prefill_batch_workspace_bytes(const int32_t* q_lens, const int32_t* kv_lens,
+                                                    int32_t num_requests, int32_t num_qo_heads,
+                                                    int32_t padded_dim) {
+  using namespace tq;
+  if (!batch_sizes_ok(q_lens, kv_lens, num_requests, num_qo_heads, padded_dim)) return 0;
+  int64_t most = 0;
+  try {
+    for (int a = 0; a < num_requests; a += kBatchReqs)
+      most = std::max(most, batch_ws_bytes(plan_batch(q_lens + a, kv_lens + a,
+                                                      std::min(kBatchReqs, num_requests - a),
+                                                      num_qo_heads, padded_dim),
+                                           num_qo_heads, padded_dim));
+  } catch (...) {
+    return 0;
+  }
+  return most;
+}
+
+extern "C" int tq_prefill_attention_batch(
+    const void* q, int64_t q_stride_tok, int64_t q_stride_head, int32_t q_dtype, const void* k,
+    int64_t k_stride_tok, int64_t k_stride_head, const void* v, int64_t v_stride_tok,
+    int64_t v_stride_head, const void* k2, const void* v2, int64_t k2_stride_tok,
+    int64_t k2_stride_head, void* o, int64_t o_stride_tok, int64_t o_stride_head, int32_t o_dtype,
+    const int32_t* q_starts, const int32_t* q_lens, const int32_t* kv_starts,
+    const int32_t* kv_lens, const int32_t* kv_sources, int32_t num_requests, int32_t num_qo_heads,
+    int32_t num_kv_heads, int32_t head_dim, int32_t padded_dim, float sm_scale, void* workspace,
+    int64_t workspace_bytes, tq_stream_t stream) {
+  using namespace tq;
+  const char* what = "prefill_attention_batch";
+  if (!batch_sizes_ok(q_lens, kv_lens, num_requests, num_qo_heads, padded_dim)) {
+    set_error("%s: bad sizes (padded_dim 64, 128 or 256; 0 <= q_len <= kv_len)", what);
+    return kEinval;
+  }
+  if (num_kv_heads <= 0 || num_qo_heads % num_kv_heads != 0) {
+    set_error("%s: num_qo_heads %d not a multiple of num_kv_heads %d", what, num_qo_heads,
+              num_kv_heads);
+    return kEinval;
+  }
+  if (head_dim <= 0 || head_dim > padded_dim || head_dim % 8 != 0) {
+    set_error("%s: head_dim %d must be a multiple of 8 up to padded_dim", what, head_dim);
+    return kEinval;
+  }
+  if ((q_dtype != TQ_F16 && q_dtype != TQ_BF16) || (o_dtype != TQ_F16 && o_dtype != TQ_BF16)) {
+    set_error("%s: q and o must be fp16 or bf16", what);
+    return kEinval;
+  }
+  if (num_requests == 0) return 0;
+  if (!q || !o || !q_starts || !kv_starts || !kv_sources) {
+    set_error("%s: null pointer", what);
+    return kEinval;
+  }
+  bool use1 = false, use2 = false;
+  for (int i = 0; i < num_requests; i++) {
+    if (q_starts[i] < 0 || kv_starts[i] < 0 || q_starts[i] > INT32_MAX - q_lens[i] - 256 ||
+        kv_starts[i] > INT32_MAX - kv_lens[i]) {
+      set_error("%s: bad request %d", what, i);
+      return kEinval;
+    }
+    (kv_sources[i] ? use2 : use1) = true;
+  }
+  if ((use1 && (!k || !v)) || (use2 && (!k2 || !v2))) {
+    set_error("%s: null pointer", what);
+    return kEinval;
+  }
+  const int64_t strides[10] = {q_stride_tok,  q_stride_head, o_stride_tok,  o_stride_head,
+                               k_stride_tok,  k_stride_head, v_stride_tok,  v_stride_head,
+                               k2_stride_tok, k2_stride_head};
+  for (int i = 0; i < 10; i++) {
+    if (i >= 4 && i < 8 && !use1) continue;
+    if (i >= 8 && !use2) continue;
+    if (strides[i] < 0 || strides[i] % 8 != 0) {
+      set_error("%s: strides must be non-negative multiples of 8 elements", what);
+      return kEinval;
+    }
+  }
+  // K and V rows are read to padded_dim
+  const int64_t lim = INT32_MAX / 2 / kBNmax;
+  if ((use1 && (k_stride_tok < padded_dim || v_stride_tok < padded_dim || k_stride_tok > lim ||
+                v_stride_tok > lim)) ||
+      (use2 && (k2_stride_tok < padded_dim || k2_stride_tok > lim))) {
+    set_error("%s: k / v token strides out of range", what);
+    return kEinval;
+  }
+  uintptr_t al = (uintptr_t)q | (uintptr_t)o | (uintptr_t)workspace;
+  if (use1) al |= (uintptr_t)k | (uintptr_t)v;
+  if (use2) al |= (uintptr_t)k2 | (uintptr_t)v2;
+  if (al & 15) {
+    set_error("%s: tensors must be 16-byte aligned", what);
+    return kEinval;
+  }
+  PrefillBatch p;
+  p.q = q;
+  p.k = static_cast<const _Float16*>(k);
+  p.v = static_cast<const _Float16*>(v);
+  p.k2 = static_cast<const _Float16*>(k2);
+  p.v2 = static_cast<const _Float16*>(v2);
+  p.o = o;
+  p.q_st = q_stride_tok;
+  p.q_sh = q_stride_head;
+  p.k_st = k_stride_tok;
+  p.k_sh = k_stride_head;
+  p.v_st = v_stride_tok;
+  p.v_sh = v_stride_head;
+  p.k2_st = k2_stride_tok;
+  p.k2_sh = k2_stride_head;
+  p.o_st = o_stride_tok;
+  p.o_sh = o_stride_head;
+  p.ratio = num_qo_heads / num_kv_heads;
+  p.hd = head_dim;
+  p.q_bf16 = q_dtype == TQ_BF16;
+  p.o_bf16 = o_dtype == TQ_BF16;
+  p.c = sm_scale * 1.4426950408889634f;
+  const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  try {
+    for (int a = 0; a < num_requests; a += kBatchReqs) {
+      const int n = std::min(kBatchReqs, num_requests - a);
+      const BatchPlan bp = plan_batch(q_lens + a, kv_lens + a, n, num_qo_heads, padded_dim);
+      if (batch_ws_bytes(bp, num_qo_heads, padded_dim) > (workspace ? workspace_bytes : 0)) {
+        set_error("%s: workspace smaller than tq_prefill_batch_workspace_bytes", what);
+        return kEinval;
+      }
+      p.ws_o = static_cast<_Float16*>(workspace);
+      p.ws_ml = reinterpret_cast<float*>(p.ws_o + (int64_t)bp.slots * 128 * num_qo_heads *
+                                                      padded_dim);
+      for (int i = 0; i < n; i++)
+        p.reqs[i] = {q_starts[a + i], q_lens[a + i], kv_starts[a + i], kv_lens[a + i],
+                     kv_sources[a + i] ? 1 : 0};
+      hipError_t e;
+      if (padded_dim == 64) e = launch_batch<64>(bp, num_qo_heads, st, p);
+      else if (padded_dim == 128) e = launch_batch<128>(bp, num_qo_heads, st, p);
+      else e = launch_batch<256>(bp, num_qo_heads, st, p);
+      if (e != hipSuccess) {
+        set_error("%s: launch failed: %s", what, hipGetErrorString(e));
+        return (int)e;
+      }
+    }
+  } catch (...) {
+    set_error("%s: out of host memory", what);
+    return (int)hipErrorOutOfMemory;
+  }
+  return 0;
+}
 
 extern "C" int64_t tq_prefill_workspace_bytes(int32_t q_len, int32_t kv_len, int32_t num_qo_heads,
                                               int32_t num_kv_heads, int32_t head_dim) {

@@ -18,6 +18,8 @@ only: CPU tensors raise.
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from . import _lib
@@ -249,6 +251,59 @@ def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torc
     return o
 
 
+def prefill_attention_batch(q: torch.Tensor, o: torch.Tensor, requests, num_kv_heads: int,
+                            head_dim: int, padded_dim: int, sm_scale: float,
+                            k: torch.Tensor | None = None, v: torch.Tensor | None = None,
+                            k2: torch.Tensor | None = None,
+                            v2: torch.Tensor | None = None) -> torch.Tensor:
+    """prefill_attention for several requests in one launch: `requests` are
+    (q_start, q_len, kv_start, kv_len, source) host integers, the request's
+    rows of q / o and of k / v (source 0) or k2 / v2 (source 1).  q and o fp16
+    or bf16 [tokens, Hq, head_dim]; K / V fp16 [tokens, Hkv, padded_dim], zero
+    past head_dim; head_dim a multiple of 8."""
+    kvs = [t for t in (k, v, k2, v2) if t is not None]
+    _require_gpu(q, o, *kvs)
+    hq = q.size(1)
+    if q.dim() != 3 or tuple(o.shape) != tuple(q.shape) or q.size(2) != head_dim:
+        raise RuntimeError("prefill_attention_batch: q / o must be [tokens, heads, head_dim]")
+    if q.dtype not in (torch.float16, torch.bfloat16) or \
+            o.dtype not in (torch.float16, torch.bfloat16) or q.stride(2) != 1 or o.stride(2) != 1:
+        raise RuntimeError("prefill_attention_batch: q / o must be fp16 or bf16 with contiguous "
+                           "dims")
+    for t in kvs:
+        if t.dtype != torch.float16 or t.dim() != 3 or t.stride(2) != 1 or \
+                tuple(t.shape[1:]) != (num_kv_heads, padded_dim):
+            raise RuntimeError("prefill_attention_batch: k / v must be fp16 [tokens, Hkv, "
+                               "padded_dim] with contiguous dims")
+    for a, b in ((k, v), (k2, v2)):
+        if (a is None) != (b is None) or (a is not None and a.size(0) != b.size(0)):
+            raise RuntimeError("prefill_attention_batch: k and v must go together")
+    if k2 is not None and k2.stride() != v2.stride():
+        raise RuntimeError("prefill_attention_batch: k2 and v2 must share their strides")
+    for qs, ql, ks, kl, src in requests:
+        kv = k2 if src else k
+        if qs < 0 or ql < 0 or qs + ql > q.size(0) or kv is None or ks < 0 or kl < ql \
+                or ks + kl > kv.size(0):
+            raise RuntimeError("prefill_attention_batch: a request is out of range")
+    n = len(requests)
+    cols = [(ctypes.c_int32 * max(1, n))(*c) for c in
+            (zip(*requests) if n else ((),) * 5)]
+    lib = _lib.load()
+    st = lambda t: (0, 0) if t is None else (t.stride(0), t.stride(1))
+    ptr = lambda t: None if t is None else t.data_ptr()
+    with torch.cuda.device(q.device):
+        nbytes = int(lib.tq_prefill_batch_workspace_bytes(cols[1], cols[3], n, hq,
+                                                          int(padded_dim)))
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes > 0 else None
+        rc = lib.tq_prefill_attention_batch(
+            q.data_ptr(), *st(q), _DTYPES[q.dtype], ptr(k), *st(k), ptr(v), *st(v), ptr(k2),
+            ptr(v2), *st(k2), o.data_ptr(), *st(o), _DTYPES[o.dtype], *cols, n, hq,
+            int(num_kv_heads), int(head_dim), int(padded_dim), float(sm_scale), ptr(ws), nbytes,
+            _stream_ptr(q.device))
+    _lib.check(rc, "prefill_attention_batch")
+    return o
+
+
 def dequant_paged(kv_cache: torch.Tensor, pages: torch.Tensor, num_tokens: int,
                   num_kv_heads: int, head_dim: int, padded_dim: int,
                   signs: torch.Tensor | None, out_k: torch.Tensor, out_v: torch.Tensor) -> None:
@@ -292,8 +347,74 @@ def dequant_paged(kv_cache: torch.Tensor, pages: torch.Tensor, num_tokens: int,
     _lib.check(rc, "dequant_paged")
 
 
+def prefill_gather(kv_cache: torch.Tensor | None, block_table: torch.Tensor | None,
+                   key: torch.Tensor, value: torch.Tensor, requests, head_dim: int,
+                   padded_dim: int, signs: torch.Tensor | None, out_k: torch.Tensor,
+                   out_v: torch.Tensor) -> None:
+    """The keys and values of several prefill requests as fp16 rows
+    [*, H_kv, padded_dim] in one launch (tq_prefill_gather): `requests` are
+    (table_row, ctx, fresh_start, fresh_len, out_start) host integers; the ctx
+    cached tokens of page-table row table_row are read back as dequant_paged
+    does, the fresh rows of key / value (fp16, bf16 or fp32) converted, both
+    zero-padded past head_dim.  kv_cache and block_table may be None when
+    every ctx is 0."""
+    _require_gpu(key, value, out_k, out_v)
+    if key.dtype not in _DTYPES or value.dtype != key.dtype:
+        raise RuntimeError(f"key/value must share a float dtype, got {key.dtype}/{value.dtype}")
+    if key.dim() != 3 or value.shape != key.shape or key.size(2) != head_dim \
+            or key.stride(2) != 1 or value.stride(2) != 1:
+        raise RuntimeError("prefill_gather: key/value must be [tokens, heads, head_dim] with "
+                           "contiguous dims")
+    h = key.size(1)
+    for t in (out_k, out_v):
+        if t.dtype != torch.float16 or t.dim() != 3 or tuple(t.shape[1:]) != (h, padded_dim) \
+                or not t.is_contiguous():
+            raise RuntimeError("prefill_gather: out_k / out_v must be contiguous fp16 "
+                               "[rows, H_kv, padded_dim]")
+    rows = min(out_k.size(0), out_v.size(0))
+    bs, nb, ebs, base, slab, bt, bt_rows = 16, 0, entry_bytes(head_dim)[2], 0, 0, 0, 0
+    if kv_cache is not None and block_table is not None:
+        _require_gpu(key, kv_cache, block_table)
+        if kv_cache.dim() != 5 or kv_cache.size(0) != 2 or not kv_cache.is_contiguous():
+            raise RuntimeError("kv_cache must be contiguous [2, num_blocks, block_size, H, ebs]")
+        _, nb, bs, hk, _ = kv_cache.shape
+        if hk != h:
+            raise RuntimeError(f"kv_cache has {hk} kv heads, num_kv_heads={h}")
+        if block_table.dtype != torch.int32 or block_table.dim() != 2 \
+                or block_table.stride(1) != 1:
+            raise RuntimeError("block_table must be int32 [requests, pages] with contiguous rows")
+        ebs = kv_cache.size(-1) * kv_cache.element_size()
+        base, slab, bt, bt_rows = kv_cache.data_ptr(), nb * bs * h * ebs, block_table.data_ptr(), \
+            block_table.size(0)
+    for row, ctx, fs, fl, dst in requests:
+        if ctx < 0 or fs < 0 or fl < 0 or dst < 0 or dst + ctx + fl > rows \
+                or fs + fl > key.size(0):
+            raise RuntimeError("prefill_gather: a request is out of range")
+        if ctx > 0 and (not bt or not 0 <= row < bt_rows):
+            raise RuntimeError("prefill_gather: cached context needs the cache and a table row")
+        if ctx > 0 and ctx > block_table.size(1) * bs:
+            raise RuntimeError("pages do not cover num_tokens")
+    sp = 0
+    if signs is not None and signs.numel() > 0:
+        if signs.dtype != torch.float32 or signs.numel() < padded_dim:
+            raise RuntimeError("signs must be fp32 [padded_dim]")
+        _require_gpu(key, signs)
+        sp = signs.data_ptr()
+    n = len(requests)
+    if n == 0:
+        return
+    cols = [(ctypes.c_int32 * n)(*c) for c in zip(*requests)]
+    lib = _lib.load()
+    with torch.cuda.device(key.device):
+        rc = lib.tq_prefill_gather(
+            base, base + slab, bt, block_table.stride(0) if bt else 0, h, int(head_dim),
+            int(padded_dim), bs, ebs, nb, sp, key.data_ptr(), value.data_ptr(),
+            _DTYPES[key.dtype], key.stride(0), key.stride(1), value.stride(0), value.stride(1),
+            *cols, n, out_k.data_ptr(), out_v.data_ptr(), _stream_ptr(key.device))
+    _lib.check(rc, "prefill_gather")
+
+
 def _host_f32(values) -> "ctypes.Array":
-    import ctypes
     vals = [float(v) for v in values]
     return (ctypes.c_float * max(1, len(vals)))(*vals)
 

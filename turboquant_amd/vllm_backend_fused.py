@@ -289,42 +289,80 @@ class TurboQuantFusedImpl(FlashAttentionImpl):
         both = torch.cat([dq.to(torch.int64), attn_metadata.seq_lens.to(torch.int64)]).cpu()
         return both[:n].tolist(), both[n:].tolist()
 
-    def _attend(self, q, k, v, ctx, out=None):
-        """q [ql, Hq, D] over k, v [ctx + ql, Hkv, D] (fp16), causal with the
-        queries at the end of the keys (lower-right alignment), in this
-        library's prefill kernel (tq_prefill_attention).  Head sizes 64, 128
-        and 256 run as they are, written into `out` when given (fp16
-        [ql, Hq, D]); a head size below its padded size (96, 80, ...) runs
-        zero-padded to it: zero dims add nothing to q.k and give zero output
-        dims, which are dropped.  The reference runs flash-attn here for
-        every head size (vllm_backend_fused.py:335-371)."""
+    def _attend_chunks(self, chunks, query, key, value, kv_cache, bt, output):
+        """Causal attention of the chunks (request, first row, q_len, ctx):
+        rows [a, a + ql) of query over the request's ctx cached tokens
+        followed by its fresh K/V, the queries at the end of the keys, written
+        to the same rows of output.  All chunks run in one launch of this
+        library's prefill kernel (tq_prefill_attention_batch); prompts without
+        context read fp16 K/V where it is, everything else (cached context,
+        bf16 or fp32 rows, a head size below its padded size) comes from one
+        launch of the gather (tq_prefill_gather).  The reference runs
+        flash-attn per request here (vllm_backend_fused.py:335-371)."""
         from . import ops
-        d, pd = self.head_size, self._pd
+        d, pd, hkv = self.head_size, self._pd, self.num_kv_heads
         if pd > 256:
             raise RuntimeError(f"prefill: head_size {d} unsupported (padded size {pd} > 256)")
-        if d == pd:
-            if out is None or out.dtype != torch.float16:
-                out = torch.empty(q.shape, dtype=torch.float16, device=q.device)
-            return ops.prefill_attention(q, k, v, out, self.scale)
-        pad = (0, pd - d)
-        qp, kp, vp = F.pad(q, pad), F.pad(k, pad), F.pad(v, pad)
-        op = torch.empty(qp.shape, dtype=torch.float16, device=q.device)
-        ops.prefill_attention(qp, kp, vp, op, self.scale)
-        return op[:, :, :d]
+
+        if not chunks:
+            return output
+        floats = (torch.float16, torch.bfloat16, torch.float32)
+        if key.dtype != value.dtype or key.dtype not in floats:
+            key, value = key.to(torch.float16), value.to(torch.float16)
+
+        def rows_ok(t, dtypes):
+            return (t.dtype in dtypes and t.stride(2) == 1 and t.stride(0) % 8 == 0
+                    and t.stride(1) % 8 == 0 and t.data_ptr() % 16 == 0)
+
+        half = (torch.float16, torch.bfloat16)
+        q, o, qd = query, output, d
+        if d % 8 != 0 or not rows_ok(q, half):
+            q = q.to(torch.float16)
+            if d % 8 != 0:
+                q, qd = F.pad(q, (0, pd - d)), pd
+            q = q.contiguous()
+            if q.data_ptr() % 16 != 0:
+                q = q.clone()
+        if qd != d or not rows_ok(o, half):
+            o = torch.empty((query.shape[0], self.num_heads, qd), dtype=torch.float16,
+                            device=query.device)
+        in_place = d == pd and rows_ok(key, half[:1]) and rows_ok(value, half[:1]) \
+            and min(key.stride(0), value.stride(0)) >= pd
+        kv = (key, value) if in_place else (None, None)
+        at = 0
+        while at < len(chunks):
+            # the gathered rows of a launch are bounded (1 GB at 8 heads of 128),
+            # one chunk's alone may be more
+            reqs, gathers, rows = [], [], 0
+            while at < len(chunks):
+                i, a, ql, ctx = chunks[at]
+                if ctx > 0 or not in_place:
+                    if gathers and rows + ctx + ql > 1 << 18:
+                        break
+                    gathers.append((i, ctx, a, ql, rows))
+                    reqs.append((a, ql, rows, ctx + ql, 1))
+                    rows += ctx + ql
+                else:
+                    reqs.append((a, ql, a, ql, 0))
+                at += 1
+            gk = gv = None
+            if gathers:
+                gk = torch.empty((rows, hkv, pd), dtype=torch.float16, device=query.device)
+                gv = torch.empty_like(gk)
+                k, v = (t if t.stride(2) == 1 else t.contiguous() for t in (key, value))
+                ops.prefill_gather(kv_cache, bt, k, v, gathers, d, pd, self._signs, gk, gv)
+            ops.prefill_attention_batch(q, o, reqs, hkv, qd, pd, self.scale, *kv, gk, gv)
+        if o is not output:
+            for _, a, ql, _ in chunks:
+                output[a:a + ql].copy_(o[a:a + ql, :, :d])
+        return output
 
     def _prefill_fresh(self, query, key, value, attn_metadata, output):
         """Causal attention of each prompt chunk over its own fresh K/V."""
         qsl, _ = self._host_boundaries(attn_metadata)
-        for i in range(len(qsl) - 1):
-            a, b = qsl[i], qsl[i + 1]
-            if b <= a:
-                continue
-            dst = output[a:b]
-            o = self._attend(query[a:b].to(torch.float16), key[a:b].to(torch.float16),
-                             value[a:b].to(torch.float16), 0, dst)
-            if o.data_ptr() != dst.data_ptr():
-                dst.copy_(o)
-        return output
+        chunks = [(i, qsl[i], qsl[i + 1] - qsl[i], 0) for i in range(len(qsl) - 1)
+                  if qsl[i + 1] > qsl[i]]
+        return self._attend_chunks(chunks, query, key, value, None, None, output)
 
     def _decode_ws(self, n, pages, device):
         """Balanced-decode workspace for n decode rows of a mixed batch."""
@@ -356,21 +394,20 @@ class TurboQuantFusedImpl(FlashAttentionImpl):
         * ctx == 0 (a fresh prompt): causal attention over the fresh K/V,
           the reference's prefill (vllm_backend_fused.py:335-371);
         * ctx > 0 (a chunk of a longer prompt): the ctx cached tokens read back
-          from the quantized cache (tq_dequant_paged) followed by the chunk's
+          from the quantized cache (tq_prefill_gather) followed by the chunk's
           fresh K/V, causal with the chunk's queries at the end.  The
           reference attends the fresh chunk only and so drops the cached
           context; its decode path already attends over the dequantized
           cache, which this extends to chunks.
-        Attention runs in this library's prefill kernel (head sizes 64, 128
-        and 256, smaller sizes zero-padded to their padded size; short chunks
-        over long contexts split their keys over workgroups).
+        The prompts and chunks of a step run in one launch of this library's
+        prefill kernel (head sizes 64, 128 and 256, smaller sizes zero-padded
+        to their padded size).
         """
-        from . import ops
         self._ensure_kernels_loaded()
         self._ensure(query.device)
         qsl, seq = self._host_boundaries(attn_metadata)
         bt = attn_metadata.block_table
-        dec = []
+        dec, chunks = [], []
         for i in range(len(qsl) - 1):
             a, b = qsl[i], qsl[i + 1]
             ql = b - a
@@ -381,24 +418,13 @@ class TurboQuantFusedImpl(FlashAttentionImpl):
                 raise RuntimeError(f"request {i}: seq_len {seq[i]} < query length {ql}")
             if ql == 1 and ctx > 0:
                 dec.append(i)
-                continue
-            q = query[a:b].to(torch.float16)
-            if ctx == 0:
-                kk = key[a:b].to(torch.float16)
-                vv = value[a:b].to(torch.float16)
             else:
-                kk = torch.empty((ctx + ql, self.num_kv_heads, self.head_size),
-                                 dtype=torch.float16, device=query.device)
-                vv = torch.empty_like(kk)
-                pages = bt[i].to(torch.int32).contiguous()
-                ops.dequant_paged(kv_cache, pages, ctx, self.num_kv_heads, self.head_size,
-                                  self._pd, self._signs, kk, vv)
-                kk[ctx:] = key[a:b]
-                vv[ctx:] = value[a:b]
-            dst = output[a:b]
-            o = self._attend(q, kk, vv, ctx, dst)
-            if o.data_ptr() != dst.data_ptr():
-                dst.copy_(o)
+                chunks.append((i, a, ql, ctx))
+        if chunks:
+            table = bt
+            if any(c[3] for c in chunks) and (bt.dtype != torch.int32 or bt.stride(1) != 1):
+                table = bt.to(torch.int32).contiguous()
+            self._attend_chunks(chunks, query, key, value, kv_cache, table, output)
         for c0 in range(0, len(dec), BALANCED_MAX_BATCH):  # a plan takes <= 1024 rows
             self._decode_rows(dec[c0:c0 + BALANCED_MAX_BATCH], qsl, query, kv_cache, bt,
                               attn_metadata, output)
@@ -410,21 +436,36 @@ class TurboQuantFusedImpl(FlashAttentionImpl):
         from . import ops
         if dec:
             dev = query.device
-            rows = torch.tensor([qsl[i] for i in dec], dtype=torch.long, device=dev)
-            idx = torch.tensor(dec, dtype=torch.long, device=dev)
-            q = query.index_select(0, rows).to(torch.float16)
+            n, run = len(dec), dec[-1] - dec[0] + 1 == len(dec)
+            if run:  # consecutive requests, so consecutive rows: views
+                rows = slice(qsl[dec[0]], qsl[dec[0]] + n)
+                idx = slice(dec[0], dec[0] + n)
+                q, sub_bt, sl = query[rows], bt[idx], attn_metadata.seq_lens[idx]
+            else:
+                rows = torch.tensor([qsl[i] for i in dec], dtype=torch.long, device=dev)
+                idx = torch.tensor(dec, dtype=torch.long, device=dev)
+                q = query.index_select(0, rows)
+                sub_bt, sl = bt.index_select(0, idx), attn_metadata.seq_lens.index_select(0, idx)
+            q = q.to(torch.float16)
             if self.head_size < self._pd:
                 q = F.pad(q, (0, self._pd - self.head_size))
             q = q.contiguous()
-            sub_bt = bt.index_select(0, idx).to(torch.int32).contiguous()
-            sl = attn_metadata.seq_lens.index_select(0, idx).to(torch.int32).contiguous()
-            ws = self._decode_ws(len(dec), sub_bt.shape[1], dev)
+            sub_bt, sl = sub_bt.to(torch.int32).contiguous(), sl.to(torch.int32).contiguous()
+            ws = self._decode_ws(n, sub_bt.shape[1], dev)
+            # the kernel writes the caller's rows directly when they have the
+            # op's layout
+            direct = (run and self.head_size == self._pd and output.dtype == torch.float16
+                      and output[rows].is_contiguous())
             o = ops.decode_paged_balanced(q, kv_cache, sub_bt.reshape(-1), ws["indptr"], sl,
                                           self.num_kv_heads, self.head_size, self._pd,
-                                          self.scale, self._signs, ws["o"],
+                                          self.scale, self._signs,
+                                          output[rows] if direct else ws["o"],
                                           ws["partition_o"], ws["partition_lse"],
                                           ws["split_indptr"])
-            output.index_copy_(0, rows, o[:, :, :self.head_size].to(output.dtype))
+            if run and not direct:
+                output[rows].copy_(o[:, :, :self.head_size])
+            elif not run:
+                output.index_copy_(0, rows, o[:, :, :self.head_size].to(output.dtype))
         return output
 
     @torch.no_grad()
