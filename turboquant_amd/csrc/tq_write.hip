@@ -23,32 +23,36 @@ namespace tq {
 
 namespace {
 
-// Load VEC consecutive input elements as fp32 (exact for fp16/bf16).
+// Load VEC consecutive input elements as fp32 (exact for fp16/bf16).  vec_ok:
+// rows aligned to VEC elements and head_dim a multiple of VEC, so a run lies
+// inside the row or past its end.
 template <int VEC>
 __device__ __forceinline__ void load_row(const void* base, int64_t off, int dtype,
                                          int d0, int head_dim, bool vec_ok, float* x) {
+  if (vec_ok) {
+#pragma unroll
+    for (int i = 0; i < VEC; i++) x[i] = 0.0f;
+    if (d0 >= head_dim) return;
+    if (dtype == TQ_F32) {
+      typedef float fv __attribute__((ext_vector_type(VEC)));
+      const fv v = *reinterpret_cast<const fv*>(static_cast<const float*>(base) + off + d0);
+#pragma unroll
+      for (int i = 0; i < VEC; i++) x[i] = v[i];
+      return;
+    }
+    typedef _Float16 hv __attribute__((ext_vector_type(VEC)));
+    const hv v = *reinterpret_cast<const hv*>(static_cast<const _Float16*>(base) + off + d0);
+#pragma unroll
+    for (int i = 0; i < VEC; i++)
+      x[i] = dtype == TQ_F16
+                 ? (float)v[i]
+                 : __uint_as_float((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v[i]) << 16);
+    return;
+  }
   if (dtype == TQ_F16) {
     const _Float16* p = reinterpret_cast<const _Float16*>(base) + off + d0;
-    if (vec_ok) {
-      if constexpr (VEC == 2) {
-        typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-        h2 v = *reinterpret_cast<const h2*>(p);
-        x[0] = (float)v[0]; x[1] = (float)v[1];
-      } else if constexpr (VEC == 4) {
-        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-        h4 v = *reinterpret_cast<const h4*>(p);
 #pragma unroll
-        for (int i = 0; i < 4; i++) x[i] = (float)v[i];
-      } else {
-        typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-        h8 v = *reinterpret_cast<const h8*>(p);
-#pragma unroll
-        for (int i = 0; i < 8; i++) x[i] = (float)v[i];
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < VEC; i++) x[i] = (d0 + i < head_dim) ? (float)p[i] : 0.0f;
-    }
+    for (int i = 0; i < VEC; i++) x[i] = (d0 + i < head_dim) ? (float)p[i] : 0.0f;
   } else if (dtype == TQ_BF16) {
     const uint16_t* p = reinterpret_cast<const uint16_t*>(base) + off + d0;
 #pragma unroll
@@ -121,6 +125,15 @@ __device__ __forceinline__ float xor_lane(float x) {
 // sign flip, FWHT stages h = 1 .. pd/2 in ascending order (the last one,
 // between lanes p and p + 16, again inside one physical lane), 1/sqrt(pd),
 // bucketize, pack.
+//
+// With 16 lanes per vector a small launch has four times the waves of the
+// fast kernel below and a quarter of the work in each: K and V of 8 tokens x 8
+// heads x 128 take 3.3 us against 4.0 us, 512 tokens 3.8 against 4.3, 1024
+// tokens 5.1 against 4.7 (so up to kSmallWrite vectors).  Above that it serves
+// the rows that the fast kernel cannot load.
+//
+// sign_first: the signs are flipped before the squares, which leaves a NaN
+// norm the sign that the fast kernel gives it (every other bit is the same).
 template <int PD, bool VEC_OK>
 __global__ __launch_bounds__(256) void write_kernel(
     uint8_t* __restrict__ k_slab, uint8_t* __restrict__ v_slab,
@@ -128,7 +141,7 @@ __global__ __launch_bounds__(256) void write_kernel(
     int64_t k_st, int64_t k_sh, int64_t v_st, int64_t v_sh,
     const float* __restrict__ signs, const int32_t* __restrict__ slots,
     uint32_t per_kv, int H, uint32_t hmul, int head_dim, int ebs, int64_t nslots,
-    float scale) {
+    float scale, bool sign_first) {
 #pragma clang fp contract(off)
   constexpr int VEC = PD / 32;
   const int lane = threadIdx.x & 15;
@@ -152,6 +165,22 @@ __global__ __launch_bounds__(256) void write_kernel(
   const int32_t slot = slots[t];
   if (slot < 0 || (int64_t)slot >= nslots) return;  // whole 16-lane group together
 
+  float g0[VEC], g1[VEC];
+#pragma unroll
+  for (int i = 0; i < VEC; i++) {
+    g0[i] = signs[da + i];
+    g1[i] = signs[db + i];
+  }
+  auto flip = [](float v, float s) {  // v * s for s = +-1, a NaN's sign too
+    return __uint_as_float(__float_as_uint(v) ^ (__float_as_uint(s) & 0x80000000u));
+  };
+  if (sign_first) {  // uniform
+#pragma unroll
+    for (int i = 0; i < VEC; i++) {
+      x0[i] = flip(x0[i], g0[i]);
+      x1[i] = flip(x1[i], g1[i]);
+    }
+  }
   // 1. per-lane sums of squares, FMA-accumulated in dim order
   float s0 = 0.0f, s1 = 0.0f;
 #pragma unroll
@@ -175,10 +204,12 @@ __global__ __launch_bounds__(256) void write_kernel(
     x0[i] = x0[i] * inv;
     x1[i] = x1[i] * inv;
   }
+  if (!sign_first) {
 #pragma unroll
-  for (int i = 0; i < VEC; i++) {
-    x0[i] = x0[i] * signs[da + i];
-    x1[i] = x1[i] * signs[db + i];
+    for (int i = 0; i < VEC; i++) {
+      x0[i] = x0[i] * g0[i];
+      x1[i] = x1[i] * g1[i];
+    }
   }
   // 5. FWHT: in-lane stages h < VEC, cross-lane stages (lane xor 1..8), then
   //    the stage between lanes p and p + 16
@@ -265,7 +296,9 @@ __global__ __launch_bounds__(256) void write_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// fp16 fast path: 32 dims per lane, P = PD/32 lanes per vector.
+// Fast path: 32 dims per lane, P = PD/32 lanes per vector, rows in whole
+// 16-byte aligned pieces (fp16, bf16 or fp32; head_dim a multiple of 8, the
+// chunks past it zero).
 //
 // Lane p of a vector holds the 16-byte chunks j = p + P*i (i = 0..3), i.e.
 // dims d = 8j + c (c = 0..7): bits 0-2 of d are in-lane, the next log2(P)
@@ -285,9 +318,9 @@ __global__ __launch_bounds__(256) void write_kernel(
 // the sign it is held with differ.
 //
 // Instruction savings over the generic kernel:
-//  * the sign flip is an XOR of the fp16 sign bits before conversion, and
-//    the normalisation reads the fp16 value directly (v_fma_mix with a -0
-//    addend, i.e. the exact product): (x*s)*inv == (x*inv)*s for s = +-1;
+//  * the sign flip is an XOR of the sign bits before conversion:
+//    (x*s)*inv == (x*inv)*s for s = +-1 (but for the sign of a zero, and both
+//    zeros give code 8);
 //  * a cross-lane butterfly is one fma with a DPP operand: lane l keeps
 //    z_l + sg_l * z_partner (sg = -1 on the upper lane), which is the
 //    reference's value times tau_l = +-1.  Negation commutes with the later
@@ -304,8 +337,15 @@ __global__ __launch_bounds__(256) void write_kernel(
 //    at most one boundary (the tests check this for every head size), so
 //    code = (8 + below + (|v| >= boundary)) for v >= 0 and its 4-bit
 //    complement for v < 0.
-//  * vectors whose sum of squares is not finite (an inf or NaN input) give
-//    NaN everywhere after the FWHT, i.e. code 0, as in the reference.
+//  * a vector with an inf or NaN input is NaN everywhere after the FWHT
+//    (every output adds every input; inf * inv is inf * 0), i.e. code 0, as in
+//    the reference: one coordinate stands for all.  (A sum of squares that
+//    overflows on finite bf16 or fp32 inputs gives inv = 0, all codes 8.)
+//
+// VALU-bound (about 20 instructions per coordinate): 8192 tokens x 8 heads x
+// 128, K and V, 14.3 us for fp16 (3.0 TB/s), 13.4 for bf16 and 16.8 for fp32
+// rows; in the general kernel, whose bf16 and fp32 loads were single elements,
+// 23.3, 24.2 and 22.2 us.
 template <int PD>
 struct FastGeom {
   // 16-byte chunks (8 dims) per lane: 4, and 2 at pd 64, where 4 would leave
@@ -392,17 +432,19 @@ __device__ __forceinline__ float add_qxor(float r) {
   return r;
 }
 
-template <int PD>
-__global__ __launch_bounds__(256) void write_f16_kernel(
+template <int PD, int DT>
+__global__ __launch_bounds__(256) void write_fast_kernel(
     uint8_t* __restrict__ k_slab, uint8_t* __restrict__ v_slab,
-    const _Float16* __restrict__ key, const _Float16* __restrict__ value,
+    const void* __restrict__ key, const void* __restrict__ value,
     int64_t k_st, int64_t k_sh, int64_t v_st, int64_t v_sh,
     const float* __restrict__ signs, const int32_t* __restrict__ slots,
-    uint32_t per_kv, int H, uint32_t hmul, int ebs, int64_t nslots, float scale) {
+    uint32_t per_kv, int H, uint32_t hmul, int head_dim, int ebs, int64_t nslots, float scale) {
 #pragma clang fp contract(off)
   using FG = FastGeom<PD>;
   constexpr int P = FG::P, E = FG::E, VEC = FG::VEC, CPL = FG::CPL, PE = FG::PE;
   constexpr int ND = 8 * CPL;  // dims per lane
+  constexpr int W = DT == TQ_F32 ? 2 : 1;       // 16-byte pieces per chunk
+  constexpr int ESZ = DT == TQ_F32 ? 4 : 2;
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   __shared__ __attribute__((aligned(512))) uint32_t tbl[128];  // 64 x (2 * boundary, 8 + below)
 
@@ -411,19 +453,34 @@ __global__ __launch_bounds__(256) void write_f16_kernel(
   const uint32_t g = blockIdx.x * (uint32_t)FG::VPB + (threadIdx.x >> 6) * FG::VPW + lane / P;
   const bool live = g < 2 * per_kv;
 
-  // this vector's row: CPL chunks j = p + P*i, issued first (zeros past the end)
+  // this vector's row: CPL chunks j = p + P*i, issued first
   const int kv = g >= per_kv ? 1 : 0;
   const uint32_t rem = g - (kv ? per_kv : 0u);
   const uint32_t t = H == 1 ? rem : __umulhi(rem, hmul);  // rem / H, exact (hmul = ceil(2^32/H))
   const int h = (int)(rem - t * (uint32_t)H);
   // lanes past the end read row 0 of K (no branch, no zero fill); they
   // store nothing (slot -1)
-  u32x4 raw[CPL];
-  const _Float16* row = !live ? key
-                        : kv  ? value + (int64_t)t * v_st + (int64_t)h * v_sh
-                              : key + (int64_t)t * k_st + (int64_t)h * k_sh;
+  u32x4 raw[CPL * W];
+  const uint8_t* row =
+      !live ? static_cast<const uint8_t*>(key)
+      : kv  ? static_cast<const uint8_t*>(value) + ((int64_t)t * v_st + (int64_t)h * v_sh) * ESZ
+            : static_cast<const uint8_t*>(key) + ((int64_t)t * k_st + (int64_t)h * k_sh) * ESZ;
+  if (head_dim == PD) {  // uniform
 #pragma unroll
-  for (int i = 0; i < CPL; i++) raw[i] = *reinterpret_cast<const u32x4*>(row + 8 * (p + P * i));
+    for (int i = 0; i < CPL; i++)
+#pragma unroll
+      for (int k = 0; k < W; k++)
+        raw[W * i + k] = *reinterpret_cast<const u32x4*>(row + 8 * ESZ * (p + P * i) + 16 * k);
+  } else {  // chunks past head_dim are zero (head_dim % 8 == 0)
+#pragma unroll
+    for (int i = 0; i < CPL; i++)
+#pragma unroll
+      for (int k = 0; k < W; k++) {
+        raw[W * i + k] = u32x4{0u, 0u, 0u, 0u};
+        if (8 * (p + P * i) < head_dim)
+          raw[W * i + k] = *reinterpret_cast<const u32x4*>(row + 8 * ESZ * (p + P * i) + 16 * k);
+      }
+  }
   const int32_t slot = live ? slots[t] : -1;
 
   // boundaries b_k * scale (k = 1..7) as integer bits (positive floats order
@@ -450,29 +507,48 @@ __global__ __launch_bounds__(256) void write_f16_kernel(
     tbl[2 * idx + 1] = below;
   }
 
-  // signed fp16 inputs: the sign bits of this lane's signs (+-1) flipped into
-  // the halves (the top bytes of two floats go to bytes 1 and 3, then the
-  // sign bits are kept)
-  uint32_t hw[CPL][4];
+  // signed inputs: the sign bits of this lane's signs (+-1) flipped in (16-bit
+  // types: the top bytes of two floats go to bytes 1 and 3, then the sign bits
+  // are kept)
+  uint32_t hw[CPL][4 * W];
 #pragma unroll
   for (int i = 0; i < CPL; i++) {
     const float4* sp = reinterpret_cast<const float4*>(signs + 8 * (p + P * i));
     const float4 s0 = sp[0], s1 = sp[1];
     const float sv[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
 #pragma unroll
-    for (int c = 0; c < 4; c++) {
-      const uint32_t sm = __builtin_amdgcn_perm(__float_as_uint(sv[2 * c + 1]),
-                                                __float_as_uint(sv[2 * c]), 0x070c030cu);
-      hw[i][c] = raw[i][c] ^ (sm & 0x80008000u);
+    for (int c = 0; c < 4 * W; c++) {
+      if constexpr (DT == TQ_F32) {
+        hw[i][c] = raw[W * i + c / 4][c % 4] ^ (__float_as_uint(sv[c]) & 0x80000000u);
+      } else {
+        const uint32_t sm = __builtin_amdgcn_perm(__float_as_uint(sv[2 * c + 1]),
+                                                  __float_as_uint(sv[2 * c]), 0x070c030cu);
+        hw[i][c] = raw[i][c] ^ (sm & 0x80008000u);
+      }
     }
   }
-  auto hv = [&](int i, int c) -> float {  // signed input dim 8j + c as fp32 (exact)
-    return c & 1 ? hi_half_f(hw[i][c / 2]) : lo_half_f(hw[i][c / 2]);
-  };
-
-  // 1. per-reference-lane sums of squares, FMA in dim order
-  float r[E];
-  {
+  // the signed inputs as fp32 (exact): xin[8i + c] = dim 8(p + P i) + c.  fp16
+  // values are converted once; read in place by v_fma_mix (twice each) the
+  // kernel took 15.5 us against 14.9 (8192 tokens x 8 heads x 128)
+  float xin[ND];
+#pragma unroll
+  for (int i = 0; i < CPL; i++)
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+      float f;
+      if constexpr (DT == TQ_F32) f = __uint_as_float(hw[i][c]);
+      else if constexpr (DT == TQ_BF16)
+        f = __uint_as_float(c & 1 ? hw[i][c / 2] & 0xffff0000u : hw[i][c / 2] << 16);
+      else f = c & 1 ? hi_half_f(hw[i][c / 2]) : lo_half_f(hw[i][c / 2]);
+#if defined(__HIP_DEVICE_COMPILE__)
+      if constexpr (DT == TQ_F16) asm("" : "+v"(f));
+#endif
+      xin[8 * i + c] = f;
+    }
+  // sum of squares of the vector's values val(i, c)
+  auto sum_squares = [&](auto val) -> float {
+    float r[E];
+    // 1. per-reference-lane sums of squares, FMA in dim order
     float a[CPL][E];
 #pragma unroll
     for (int i = 0; i < CPL; i++)
@@ -481,7 +557,7 @@ __global__ __launch_bounds__(256) void write_f16_kernel(
         float sacc = 0.0f;
 #pragma unroll
         for (int c = 0; c < VEC; c++) {
-          const float xv = hv(i, e * VEC + c);
+          const float xv = val(i, e * VEC + c);
           sacc = __builtin_fmaf(xv, xv, sacc);
         }
         a[i][e] = sacc;
@@ -495,39 +571,52 @@ __global__ __launch_bounds__(256) void write_f16_kernel(
         for (int e = 0; e < E; e++) a[i][e] = a[i][e] + a[i + L / PE][e];
 #pragma unroll
     for (int e = 0; e < E; e++) r[e] = a[0][e];
-  }
-  // levels below PE: lane bits (xor across the vector's lanes) from E up,
-  // in-lane below
-  auto level = [&](auto lv) {
-    constexpr int L = decltype(lv)::value;
-    if constexpr (L < PE) {
-      if constexpr (L >= E) {
+    // levels below PE: lane bits (xor across the vector's lanes) from E up,
+    // in-lane below
+    auto level = [&](auto lv) {
+      constexpr int L = decltype(lv)::value;
+      if constexpr (L < PE) {
+        if constexpr (L >= E) {
 #pragma unroll
-        for (int e = 0; e < E; e++) {
-          if constexpr (L / E <= 2) r[e] = add_qxor<L / E>(r[e]);
-          else r[e] = r[e] + xor8<L / E>(r[e]);
+          for (int e = 0; e < E; e++) {
+            if constexpr (L / E <= 2) r[e] = add_qxor<L / E>(r[e]);
+            else r[e] = r[e] + xor8<L / E>(r[e]);
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < L; e++) r[e] = r[e] + r[e + L];
         }
-      } else {
-#pragma unroll
-        for (int e = 0; e < L; e++) r[e] = r[e] + r[e + L];
       }
-    }
+    };
+    level(std::integral_constant<int, 16>{});
+    level(std::integral_constant<int, 8>{});
+    level(std::integral_constant<int, 4>{});
+    level(std::integral_constant<int, 2>{});
+    level(std::integral_constant<int, 1>{});
+    return r[0];
   };
-  level(std::integral_constant<int, 16>{});
-  level(std::integral_constant<int, 8>{});
-  level(std::integral_constant<int, 4>{});
-  level(std::integral_constant<int, 2>{});
-  level(std::integral_constant<int, 1>{});
-  const float ss = r[0];
+  float ss = sum_squares([&](int i, int c) { return xin[8 * i + c]; });
+  if ((DT != TQ_F16 || head_dim != PD) && __builtin_amdgcn_ballot_w64(ss != ss) != 0) {
+    // a NaN input keeps its own sign in the stored norm, as the general kernel
+    // leaves it: the squares of the values as they came (the same bits for
+    // every other vector)
+    ss = sum_squares([&](int i, int c) -> float {
+      if (8 * (p + P * i) >= head_dim) return 0.0f;
+      const uint8_t* e = row + ESZ * (8 * (p + P * i) + c);
+      if constexpr (DT == TQ_F32) return *reinterpret_cast<const float*>(e);
+      else if constexpr (DT == TQ_BF16)
+        return __uint_as_float((uint32_t)*reinterpret_cast<const uint16_t*>(e) << 16);
+      else return (float)*reinterpret_cast<const _Float16*>(e);
+    });
+  }
   // 3. IEEE sqrt and reciprocal; normalise (exact products of the fp16 inputs)
   const float l2 = __builtin_sqrtf(ss);
   const float inv = (l2 > 1e-8f) ? (1.0f / l2) : 0.0f;
-  const bool finite = ss <= 3.402823466e38f;  // false for inf and NaN
   float x[ND];  // x[8i + c] = dim 8(p + P i) + c, times tau
 #pragma unroll
   for (int i = 0; i < CPL; i++)
 #pragma unroll
-    for (int c = 0; c < 8; c++) x[8 * i + c] = __builtin_fmaf(hv(i, c), inv, 0.0f);
+    for (int c = 0; c < 8; c++) x[8 * i + c] = xin[8 * i + c] * inv;
   // 4. FWHT, ascending h: dim bits 0-2 in-lane, then the lane bits, then the
   //    chunk-row bits in-lane
 #pragma unroll
@@ -567,6 +656,7 @@ __global__ __launch_bounds__(256) void write_f16_kernel(
           x[8 * i + c] = u + w;
           x[8 * (i + hi2) + c] = u - w;
         }
+  const bool finite = x[0] == x[0];
   // 5. scale (with tau), bucketize through the bin table, pack
   const float ts = (__builtin_popcount(lane & (P - 1)) & 1) ? -scale : scale;
   __syncthreads();  // bin table ready
@@ -617,29 +707,33 @@ hipError_t launch_write(bool vec_ok, dim3 grid, hipStream_t stream, uint8_t* ks,
                         const void* key, const void* value, int dtype, int64_t k_st,
                         int64_t k_sh, int64_t v_st, int64_t v_sh, const float* signs,
                         const int32_t* slots, uint32_t per_kv, int H, uint32_t hmul, int hd,
-                        int ebs, int64_t nslots, float scale) {
+                        int ebs, int64_t nslots, float scale, bool sign_first) {
   if (vec_ok)
     hipLaunchKernelGGL((write_kernel<PD, true>), grid, dim3(256), 0, stream, ks, vs, key, value,
                        dtype, k_st, k_sh, v_st, v_sh, signs, slots, per_kv, H, hmul, hd, ebs,
-                       nslots, scale);
+                       nslots, scale, sign_first);
   else
     hipLaunchKernelGGL((write_kernel<PD, false>), grid, dim3(256), 0, stream, ks, vs, key, value,
                        dtype, k_st, k_sh, v_st, v_sh, signs, slots, per_kv, H, hmul, hd, ebs,
-                       nslots, scale);
+                       nslots, scale, sign_first);
   return hipGetLastError();
 }
 
 template <int PD>
-hipError_t launch_write_f16(hipStream_t stream, uint8_t* ks, uint8_t* vs, const void* key,
-                            const void* value, int64_t k_st, int64_t k_sh, int64_t v_st,
-                            int64_t v_sh, const float* signs, const int32_t* slots,
-                            uint32_t per_kv, int H, uint32_t hmul, int ebs, int64_t nslots,
-                            float scale) {
+hipError_t launch_write_fast(hipStream_t stream, uint8_t* ks, uint8_t* vs, const void* key,
+                             const void* value, int dtype, int64_t k_st, int64_t k_sh,
+                             int64_t v_st, int64_t v_sh, const float* signs, const int32_t* slots,
+                             uint32_t per_kv, int H, uint32_t hmul, int hd, int ebs,
+                             int64_t nslots, float scale) {
   const int64_t blocks = (2 * (int64_t)per_kv + FastGeom<PD>::VPB - 1) / FastGeom<PD>::VPB;
-  const unsigned grid = (unsigned)blocks;
-  hipLaunchKernelGGL((write_f16_kernel<PD>), dim3(grid), dim3(256), 0, stream, ks, vs,
-                     static_cast<const _Float16*>(key), static_cast<const _Float16*>(value), k_st,
-                     k_sh, v_st, v_sh, signs, slots, per_kv, H, hmul, ebs, nslots, scale);
+  const dim3 grid((unsigned)blocks);
+#define TQ_FAST(DT)                                                                              \
+  hipLaunchKernelGGL((write_fast_kernel<PD, DT>), grid, dim3(256), 0, stream, ks, vs, key, value, \
+                     k_st, k_sh, v_st, v_sh, signs, slots, per_kv, H, hmul, hd, ebs, nslots, scale)
+  if (dtype == TQ_F16) TQ_FAST(TQ_F16);
+  else if (dtype == TQ_BF16) TQ_FAST(TQ_BF16);
+  else TQ_FAST(TQ_F32);
+#undef TQ_FAST
   return hipGetLastError();
 }
 
@@ -709,11 +803,11 @@ extern "C" int tq_quantize_write_kv_cache(void* k_slab, void* v_slab, const void
   }
   const int vec = pd / 32;
   const int esz = in_dtype == TQ_F32 ? 4 : 2;
-  // vector loads need the full row, and every row start aligned to VEC elements
-  bool vec_ok = in_dtype == TQ_F16 && head_dim == pd &&
-                (k_stride_tok % vec == 0) && (k_stride_head % vec == 0) &&
-                (v_stride_tok % vec == 0) && (v_stride_head % vec == 0) &&
-                ((uintptr_t)key % (vec * esz) == 0) && ((uintptr_t)value % (vec * esz) == 0);
+  // vector loads: rows in whole runs of VEC elements, every row start aligned to them
+  const bool vec_ok = head_dim % vec == 0 && (k_stride_tok % vec == 0) &&
+                      (k_stride_head % vec == 0) && (v_stride_tok % vec == 0) &&
+                      (v_stride_head % vec == 0) && ((uintptr_t)key % (vec * esz) == 0) &&
+                      ((uintptr_t)value % (vec * esz) == 0);
   // 16 vectors per workgroup; token = rem / H by multiply-high, exact while
   // num_tokens * H < 2^32 / H
   const int64_t per_kv = num_tokens * (int64_t)num_kv_heads;
@@ -732,28 +826,24 @@ extern "C" int tq_quantize_write_kv_cache(void* k_slab, void* v_slab, const void
   uint8_t* ks = static_cast<uint8_t*>(k_slab);
   uint8_t* vs = static_cast<uint8_t*>(v_slab);
   hipError_t e;
-  // fp16 rows of full width with 16-byte aligned chunks take the fast kernel
-  const bool fast_ok = in_dtype == TQ_F16 && head_dim == pd && k_stride_tok % 8 == 0 &&
-                       k_stride_head % 8 == 0 && v_stride_tok % 8 == 0 &&
-                       v_stride_head % 8 == 0 && (uintptr_t)key % 16 == 0 &&
-                       (uintptr_t)value % 16 == 0;
-  if (fast_ok) {
-    switch (pd) {
-      case 64:
-        e = launch_write_f16<64>(s, ks, vs, key, value, k_stride_tok, k_stride_head, v_stride_tok,
-                                 v_stride_head, signs, slot_mapping, (uint32_t)per_kv,
-                                 num_kv_heads, hmul, ebs, nslots, scale);
-        break;
-      case 128:
-        e = launch_write_f16<128>(s, ks, vs, key, value, k_stride_tok, k_stride_head,
-                                  v_stride_tok, v_stride_head, signs, slot_mapping,
-                                  (uint32_t)per_kv, num_kv_heads, hmul, ebs, nslots, scale);
-        break;
-      default:
-        e = launch_write_f16<256>(s, ks, vs, key, value, k_stride_tok, k_stride_head,
-                                  v_stride_tok, v_stride_head, signs, slot_mapping,
-                                  (uint32_t)per_kv, num_kv_heads, hmul, ebs, nslots, scale);
-    }
+  // rows in whole 16-byte aligned pieces take the fast kernel
+  const int al = 16 / esz;
+  const bool fast_ok = head_dim % 8 == 0 && k_stride_tok % al == 0 && k_stride_head % al == 0 &&
+                       v_stride_tok % al == 0 && v_stride_head % al == 0 &&
+                       (uintptr_t)key % 16 == 0 && (uintptr_t)value % 16 == 0 &&
+                       (uintptr_t)signs % 16 == 0;
+  // small launches of padded size 64 or 128 take the general kernel (see there;
+  // at 256 the fast one is as fast from one token on)
+  constexpr int64_t kSmallWrite = 8192;
+  const bool small = pd <= 128 && 2 * per_kv <= kSmallWrite;
+  const bool sign_first = fast_ok && in_dtype == TQ_F16 && head_dim == pd;
+  if (fast_ok && !small) {
+#define TQ_FAST_PD(PD)                                                                            \
+  launch_write_fast<PD>(s, ks, vs, key, value, in_dtype, k_stride_tok, k_stride_head,             \
+                        v_stride_tok, v_stride_head, signs, slot_mapping, (uint32_t)per_kv,       \
+                        num_kv_heads, hmul, head_dim, ebs, nslots, scale)
+    e = pd == 64 ? TQ_FAST_PD(64) : pd == 128 ? TQ_FAST_PD(128) : TQ_FAST_PD(256);
+#undef TQ_FAST_PD
     if (e != hipSuccess) {
       set_error("quantize_write: launch failed: %s", hipGetErrorString(e));
       return (int)e;
@@ -764,17 +854,20 @@ extern "C" int tq_quantize_write_kv_cache(void* k_slab, void* v_slab, const void
     case 64:
       e = launch_write<64>(vec_ok, grid, s, ks, vs, key, value, in_dtype, k_stride_tok,
                            k_stride_head, v_stride_tok, v_stride_head, signs, slot_mapping,
-                           (uint32_t)per_kv, num_kv_heads, hmul, head_dim, ebs, nslots, scale);
+                           (uint32_t)per_kv, num_kv_heads, hmul, head_dim, ebs, nslots, scale,
+                           sign_first);
       break;
     case 128:
       e = launch_write<128>(vec_ok, grid, s, ks, vs, key, value, in_dtype, k_stride_tok,
                             k_stride_head, v_stride_tok, v_stride_head, signs, slot_mapping,
-                            (uint32_t)per_kv, num_kv_heads, hmul, head_dim, ebs, nslots, scale);
+                            (uint32_t)per_kv, num_kv_heads, hmul, head_dim, ebs, nslots, scale,
+                           sign_first);
       break;
     default:
       e = launch_write<256>(vec_ok, grid, s, ks, vs, key, value, in_dtype, k_stride_tok,
                             k_stride_head, v_stride_tok, v_stride_head, signs, slot_mapping,
-                            (uint32_t)per_kv, num_kv_heads, hmul, head_dim, ebs, nslots, scale);
+                            (uint32_t)per_kv, num_kv_heads, hmul, head_dim, ebs, nslots, scale,
+                            sign_first);
   }
   if (e != hipSuccess) {
     set_error("quantize_write: launch failed: %s", hipGetErrorString(e));
