@@ -121,6 +121,20 @@ int tq_decode_paged_balanced(const void* q, int64_t q_stride_b, int64_t q_stride
                              int32_t* split_rows, void* o, tq_stream_t stream);
 
 /*
+ * The same with q and o as rows of head_dim elements (a multiple of 8; dims up
+ * to padded_dim count as zero), each fp16 or bf16 (TQ_F16 / TQ_BF16): o
+ * [batch, num_qo_heads, head_dim] contiguous.  The model's own rows go in and
+ * come out without conversion, padding or slicing around the call.
+ */
+int tq_decode_paged_balanced_rows(
+    const void* q, int64_t q_stride_b, int64_t q_stride_h, int32_t q_dtype, const uint8_t* k_slab,
+    const uint8_t* v_slab, const int32_t* indices, const int32_t* indptr,
+    const int32_t* seq_lens, int32_t batch, int32_t num_qo_heads, int32_t num_kv_heads,
+    int32_t head_dim, int32_t padded_dim, int32_t block_size, int32_t ebs, int64_t num_blocks,
+    float sm_scale, const float* signs, int32_t max_rows, float* partition_o,
+    float* partition_lse, int32_t* split_rows, void* o, int32_t o_dtype, tq_stream_t stream);
+
+/*
  * tq_decode_paged_balanced without workspace arguments and without any
  * allocation: the row table, partial LSEs and partial rows live in a
  * 16 MiB device array inside this library (one per GPU, kept until the

@@ -28,6 +28,9 @@ SIGNATURES = {
     "tq_decode_paged_balanced": (_I32, [_P, _I64, _I64, _P, _P, _P, _P, _P, _I32, _I32, _I32,
                                         _I32, _I32, _I32, _I32, _I64, _F32, _P, _I32, _P, _P,
                                         _P, _P, _P]),
+    "tq_decode_paged_balanced_rows": (_I32, [_P, _I64, _I64, _I32, _P, _P, _P, _P, _P, _I32,
+                                             _I32, _I32, _I32, _I32, _I32, _I32, _I64, _F32, _P,
+                                             _I32, _P, _P, _P, _P, _I32, _P]),
     "tq_decode_paged_balanced_noalloc": (_I32, [_P, _I64, _I64, _P, _P, _P, _P, _P, _I32, _I32,
                                                 _I32, _I32, _I32, _I32, _I32, _I64, _F32, _P,
                                                 _P, _P]),

@@ -110,8 +110,10 @@ __device__ __forceinline__ uint32_t quad_bcast(uint32_t v) {
 
 
 struct DecodeParams {
-  const _Float16* q;
+  const _Float16* q;  // (bf16 rows when q_bf16)
   int64_t q_sb, q_sh;
+  int hd;      // elements of a q row; dims hd .. pd - 1 are zero (hd % 8 == 0)
+  int q_bf16;
   const uint8_t* ks;
   const uint8_t* vs;
   const int32_t* indices;
@@ -958,7 +960,10 @@ constexpr bool kPvLo = TQ_PV_LO != 0;
 // the attention math compiled out (q' setup, table build and partial-row
 // stores kept), 0 = the bare copy ring (page walk, copies, waits, barriers
 // and slot reads only).
-template <int PD, int G, int PACK, bool QC, bool PLAN, int MATH = TQ_DECODE_MATH>
+// ROWS: q rows of p.hd elements, fp16 or bf16 (else fp16 rows of PD; as a
+// run-time choice this cost the fp16 path 0.1 .. 0.6 us a step).
+template <int PD, int G, int PACK, bool QC, bool PLAN, int MATH = TQ_DECODE_MATH,
+          bool ROWS = false>
 __global__ __launch_bounds__(64 * G)
 __attribute__((amdgpu_waves_per_eu(PD == 256 ? 2 : (PACK == 1 ? 3 : 4))))
 void decode_partials_kernel(DecodeParams p) {
@@ -1099,7 +1104,7 @@ void decode_partials_kernel(DecodeParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   if constexpr (MATH >= 1) {
     const _Float16* qbase = p.q + (int64_t)b * p.q_sb + (int64_t)kvh * ratio * p.q_sh;
-    const int qrec = qreg ? (int)(((ratio - 1) * p.q_sh + PD) * 2) : 0;
+    const int qrec = qreg ? (int)(((ratio - 1) * p.q_sh + (ROWS ? p.hd : PD)) * 2) : 0;
     const __amdgpu_buffer_rsrc_t rq =
         __builtin_amdgcn_make_buffer_rsrc((void*)qbase, (short)0, qrec, 0x00020000);
     const __amdgpu_buffer_rsrc_t rsg = __builtin_amdgcn_make_buffer_rsrc(
@@ -1108,8 +1113,9 @@ void decode_partials_kernel(DecodeParams p) {
     for (int j = 0; j < NQL; j++) {
       const int e = 512 * j + 8 * lane;
       const int r = e / PD, d = e % PD;
+      // (past a row's end: out of range, zeros)
       const u32x4 qv = __builtin_amdgcn_raw_buffer_load_b128(
-          rq, (uint32_t)((r * p.q_sh + d) * 2), 0, 0);
+          rq, !ROWS || d < p.hd ? (uint32_t)((r * p.q_sh + d) * 2) : 0x80000000u, 0, 0);
       const u32x4 s0 = __builtin_amdgcn_raw_buffer_load_b128(rsg, (uint32_t)(d * 4), 0, 0);
       const u32x4 s1 = __builtin_amdgcn_raw_buffer_load_b128(rsg, (uint32_t)(d * 4 + 16), 0, 0);
       const uint32_t sw[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
@@ -1117,9 +1123,13 @@ void decode_partials_kernel(DecodeParams p) {
 #pragma unroll
         for (int k = 0; k < 8; k++) sgnbits |= (sw[k] >> 31) << k;
       }
+      // (selects, no branch: a branch here would wait for the loads before
+      // the page-table loads go out, 0.6 us of a launch)
 #pragma unroll
       for (int k = 0; k < 8; k++) {
-        const float x = k & 1 ? hi_half(qv[k / 2]) : lo_half(qv[k / 2]);
+        const float xh = k & 1 ? hi_half(qv[k / 2]) : lo_half(qv[k / 2]);
+        const float xb = __uint_as_float(k & 1 ? qv[k / 2] & 0xffff0000u : qv[k / 2] << 16);
+        const float x = ROWS && p.q_bf16 ? xb : xh;
         qx[j][k] = p.signs ? x * __uint_as_float(sw[k]) : x;
       }
     }
@@ -1393,7 +1403,12 @@ void decode_partials_kernel(DecodeParams p) {
       };
       for (int i = lane; i < ratio * PD; i += 64) {
         const int r = i / PD, d = i - r * PD;
-        float x = (float)p.q[b * p.q_sb + (int64_t)(kvh * ratio + r) * p.q_sh + d];
+        const int64_t qi = b * p.q_sb + (int64_t)(kvh * ratio + r) * p.q_sh + d;
+        float x = 0.0f;
+        if (!ROWS || d < p.hd)
+          x = ROWS && p.q_bf16
+                  ? __uint_as_float((uint32_t)reinterpret_cast<const uint16_t*>(p.q)[qi] << 16)
+                  : (float)p.q[qi];
         if (p.signs) x = x * p.signs[d];
         qs[i] = x;
       }
@@ -1637,11 +1652,14 @@ __device__ __forceinline__ float4_t load_half4(const _Float16* src) {
 // g + NG, ... (NG = 64 / (PD/16) split groups), with a running max per lane;
 // the groups then meet through lane swaps (no LDS, no barrier), and the lanes
 // of group 0 store.
-template <int PD>
+//
+// ROWS: o rows of hd elements (hd % 4 == 0), fp16 or bf16 (else fp16 rows of PD).
+template <int PD, bool ROWS>
 __global__ __launch_bounds__(256) void combine_kernel(const _Float16* __restrict__ po,
                                                       const float* __restrict__ plse, int S_fixed,
                                                       const int32_t* __restrict__ split_rows,
-                                                      int Hq, _Float16* __restrict__ o) {
+                                                      int Hq, int hd, int o_bf16,
+                                                      _Float16* __restrict__ o) {
   constexpr int CW = PD / 16;      // float4 columns per wave (PD / 4 dims)
   constexpr int NG = 64 / CW;      // split groups per wave
   constexpr int R = 8;             // splits per lane per round trip
@@ -1717,9 +1735,14 @@ __global__ __launch_bounds__(256) void combine_kernel(const _Float16* __restrict
   }
   if (g == 0) {
     const float inv = den > 0.f ? 1.0f / den : 0.0f;
-    const half4_t hv = {(_Float16)(acc[0] * inv), (_Float16)(acc[1] * inv),
-                        (_Float16)(acc[2] * inv), (_Float16)(acc[3] * inv)};
-    *reinterpret_cast<half4_t*>(o + ((int64_t)b * Hq + h) * PD + col) = hv;
+    if (ROWS && col >= hd) return;
+    half4_t hv = {(_Float16)(acc[0] * inv), (_Float16)(acc[1] * inv),
+                  (_Float16)(acc[2] * inv), (_Float16)(acc[3] * inv)};
+    if (ROWS && o_bf16) {
+      typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
+      hv = __builtin_bit_cast(half4_t, __builtin_convertvector(acc * inv, bf4));
+    }
+    *reinterpret_cast<half4_t*>(o + ((int64_t)b * Hq + h) * (ROWS ? hd : PD) + col) = hv;
   }
 }
 
@@ -1812,16 +1835,18 @@ typedef void (*PartialsFn)(DecodeParams);
 // register set when ratio <= 8 (head size 256 keeps one tile per set: two
 // would exceed the register file); q hi/lo parts share one B operand when
 // the GQA ratio leaves 8 columns free.
-template <bool PLAN>
+template <bool PLAN, bool ROWS>
 PartialsFn partials_kernel_t(int pd, int G, int ratio) {
   const bool pack2 = ratio <= 8 && pd <= 128;
   const bool qc = ratio <= 8;
-#define TQ_PICK_G(PDV, PK, QCV)                                                        \
-  switch (G) {                                                                         \
-    case 8: return &decode_partials_kernel<PDV, (PDV == 256 ? 4 : 8), PK, QCV, PLAN>; \
-    case 4: return &decode_partials_kernel<PDV, 4, PK, QCV, PLAN>;                    \
-    case 2: return &decode_partials_kernel<PDV, 2, PK, QCV, PLAN>;                    \
-    default: return &decode_partials_kernel<PDV, 1, PK, QCV, PLAN>;                   \
+#define TQ_FN(PDV, GV, PK, QCV) \
+  &decode_partials_kernel<PDV, GV, PK, QCV, PLAN, TQ_DECODE_MATH, ROWS>
+#define TQ_PICK_G(PDV, PK, QCV)                               \
+  switch (G) {                                                \
+    case 8: return TQ_FN(PDV, (PDV == 256 ? 4 : 8), PK, QCV); \
+    case 4: return TQ_FN(PDV, 4, PK, QCV);                    \
+    case 2: return TQ_FN(PDV, 2, PK, QCV);                    \
+    default: return TQ_FN(PDV, 1, PK, QCV);                   \
   }
   switch (pd) {
     case 64:
@@ -1832,9 +1857,12 @@ PartialsFn partials_kernel_t(int pd, int G, int ratio) {
       if (qc) { TQ_PICK_G(256, 1, true) } else { TQ_PICK_G(256, 1, false) }
   }
 #undef TQ_PICK_G
+#undef TQ_FN
 }
-PartialsFn partials_kernel(int pd, int G, int ratio, bool plan) {
-  return plan ? partials_kernel_t<true>(pd, G, ratio) : partials_kernel_t<false>(pd, G, ratio);
+PartialsFn partials_kernel(int pd, int G, int ratio, bool plan, bool rows = false) {
+  return !plan  ? partials_kernel_t<false, false>(pd, G, ratio)
+         : rows ? partials_kernel_t<true, true>(pd, G, ratio)
+                : partials_kernel_t<true, false>(pd, G, ratio);
 }
 
 // Checks shared by the partials launchers and the parameter block they fill
@@ -1844,7 +1872,8 @@ int decode_setup(const void* q, int64_t q_stride_b, int64_t q_stride_h, const ui
                  const int32_t* seq_lens, int32_t batch, int32_t num_qo_heads,
                  int32_t num_kv_heads, int32_t padded_dim, int32_t block_size, int32_t ebs,
                  int64_t num_blocks, float sm_scale, const float* signs, float* partition_o,
-                 float* partition_lse, DecodeParams& p) {
+                 float* partition_lse, DecodeParams& p, int32_t row_dim = 0, bool q_bf16 = false) {
+  if (row_dim == 0) row_dim = padded_dim;  // elements of a q row
   int rc = check_geometry(padded_dim, num_qo_heads, num_kv_heads, block_size, ebs, "decode");
   if (rc) return rc;
   if (batch < 0) {
@@ -1861,9 +1890,9 @@ int decode_setup(const void* q, int64_t q_stride_b, int64_t q_stride_h, const ui
     set_error("decode: cache slabs and partition_o must be 16-byte aligned");
     return kEinval;
   }
-  if ((uintptr_t)q % 16 || q_stride_b % 8 || q_stride_h % 8 || q_stride_h < padded_dim) {
+  if ((uintptr_t)q % 16 || q_stride_b % 8 || q_stride_h % 8 || q_stride_h < row_dim) {
     set_error("decode: q must be 16-byte aligned with strides multiple of 8 elements and "
-              "q_stride_h >= padded_dim");
+              "q_stride_h >= %s", row_dim == padded_dim ? "padded_dim" : "head_dim");
     return kEinval;
   }
   const int pd = padded_dim;
@@ -1882,6 +1911,8 @@ int decode_setup(const void* q, int64_t q_stride_b, int64_t q_stride_h, const ui
   p.q = static_cast<const _Float16*>(q);
   p.q_sb = q_stride_b;
   p.q_sh = q_stride_h;
+  p.hd = row_dim;
+  p.q_bf16 = q_bf16;
   p.ks = k_slab;
   p.vs = v_slab;
   p.indices = indices;
@@ -1992,7 +2023,9 @@ namespace tq {
 static int combine_splits(const float* partition_o, const float* partition_lse,
                           int32_t batch, int32_t num_splits, const int32_t* split_rows,
                           int32_t max_rows, int32_t num_qo_heads, int32_t padded_dim,
-                          const float* signs, void* o, tq_stream_t stream) {
+                          const float* signs, void* o, tq_stream_t stream, int32_t row_dim = 0,
+                          bool o_bf16 = false) {
+  if (row_dim == 0) row_dim = padded_dim;
   const int pd = padded_dim;
   if (pd != 64 && pd != 128 && pd != 256) {
     set_error("combine: padded_dim must be 64, 128 or 256, got %d", pd);
@@ -2018,19 +2051,17 @@ static int combine_splits(const float* partition_o, const float* partition_lse,
   (void)max_rows;
   dim3 grid((unsigned)blocks), block(256);
   const _Float16* prow = reinterpret_cast<const _Float16*>(partition_o);
-  switch (pd) {
-    case 64:
-      hipLaunchKernelGGL(combine_kernel<64>, grid, block, 0, st, prow, partition_lse, num_splits,
-                         split_rows, num_qo_heads, out);
-      break;
-    case 128:
-      hipLaunchKernelGGL(combine_kernel<128>, grid, block, 0, st, prow, partition_lse, num_splits,
-                         split_rows, num_qo_heads, out);
-      break;
-    default:
-      hipLaunchKernelGGL(combine_kernel<256>, grid, block, 0, st, prow, partition_lse, num_splits,
-                         split_rows, num_qo_heads, out);
-  }
+  const bool rows = row_dim != pd || o_bf16;
+#define TQ_COMBINE(PDV, R)                                                                       \
+  hipLaunchKernelGGL((combine_kernel<PDV, R>), grid, block, 0, st, prow, partition_lse, num_splits, \
+                     split_rows, num_qo_heads, row_dim, (int)o_bf16, out)
+  if (pd == 64 && rows) TQ_COMBINE(64, true);
+  else if (pd == 64) TQ_COMBINE(64, false);
+  else if (pd == 128 && rows) TQ_COMBINE(128, true);
+  else if (pd == 128) TQ_COMBINE(128, false);
+  else if (rows) TQ_COMBINE(256, true);
+  else TQ_COMBINE(256, false);
+#undef TQ_COMBINE
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     set_error("combine: launch failed: %s", hipGetErrorString(e));
@@ -2049,7 +2080,7 @@ static int partials_balanced(const void* q, int64_t q_stride_b, int64_t q_stride
                              int32_t block_size, int32_t ebs, int64_t num_blocks, float sm_scale,
                              const float* signs, int32_t max_rows, float* partition_o,
                              float* partition_lse, int32_t* split_rows, tq_stream_t stream,
-                             int* rows) {
+                             int* rows, int32_t row_dim = 0, bool q_bf16 = false) {
   if (head_dim <= 0 || head_dim > padded_dim) {
     set_error("decode: head_dim %d exceeds padded_dim %d", head_dim, padded_dim);
     return kEinval;
@@ -2057,7 +2088,8 @@ static int partials_balanced(const void* q, int64_t q_stride_b, int64_t q_stride
   DecodeParams p;
   int rc = decode_setup(q, q_stride_b, q_stride_h, k_slab, v_slab, indices, indptr, seq_lens,
                         batch, num_qo_heads, num_kv_heads, padded_dim, block_size, ebs,
-                        num_blocks, sm_scale, signs, partition_o, partition_lse, p);
+                        num_blocks, sm_scale, signs, partition_o, partition_lse, p, row_dim,
+                        q_bf16);
   if (rc || batch == 0) return rc;
   if (batch > kPlanMaxBatch) {
     set_error("decode: a balanced plan takes at most %d sequences, got %d", kPlanMaxBatch,
@@ -2068,7 +2100,8 @@ static int partials_balanced(const void* q, int64_t q_stride_b, int64_t q_stride
     set_error("decode: null pointer");
     return kEinval;
   }
-  const PartialsFn fn = partials_kernel(padded_dim, p.G, p.ratio, true);
+  const PartialsFn fn = partials_kernel(padded_dim, p.G, p.ratio, true,
+                                        p.hd != padded_dim || p.q_bf16 != 0);
   BalancedGrid g;
   rc = balanced_grid(fn, p, max_rows, g);
   if (rc) return rc;
@@ -2090,7 +2123,8 @@ static int decode_balanced(const void* q, int64_t q_stride_b, int64_t q_stride_h
                            int32_t padded_dim, int32_t block_size, int32_t ebs,
                            int64_t num_blocks, float sm_scale, const float* signs,
                            int32_t max_rows, float* partition_o, float* partition_lse,
-                           int32_t* split_rows, void* o, tq_stream_t stream) {
+                           int32_t* split_rows, void* o, tq_stream_t stream, int32_t row_dim = 0,
+                           bool q_bf16 = false, bool o_bf16 = false) {
   if (!o) {
     set_error("decode: null pointer");
     return kEinval;
@@ -2100,10 +2134,10 @@ static int decode_balanced(const void* q, int64_t q_stride_b, int64_t q_stride_h
                                    seq_lens, batch, num_qo_heads, num_kv_heads, head_dim,
                                    padded_dim, block_size, ebs, num_blocks, sm_scale, signs,
                                    max_rows, partition_o, partition_lse, split_rows, stream,
-                                   &rows);
+                                   &rows, row_dim, q_bf16);
   if (rc || batch == 0) return rc;
   return combine_splits(partition_o, partition_lse, batch, 1, split_rows, rows,
-                        num_qo_heads, padded_dim, signs, o, stream);
+                        num_qo_heads, padded_dim, signs, o, stream, row_dim, o_bf16);
 }
 
 }  // namespace tq
@@ -2154,6 +2188,34 @@ extern "C" int tq_decode_paged_balanced(const void* q, int64_t q_stride_b, int64
                              seq_lens, batch, num_qo_heads, num_kv_heads, head_dim, padded_dim,
                              block_size, ebs, num_blocks, sm_scale, signs, max_rows,
                              partition_o, partition_lse, split_rows, o, stream);
+}
+
+extern "C" int tq_decode_paged_balanced_rows(
+    const void* q, int64_t q_stride_b, int64_t q_stride_h, int32_t q_dtype, const uint8_t* k_slab,
+    const uint8_t* v_slab, const int32_t* indices, const int32_t* indptr,
+    const int32_t* seq_lens, int32_t batch, int32_t num_qo_heads, int32_t num_kv_heads,
+    int32_t head_dim, int32_t padded_dim, int32_t block_size, int32_t ebs, int64_t num_blocks,
+    float sm_scale, const float* signs, int32_t max_rows, float* partition_o,
+    float* partition_lse, int32_t* split_rows, void* o, int32_t o_dtype, tq_stream_t stream) {
+  using namespace tq;
+  if (head_dim <= 0 || head_dim > padded_dim || head_dim % 8 != 0) {
+    set_error("decode_rows: head_dim %d must be a multiple of 8 up to padded_dim %d", head_dim,
+              padded_dim);
+    return kEinval;
+  }
+  if ((q_dtype != TQ_F16 && q_dtype != TQ_BF16) || (o_dtype != TQ_F16 && o_dtype != TQ_BF16)) {
+    set_error("decode_rows: q and o must be fp16 or bf16");
+    return kEinval;
+  }
+  if ((uintptr_t)o % 8) {
+    set_error("decode_rows: o must be 8-byte aligned");
+    return kEinval;
+  }
+  return tq::decode_balanced(q, q_stride_b, q_stride_h, k_slab, v_slab, indices, indptr,
+                             seq_lens, batch, num_qo_heads, num_kv_heads, head_dim, padded_dim,
+                             block_size, ebs, num_blocks, sm_scale, signs, max_rows,
+                             partition_o, partition_lse, split_rows, o, stream, head_dim,
+                             q_dtype == TQ_BF16, o_dtype == TQ_BF16);
 }
 
 namespace tq {

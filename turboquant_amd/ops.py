@@ -171,11 +171,44 @@ def decode_paged_balanced(q: torch.Tensor, kv_cache: torch.Tensor, indices: torc
     partial-row table (sequence b owns rows split_indptr[b] ..
     split_indptr[b + 1]) and, last, the unit size in tokens.  No host read,
     so it can be captured in a HIP graph whose seq_lens change per replay."""
+    _require_gpu(q, o)
+    if q.dtype != torch.float16:
+        raise RuntimeError("q must be fp16 [B, Hq, padded_dim] with a contiguous last dim")
+    if o.dtype != torch.float16:
+        raise RuntimeError("o_ws shape mismatch")
+    return _decode_balanced(q, kv_cache, indices, indptr, seq_lens, num_kv_heads, head_dim,
+                            padded_dim, sm_scale, signs, o, partition_o, partition_lse,
+                            split_indptr, int(padded_dim))
+
+
+def decode_paged_balanced_rows(q: torch.Tensor, kv_cache: torch.Tensor, indices: torch.Tensor,
+                               indptr: torch.Tensor, seq_lens: torch.Tensor, num_kv_heads: int,
+                               head_dim: int, padded_dim: int, sm_scale: float,
+                               signs: torch.Tensor | None, o: torch.Tensor,
+                               partition_o: torch.Tensor, partition_lse: torch.Tensor,
+                               split_indptr: torch.Tensor) -> torch.Tensor:
+    """decode_paged_balanced over the model's own rows: q and o [B, Hq,
+    head_dim] (head_dim a multiple of 8), each fp16 or bf16, dims up to
+    padded_dim counting as zero (tq_decode_paged_balanced_rows)."""
+    if q.dtype not in (torch.float16, torch.bfloat16) or \
+            o.dtype not in (torch.float16, torch.bfloat16):
+        raise RuntimeError("q and o must be fp16 or bf16 [B, Hq, head_dim]")
+    return _decode_balanced(q, kv_cache, indices, indptr, seq_lens, num_kv_heads, head_dim,
+                            padded_dim, sm_scale, signs, o, partition_o, partition_lse,
+                            split_indptr, int(head_dim))
+
+
+def _decode_balanced(q, kv_cache, indices, indptr, seq_lens, num_kv_heads, head_dim, padded_dim,
+                     sm_scale, signs, o, partition_o, partition_lse, split_indptr, row_dim):
     _require_gpu(q, kv_cache, indices, indptr, seq_lens, o, partition_o, partition_lse,
                  split_indptr)
-    if q.dtype != torch.float16 or q.dim() != 3 or q.size(2) != padded_dim or q.stride(2) != 1:
-        raise RuntimeError("q must be fp16 [B, Hq, padded_dim] with a contiguous last dim")
-    b, hq, pd = q.shape
+    if q.dim() != 3 or q.size(2) != row_dim or q.stride(2) != 1:
+        raise RuntimeError("q must be fp16 [B, Hq, padded_dim] with a contiguous last dim"
+                           if row_dim == padded_dim else
+                           "q must be [B, Hq, head_dim] with a contiguous last dim")
+    b, hq, _ = q.shape
+    pd = int(padded_dim)
+    rows_op = row_dim != pd or q.dtype != torch.float16 or o.dtype != torch.float16
     for t, name in ((indices, "indices"), (indptr, "indptr"), (seq_lens, "seq_lens"),
                     (split_indptr, "split_indptr")):
         if t.dtype != torch.int32 or not t.is_contiguous():
@@ -184,7 +217,7 @@ def decode_paged_balanced(q: torch.Tensor, kv_cache: torch.Tensor, indices: torc
         raise RuntimeError("seq_lens / indptr shorter than the batch")
     if split_indptr.numel() < b + 2:
         raise RuntimeError("split_indptr must hold batch + 2 entries")
-    if tuple(o.shape) != (b, hq, pd) or o.dtype != torch.float16 or not o.is_contiguous():
+    if tuple(o.shape) != (b, hq, row_dim) or not o.is_contiguous():
         raise RuntimeError("o_ws shape mismatch")
     if (partition_o.dtype != torch.float32 or partition_o.dim() != 3
             or tuple(partition_o.shape[1:]) != (hq, pd) or not partition_o.is_contiguous()):
@@ -209,12 +242,16 @@ def decode_paged_balanced(q: torch.Tensor, kv_cache: torch.Tensor, indices: torc
     base = kv_cache.data_ptr()
     slab = nb * bs * hk * ebs
     with torch.cuda.device(q.device):
-        rc = lib.tq_decode_paged_balanced(
-            q.data_ptr(), q.stride(0), q.stride(1), base, base + slab, indices.data_ptr(),
-            indptr.data_ptr(), seq_lens.data_ptr(), b, hq, int(num_kv_heads), int(head_dim),
-            int(padded_dim), bs, ebs, nb, float(sm_scale), sp, rows, partition_o.data_ptr(),
-            partition_lse.data_ptr(), split_indptr.data_ptr(), o.data_ptr(),
-            _stream_ptr(q.device))
+        args = (base, base + slab, indices.data_ptr(), indptr.data_ptr(), seq_lens.data_ptr(), b,
+                hq, int(num_kv_heads), int(head_dim), pd, bs, ebs, nb, float(sm_scale), sp, rows,
+                partition_o.data_ptr(), partition_lse.data_ptr(), split_indptr.data_ptr(),
+                o.data_ptr())
+        st = _stream_ptr(q.device)
+        if rows_op:
+            rc = lib.tq_decode_paged_balanced_rows(q.data_ptr(), q.stride(0), q.stride(1),
+                                                   _DTYPES[q.dtype], *args, _DTYPES[o.dtype], st)
+        else:
+            rc = lib.tq_decode_paged_balanced(q.data_ptr(), q.stride(0), q.stride(1), *args, st)
     _lib.check(rc, "decode_paged_balanced")
     return o
 
@@ -810,6 +847,16 @@ def _balanced_ws(q, kv_cache, indices, indptr, seq_lens, num_kv_heads, head_dim,
                           partition_lse_ws, split_indptr)
 
 
+def _balanced_rows_ws(q, kv_cache, indices, indptr, seq_lens, num_kv_heads, head_dim, padded_dim,
+                      sm_scale, hadamard_signs, o_ws, partition_o_ws, partition_lse_ws,
+                      split_indptr) -> None:
+    """turboquant_v5::decode_paged_balanced_rows_ws: decode_paged_balanced_rows,
+    its result in o_ws."""
+    decode_paged_balanced_rows(q, kv_cache, indices, indptr, seq_lens, num_kv_heads, head_dim,
+                               padded_dim, sm_scale, hadamard_signs, o_ws, partition_o_ws,
+                               partition_lse_ws, split_indptr)
+
+
 def _register_fakes() -> None:
     """Meta ("fake") kernels, so that torch.compile and vLLM's graph capture
     can trace the ops without running them: the write mutates its cache
@@ -829,11 +876,13 @@ def _register_fakes() -> None:
                  "decode_v5_from_cache_splitkv_ws"):
         register_fake(f"turboquant_v5::{name}", _decode_fake, lib=_libs[1])
 
-    @register_fake("turboquant_v5::decode_paged_balanced_ws", lib=_libs[1])
     def _balanced_fake(q, kv_cache, indices, indptr, seq_lens, num_kv_heads, head_dim,
                        padded_dim, sm_scale, hadamard_signs, o_ws, partition_o_ws,
                        partition_lse_ws, split_indptr):
         return None
+
+    for name in ("decode_paged_balanced_ws", "decode_paged_balanced_rows_ws"):
+        register_fake(f"turboquant_v5::{name}", _balanced_fake, lib=_libs[1])
 
 
 def register_ops() -> None:
@@ -880,12 +929,14 @@ def register_ops() -> None:
     # into the other workspaces, and says so in its schema (returning
     # nothing: functionalization refuses aliased outputs of custom ops), so
     # functionalization and torch.compile keep the call and its writes
-    d.define("decode_paged_balanced_ws(Tensor q, Tensor kv_cache, Tensor indices, "
-             "Tensor indptr, Tensor seq_lens, int num_kv_heads, int head_dim, "
-             "int padded_dim, float sm_scale, Tensor hadamard_signs, Tensor(a!) o_ws, "
-             "Tensor(b!) partition_o_ws, Tensor(c!) partition_lse_ws, "
-             "Tensor(d!) split_indptr) -> ()")
-    d.impl("decode_paged_balanced_ws", _balanced_ws, "CUDA")
+    for name, fn in (("decode_paged_balanced_ws", _balanced_ws),
+                     ("decode_paged_balanced_rows_ws", _balanced_rows_ws)):
+        d.define(f"{name}(Tensor q, Tensor kv_cache, Tensor indices, "
+                 "Tensor indptr, Tensor seq_lens, int num_kv_heads, int head_dim, "
+                 "int padded_dim, float sm_scale, Tensor hadamard_signs, Tensor(a!) o_ws, "
+                 "Tensor(b!) partition_o_ws, Tensor(c!) partition_lse_ws, "
+                 "Tensor(d!) split_indptr) -> ()")
+        d.impl(name, fn, "CUDA")
     _libs.extend([w, d])
     _register_fakes()
     _registered = True

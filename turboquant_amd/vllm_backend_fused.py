@@ -156,6 +156,7 @@ class TurboQuantFusedImpl(FlashAttentionImpl):
         self._decode_op = None
         self._decode_op_name = None
         self._write_op = None
+        self._rows_op = None
 
     # ---------------------------------------------------------------- setup
     @staticmethod
@@ -247,6 +248,7 @@ class TurboQuantFusedImpl(FlashAttentionImpl):
             from .decoder_dispatch import pick_decode_op
             ops.register_ops()
             self._write_op = torch.ops.turboquant_write.quantize_write_kv_cache
+            self._rows_op = torch.ops.turboquant_v5.decode_paged_balanced_rows_ws
             self._decode_op, self._decode_op_name = pick_decode_op()
 
     # ---------------------------------------------------------------- write
@@ -364,6 +366,18 @@ class TurboQuantFusedImpl(FlashAttentionImpl):
                   if qsl[i + 1] > qsl[i]]
         return self._attend_chunks(chunks, query, key, value, None, None, output)
 
+    def _rows_op_takes(self, q, o):
+        """Whether the decode over the model's own rows
+        (decode_paged_balanced_rows) takes q and o [n, Hq, head_size]."""
+        if torch.compiler.is_compiling() or type(q) is not torch.Tensor \
+                or type(o) is not torch.Tensor:
+            return False  # no addresses to look at
+        half = (torch.float16, torch.bfloat16)
+        return (q.dtype in half and o.dtype in half and self.head_size % 8 == 0
+                and q.stride(2) == 1 and q.stride(0) % 8 == 0 and q.stride(1) % 8 == 0
+                and q.stride(1) >= self.head_size and q.data_ptr() % 16 == 0
+                and o.is_contiguous() and o.data_ptr() % 8 == 0)
+
     def _decode_ws(self, n, pages, device):
         """Balanced-decode workspace for n decode rows of a mixed batch."""
         key = ("mixed", n, pages)
@@ -446,25 +460,21 @@ class TurboQuantFusedImpl(FlashAttentionImpl):
                 idx = torch.tensor(dec, dtype=torch.long, device=dev)
                 q = query.index_select(0, rows)
                 sub_bt, sl = bt.index_select(0, idx), attn_metadata.seq_lens.index_select(0, idx)
+            sub_bt, sl = sub_bt.to(torch.int32).contiguous(), sl.to(torch.int32).contiguous()
+            ws = self._decode_ws(n, sub_bt.shape[1], dev)
+            args = (kv_cache, sub_bt.reshape(-1), ws["indptr"], sl, self.num_kv_heads,
+                    self.head_size, self._pd, self.scale, self._signs)
+            parts = (ws["partition_o"], ws["partition_lse"], ws["split_indptr"])
+            if run and self._rows_op_takes(q, output[rows]):
+                ops.decode_paged_balanced_rows(q, *args, output[rows], *parts)
+                return output
             q = q.to(torch.float16)
             if self.head_size < self._pd:
                 q = F.pad(q, (0, self._pd - self.head_size))
-            q = q.contiguous()
-            sub_bt, sl = sub_bt.to(torch.int32).contiguous(), sl.to(torch.int32).contiguous()
-            ws = self._decode_ws(n, sub_bt.shape[1], dev)
-            # the kernel writes the caller's rows directly when they have the
-            # op's layout
-            direct = (run and self.head_size == self._pd and output.dtype == torch.float16
-                      and output[rows].is_contiguous())
-            o = ops.decode_paged_balanced(q, kv_cache, sub_bt.reshape(-1), ws["indptr"], sl,
-                                          self.num_kv_heads, self.head_size, self._pd,
-                                          self.scale, self._signs,
-                                          output[rows] if direct else ws["o"],
-                                          ws["partition_o"], ws["partition_lse"],
-                                          ws["split_indptr"])
-            if run and not direct:
+            o = ops.decode_paged_balanced(q.contiguous(), *args, ws["o"], *parts)
+            if run:
                 output[rows].copy_(o[:, :, :self.head_size])
-            elif not run:
+            else:
                 output.index_copy_(0, rows, o[:, :, :self.head_size].to(output.dtype))
         return output
 
@@ -514,10 +524,8 @@ class TurboQuantFusedImpl(FlashAttentionImpl):
             if kv_indices.dtype != torch.int32:
                 kv_indices = kv_indices.to(torch.int32)
             q3 = q.view(num_actual, self.num_heads, self.head_size)
-            q_fp16 = q3.to(torch.float16)
-            if self.head_size < self._pd:
-                q_fp16 = F.pad(q_fp16, (0, self._pd - self.head_size))
-            batch_size = q_fp16.shape[0]
+            out3 = output[:num_actual].view(num_actual, self.num_heads, self.head_size)
+            batch_size = num_actual
             # the balanced plan takes up to BALANCED_MAX_BATCH sequences; a
             # larger decode batch takes the reference's static-split op (same
             # kernels, host-planned splits)
@@ -534,7 +542,16 @@ class TurboQuantFusedImpl(FlashAttentionImpl):
                 kv_indptr = ws["indptr"] = torch.arange(
                     batch_size + 1, dtype=torch.int32, device=q.device) * max_pages
             sl = seq_lens if seq_lens.dtype == torch.int32 else seq_lens.to(torch.int32)
-            out3 = output[:num_actual].view(num_actual, self.num_heads, self.head_size)
+            if balanced and not (self.head_size == self._pd and q3.dtype == out3.dtype
+                                 == torch.float16) and self._rows_op_takes(q3, out3):
+                # bf16 rows or a padded head size, read and written as they are
+                self._rows_op(q3, kv_cache, kv_indices, kv_indptr, sl, self.num_kv_heads,
+                              self.head_size, self._pd, self.scale, self._signs, out3,
+                              ws["partition_o"], ws["partition_lse"], ws["split_indptr"])
+                return output
+            q_fp16 = q3.to(torch.float16)
+            if self.head_size < self._pd:
+                q_fp16 = F.pad(q_fp16, (0, self._pd - self.head_size))
             # the kernel writes the caller's output directly when it has the
             # op's layout (fp16, contiguous, head_size == padded_dim)
             direct = (self.head_size == self._pd and out3.dtype == torch.float16
