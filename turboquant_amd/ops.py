@@ -28,6 +28,27 @@ from .geometry import entry_bytes
 _DTYPES = {torch.float32: _lib.TQ_F32, torch.float16: _lib.TQ_F16, torch.bfloat16: _lib.TQ_BF16}
 
 
+_nat = None
+
+
+def _native():
+    """The C++ forms of the calls below (_tq_torch.so, built beside the
+    library by ``python -m turboquant_amd.build``); loading it also binds the
+    registered ops.  Each takes the ordinary call and returns its result (True
+    where the call has none); False or None means that it did nothing, and the
+    checks here decide."""
+    global _nat
+    if _nat is None:
+        _lib.load()
+        try:
+            from . import _tq_torch
+        except ImportError as e:
+            raise RuntimeError(f"turboquant_amd._tq_torch cannot be loaded ({e}). "
+                               "Run `python -m turboquant_amd.build`.") from e
+        _nat = _tq_torch
+    return _nat
+
+
 def _stream_ptr(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
@@ -54,6 +75,9 @@ def quantize_write_kv_cache(kv_cache: torch.Tensor, key: torch.Tensor, value: to
     quantize_write_kv_cache (quantize_write_binding.cu:207-269) including its
     checks; key/value may be fp32 (as the reference requires), fp16 or bf16.
     """
+    if (_nat or _native()).write_cache(kv_cache, key, value, signs, slot_mapping, head_dim,
+                                       padded_dim):
+        return
     if kv_cache.dim() != 5 or kv_cache.size(0) != 2:
         raise RuntimeError("kv_cache leading dim must be 2 (K,V)")
     if slot_mapping.dtype != torch.int32:
@@ -171,6 +195,10 @@ def decode_paged_balanced(q: torch.Tensor, kv_cache: torch.Tensor, indices: torc
     partial-row table (sequence b owns rows split_indptr[b] ..
     split_indptr[b + 1]) and, last, the unit size in tokens.  No host read,
     so it can be captured in a HIP graph whose seq_lens change per replay."""
+    if (_nat or _native()).decode_balanced(q, kv_cache, indices, indptr, seq_lens, num_kv_heads,
+                                           head_dim, padded_dim, sm_scale, signs, o, partition_o,
+                                           partition_lse, split_indptr, False):
+        return o
     _require_gpu(q, o)
     if q.dtype != torch.float16:
         raise RuntimeError("q must be fp16 [B, Hq, padded_dim] with a contiguous last dim")
@@ -190,6 +218,10 @@ def decode_paged_balanced_rows(q: torch.Tensor, kv_cache: torch.Tensor, indices:
     """decode_paged_balanced over the model's own rows: q and o [B, Hq,
     head_dim] (head_dim a multiple of 8), each fp16 or bf16, dims up to
     padded_dim counting as zero (tq_decode_paged_balanced_rows)."""
+    if (_nat or _native()).decode_balanced(q, kv_cache, indices, indptr, seq_lens, num_kv_heads,
+                                           head_dim, padded_dim, sm_scale, signs, o, partition_o,
+                                           partition_lse, split_indptr, True):
+        return o
     if q.dtype not in (torch.float16, torch.bfloat16) or \
             o.dtype not in (torch.float16, torch.bfloat16):
         raise RuntimeError("q and o must be fp16 or bf16 [B, Hq, head_dim]")
@@ -298,6 +330,9 @@ def prefill_attention_batch(q: torch.Tensor, o: torch.Tensor, requests, num_kv_h
     rows of q / o and of k / v (source 0) or k2 / v2 (source 1).  q and o fp16
     or bf16 [tokens, Hq, head_dim]; K / V fp16 [tokens, Hkv, padded_dim], zero
     past head_dim; head_dim a multiple of 8."""
+    if (_nat or _native()).prefill_batch(q, o, requests, num_kv_heads, head_dim, padded_dim,
+                                         sm_scale, k, v, k2, v2):
+        return o
     kvs = [t for t in (k, v, k2, v2) if t is not None]
     _require_gpu(q, o, *kvs)
     hq = q.size(1)
@@ -395,6 +430,9 @@ def prefill_gather(kv_cache: torch.Tensor | None, block_table: torch.Tensor | No
     does, the fresh rows of key / value (fp16, bf16 or fp32) converted, both
     zero-padded past head_dim.  kv_cache and block_table may be None when
     every ctx is 0."""
+    if (_nat or _native()).prefill_gather(kv_cache, block_table, key, value, requests, head_dim,
+                                          padded_dim, signs, out_k, out_v):
+        return
     _require_gpu(key, value, out_k, out_v)
     if key.dtype not in _DTYPES or value.dtype != key.dtype:
         raise RuntimeError(f"key/value must share a float dtype, got {key.dtype}/{value.dtype}")
@@ -451,6 +489,11 @@ def prefill_gather(kv_cache: torch.Tensor | None, block_table: torch.Tensor | No
     _lib.check(rc, "prefill_gather")
 
 
+def _floats(values) -> list | tuple:
+    """A host table as the sequence that the native calls take."""
+    return values if isinstance(values, (list, tuple)) else list(values)
+
+
 def _host_f32(values) -> "ctypes.Array":
     vals = [float(v) for v in values]
     return (ctypes.c_float * max(1, len(vals)))(*vals)
@@ -469,6 +512,10 @@ def mse_quantize(x: torch.Tensor, padded_dim: int, bit_width: int, signs: torch.
     [..., dim] -> (packed uint8 [..., padded_dim / per], norms fp32 [...]).
     `boundaries` are the codebook's 2^b - 1 scaled boundaries as host
     floats."""
+    boundaries = _floats(boundaries)
+    r = (_nat or _native()).mse_quantize(x, padded_dim, bit_width, signs, boundaries)
+    if r is not None:
+        return r
     _require_gpu(x, signs)
     if x.dtype != torch.float32:
         raise RuntimeError("mse_quantize: x must be fp32")
@@ -498,6 +545,11 @@ def mse_dequantize(packed: torch.Tensor, norms: torch.Tensor, dim: int, padded_d
     """TurboQuantMSE.dequantize on the GPU (tq_mse_dequantize): packed uint8
     [..., padded_dim / per] and norms [...] -> fp32 [..., dim].  `centroids`
     are the codebook's 2^b scaled levels as host floats."""
+    centroids = _floats(centroids)
+    r = (_nat or _native()).mse_dequantize(packed, norms, dim, padded_dim, bit_width, signs,
+                                           centroids)
+    if r is not None:
+        return r
     _require_gpu(packed, norms, signs)
     per = 2 if bit_width == 3 else 8 // bit_width
     if packed.dtype != torch.uint8 or packed.shape[-1] != padded_dim // per:
@@ -610,6 +662,11 @@ def prod_quantize_qjl_ws(x: torch.Tensor, padded_dim: int, mse_bit_width: int,
 
 def _prod_quantize_qjl(x, padded_dim, mse_bit_width, signs, boundaries, centroids, s_hi, s_lo,
                        large: bool):
+    boundaries, centroids = _floats(boundaries), _floats(centroids)
+    r = (_nat or _native()).prod_quantize_qjl(x, padded_dim, mse_bit_width, signs, boundaries,
+                                              centroids, s_hi, s_lo, large)
+    if r is not None:
+        return r
     _require_gpu(x, signs, s_hi, s_lo)
     if x.dtype != torch.float32:
         raise RuntimeError("prod_quantize_qjl: x must be fp32")
@@ -669,6 +726,12 @@ def prod_dequantize_qjl_ws(packed: torch.Tensor, norms: torch.Tensor, qjl_signs:
 
 def _prod_dequantize_qjl(packed, norms, qjl_signs, residual_norms, dim, padded_dim, mse_bit_width,
                          signs, centroids, st_hi, st_lo, large: bool):
+    centroids = _floats(centroids)
+    r = (_nat or _native()).prod_dequantize_qjl(packed, norms, qjl_signs, residual_norms, dim,
+                                                padded_dim, mse_bit_width, signs, centroids, st_hi,
+                                                st_lo, large)
+    if r is not None:
+        return r
     _require_gpu(packed, norms, qjl_signs, residual_norms, signs, st_hi, st_lo)
     per = 2 if mse_bit_width == 3 else 8 // mse_bit_width
     if packed.dtype != torch.uint8 or packed.shape[-1] != padded_dim // per:
@@ -837,26 +900,6 @@ def decode_v5_from_cache(q, kv_cache, indices, indptr, last_page_len, seq_lens, 
                                 splits, chunk)
 
 
-def _balanced_ws(q, kv_cache, indices, indptr, seq_lens, num_kv_heads, head_dim, padded_dim,
-                 sm_scale, hadamard_signs, o_ws, partition_o_ws, partition_lse_ws,
-                 split_indptr) -> None:
-    """turboquant_v5::decode_paged_balanced_ws: decode_paged_balanced, its
-    result in o_ws (the schema returns nothing)."""
-    decode_paged_balanced(q, kv_cache, indices, indptr, seq_lens, num_kv_heads, head_dim,
-                          padded_dim, sm_scale, hadamard_signs, o_ws, partition_o_ws,
-                          partition_lse_ws, split_indptr)
-
-
-def _balanced_rows_ws(q, kv_cache, indices, indptr, seq_lens, num_kv_heads, head_dim, padded_dim,
-                      sm_scale, hadamard_signs, o_ws, partition_o_ws, partition_lse_ws,
-                      split_indptr) -> None:
-    """turboquant_v5::decode_paged_balanced_rows_ws: decode_paged_balanced_rows,
-    its result in o_ws."""
-    decode_paged_balanced_rows(q, kv_cache, indices, indptr, seq_lens, num_kv_heads, head_dim,
-                               padded_dim, sm_scale, hadamard_signs, o_ws, partition_o_ws,
-                               partition_lse_ws, split_indptr)
-
-
 def _register_fakes() -> None:
     """Meta ("fake") kernels, so that torch.compile and vLLM's graph capture
     can trace the ops without running them: the write mutates its cache
@@ -887,7 +930,8 @@ def _register_fakes() -> None:
 
 def register_ops() -> None:
     """Define turboquant_write::* and turboquant_v5::* with the reference
-    schemas and bind the HIP implementations to the CUDA dispatch key."""
+    schemas and bind the HIP implementations to the CUDA dispatch key (the
+    write and the balanced decodes in C++, tq_torch.cpp; the others here)."""
     global _registered
     if _registered:
         return
@@ -895,7 +939,6 @@ def register_ops() -> None:
     w = Library("turboquant_write", "DEF")
     w.define("quantize_write_kv_cache(Tensor(a!) kv_cache, Tensor key, Tensor value, "
              "Tensor signs, Tensor slot_mapping, int head_dim, int padded_dim) -> ()")
-    w.impl("quantize_write_kv_cache", quantize_write_kv_cache, "CUDA")
     d = Library("turboquant_v5", "DEF")
     d.define("decode_v5_from_cache_paged_splitkv_ws(Tensor q, Tensor kv_cache, "
              "Tensor indices, Tensor indptr, Tensor last_page_len, Tensor seq_lens, "
@@ -929,14 +972,13 @@ def register_ops() -> None:
     # into the other workspaces, and says so in its schema (returning
     # nothing: functionalization refuses aliased outputs of custom ops), so
     # functionalization and torch.compile keep the call and its writes
-    for name, fn in (("decode_paged_balanced_ws", _balanced_ws),
-                     ("decode_paged_balanced_rows_ws", _balanced_rows_ws)):
+    for name in ("decode_paged_balanced_ws", "decode_paged_balanced_rows_ws"):
         d.define(f"{name}(Tensor q, Tensor kv_cache, Tensor indices, "
                  "Tensor indptr, Tensor seq_lens, int num_kv_heads, int head_dim, "
                  "int padded_dim, float sm_scale, Tensor hadamard_signs, Tensor(a!) o_ws, "
                  "Tensor(b!) partition_o_ws, Tensor(c!) partition_lse_ws, "
                  "Tensor(d!) split_indptr) -> ()")
-        d.impl(name, fn, "CUDA")
+    _native()  # binds the write and the two balanced ops
     _libs.extend([w, d])
     _register_fakes()
     _registered = True

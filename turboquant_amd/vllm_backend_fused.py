@@ -258,8 +258,9 @@ class TurboQuantFusedImpl(FlashAttentionImpl):
         sm = slot_mapping if slot_mapping.dtype == torch.int32 else slot_mapping.to(torch.int32)
         # fp16/bf16/fp32 rows go in as they are (the kernel converts exactly);
         # the reference's .float() copy is not needed
-        self._write_op(kv_cache, key[:num_tokens], value[:num_tokens], self._signs, sm,
-                       self.head_size, self._pd)
+        if key.shape[0] != num_tokens or value.shape[0] != num_tokens:
+            key, value = key[:num_tokens], value[:num_tokens]
+        self._write_op(kv_cache, key, value, self._signs, sm, self.head_size, self._pd)
 
     @torch.no_grad()
     def do_kv_cache_update(self, layer, key, value, kv_cache, slot_mapping):
@@ -505,7 +506,7 @@ class TurboQuantFusedImpl(FlashAttentionImpl):
                                    output, output_scale, **kwargs)
 
         num_actual = attn_metadata.num_actual_tokens
-        q = query[:num_actual]
+        q = query if query.shape[0] == num_actual else query[:num_actual]
         if output is None:
             output = torch.empty_like(q)
         block_table = attn_metadata.block_table
@@ -523,8 +524,9 @@ class TurboQuantFusedImpl(FlashAttentionImpl):
             kv_indices = block_table.reshape(-1)
             if kv_indices.dtype != torch.int32:
                 kv_indices = kv_indices.to(torch.int32)
-            q3 = q.view(num_actual, self.num_heads, self.head_size)
-            out3 = output[:num_actual].view(num_actual, self.num_heads, self.head_size)
+            rows = (num_actual, self.num_heads, self.head_size)
+            q3 = q.view(rows)
+            out3 = (output if output.shape[0] == num_actual else output[:num_actual]).view(rows)
             batch_size = num_actual
             # the balanced plan takes up to BALANCED_MAX_BATCH sequences; a
             # larger decode batch takes the reference's static-split op (same
