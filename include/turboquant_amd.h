@@ -404,6 +404,15 @@ int tq_prod_dequantize_qjl(const uint8_t* packed, const float* norms, const int8
                            float* out, tq_stream_t stream);
 
 /*
+ * The operand halves of the calls around it from the QJL matrix S fp32
+ * [dim, dim]: `halves` receives fp16 [4][padded_dim][padded_dim], S hi, S lo,
+ * S^T hi, S^T lo (hi + lo = S to 22 bits), zero past dim.  padded_dim a power
+ * of two 64..1024.
+ */
+int tq_qjl_halves(const float* s, int32_t dim, int32_t padded_dim, void* halves,
+                  tq_stream_t stream);
+
+/*
  * The same above padded_dim 128 (256, 512 or 1024), where S no longer fits a
  * wave's registers: the row kernels of tq_prod_quantize / tq_prod_dequantize
  * and the QJL product as a matrix-core kernel of its own.  Operands as above

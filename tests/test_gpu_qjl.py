@@ -109,3 +109,12 @@ def test_first_call_inside_a_graph():
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(z, eager)
+
+
+@pytest.mark.parametrize("dim", [50, 64, 97, 128, 257, 1000])
+def test_operand_halves(dim):
+    q = A.QJL(dim, device="cuda:0", seed=3)
+    pd = max(64, A.next_power_of_2(dim))
+    cpu = A.QJL(dim, device="cpu", seed=3).halves(pd)
+    for got, want in zip(q.halves(pd), cpu):
+        assert got.is_contiguous() and torch.equal(got.cpu(), want)

@@ -68,6 +68,7 @@ SIGNATURES = {
                                     _P, _P]),
     "tq_prod_dequantize_qjl": (_I32, [_P, _P, _P, _P, _I64, _I32, _I32, _I32, _P, _P, _P, _P,
                                       _P, _P]),
+    "tq_qjl_halves": (_I32, [_P, _I32, _I32, _P, _P]),
     "tq_prod_workspace_bytes": (_I64, [_I64, _I32]),
     "tq_prod_quantize_qjl_ws": (_I32, [_P, _I64, _I32, _I32, _I32, _P, _P, _P, _P, _P, _P, _P,
                                        _P, _P, _P, _I64, _P]),

@@ -189,15 +189,19 @@ class QJL:
             cache = {}
         if key in cache:
             return cache[key]
-        out = []
-        for m in (self.S, self.S.t()):
-            hi = m.half()
-            lo = (m - hi.float()).half()
-            for h in (hi, lo):
-                pad = torch.zeros((padded_dim, padded_dim), dtype=torch.float16,
-                                  device=self.S.device)
-                pad[:self.dim, :self.dim] = h
-                out.append(pad)
+        if self.S.is_cuda and self.S.dtype == torch.float32:
+            from . import ops
+            out = ops.qjl_halves(self.S, padded_dim)
+        else:
+            out = []
+            for m in (self.S, self.S.t()):
+                hi = m.half()
+                lo = (m - hi.float()).half()
+                for h in (hi, lo):
+                    pad = torch.zeros((padded_dim, padded_dim), dtype=torch.float16,
+                                      device=self.S.device)
+                    pad[:self.dim, :self.dim] = h
+                    out.append(pad)
         if self.S.is_cuda:
             if torch.cuda.is_current_stream_capturing():
                 return tuple(out)  # they hold values only once the graph runs: not kept

@@ -292,6 +292,33 @@ void qjl_gemm_kernel(QjlGemmParams p) {
   }
 }
 
+// S [dim][dim] and its transpose as fp16 hi + lo halves, zero-padded: out is
+// [4][pd][pd], S hi, S lo, S^T hi, S^T lo.  32 x 32 tiles through LDS; one
+// launch where torch took a dozen small ones (120 us of a first call).
+__global__ __launch_bounds__(256) void split_halves_kernel(const float* __restrict__ s, int dim,
+                                                           int pd, _Float16* __restrict__ out) {
+  __shared__ float tile[32][33];
+  const int r0 = 32 * (int)blockIdx.y, c0 = 32 * (int)blockIdx.x;
+  const int x = threadIdx.x & 31, y = threadIdx.x >> 5;
+  const int64_t sq = (int64_t)pd * pd;
+  auto put = [&](int64_t at, float v) {
+    const _Float16 hi = (_Float16)v;
+    out[at] = hi;
+    out[at + sq] = (_Float16)(v - (float)hi);
+  };
+#pragma unroll
+  for (int i = y; i < 32; i += 8) {
+    const int r = r0 + i, c = c0 + x;
+    const float v = r < dim && c < dim ? s[(int64_t)r * dim + c] : 0.0f;
+    tile[i][x] = v;
+    put((int64_t)r * pd + c, v);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = y; i < 32; i += 8)  // row c0 + i of S^T
+    put(2 * sq + (int64_t)(c0 + i) * pd + r0 + x, tile[x][i]);
+}
+
 }  // namespace
 
 hipError_t launch_qjl(bool quant, const _Float16* xh, const _Float16* xl, const int8_t* z,
@@ -320,3 +347,24 @@ hipError_t launch_qjl(bool quant, const _Float16* xh, const _Float16* xl, const 
 }
 
 }  // namespace tq
+
+extern "C" int tq_qjl_halves(const float* s, int32_t dim, int32_t padded_dim, void* halves,
+                             tq_stream_t stream) {
+  using namespace tq;
+  if (padded_dim < 64 || padded_dim > 1024 || (padded_dim & (padded_dim - 1)) != 0 || dim < 1 ||
+      dim > padded_dim) {
+    set_error("qjl_halves: padded_dim %d must be a power of two 64..1024, dim %d at most that",
+              padded_dim, dim);
+    return kEinval;
+  }
+  if (!s || !halves) {
+    set_error("qjl_halves: null pointer");
+    return kEinval;
+  }
+  hipLaunchKernelGGL(split_halves_kernel, dim3(padded_dim / 32, padded_dim / 32), dim3(256), 0,
+                     reinterpret_cast<hipStream_t>(stream), s, dim, padded_dim,
+                     static_cast<_Float16*>(halves));
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) set_error("qjl_halves: launch failed: %s", hipGetErrorString(e));
+  return (int)e;
+}

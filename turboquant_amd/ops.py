@@ -506,6 +506,22 @@ def _aligned16(t: torch.Tensor) -> torch.Tensor:
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
+def qjl_halves(s: torch.Tensor, padded_dim: int):
+    """(S hi, S lo, S^T hi, S^T lo): fp16 halves of the QJL matrix s fp32
+    [dim, dim], zero-padded to [padded_dim, padded_dim] (tq_qjl_halves)."""
+    _require_gpu(s)
+    if s.dtype != torch.float32 or s.dim() != 2 or s.size(0) != s.size(1):
+        raise RuntimeError("qjl_halves: S must be a square fp32 matrix")
+    s = s.contiguous()
+    out = torch.empty((4, padded_dim, padded_dim), dtype=torch.float16, device=s.device)
+    lib = _lib.load()
+    with torch.cuda.device(s.device):
+        rc = lib.tq_qjl_halves(s.data_ptr(), s.size(0), int(padded_dim), out.data_ptr(),
+                               _stream_ptr(s.device))
+    _lib.check(rc, "qjl_halves")
+    return out.unbind(0)
+
+
 def mse_quantize(x: torch.Tensor, padded_dim: int, bit_width: int, signs: torch.Tensor,
                  boundaries) -> tuple[torch.Tensor, torch.Tensor]:
     """TurboQuantMSE.quantize on the GPU (tq_mse_quantize): x fp32
