@@ -46,8 +46,8 @@ CENTROIDS_N01 = {
 
 # Vectors from which TurboQuantProd.dequantize above padded size 128 forms z S
 # with this package's kernel.  The kernel is the faster one at every size (1500
-# vectors of dim 1000: 42 against 63 us; 4096: 48 against 88; 20011: 143
-# against 386) and the nearer one to 64 bits; below the line the product stays
+# vectors of dim 1000: 41 against 63 us; 4096 of 1024: 43 against 88; 20011:
+# 135 against 386) and the nearer one to 64 bits; below the line the product stays
 # torch's fp32 GEMM so that small batches keep equalling torch's expression
 # z.float() @ S bit for bit, which callers compare against.
 QJL_GEMM_MIN = 2048

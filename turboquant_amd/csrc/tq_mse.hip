@@ -323,6 +323,51 @@ __device__ __forceinline__ void load_row(const MseParams& p, int64_t row, int su
   }
 }
 
+// The rows of a wave (64 / P vectors from row0) through its LDS stage: 1 KB of
+// consecutive bytes per copy instruction, 16-byte pieces swizzled within each
+// 128 bytes so that the lanes' reads of their own E dims spread over the banks.
+// dim % 4 == 0.  Used by the plain quantize from padded size 256 up where dim
+// is not the padded size (60,000 x 1000: 59 us against 82 with float4 loads
+// under a mask; 300,000 x 200: 68 against 83).  Full rows gain nothing from it
+// (256 .. 1024 dims: -8% with the input in the last-level cache, +4% from HBM),
+// narrower ones and the residual kernel lose 5-10%.
+template <int PD>
+__device__ __forceinline__ void load_rows_staged(const MseParams& p, int64_t row0, int lane,
+                                                 float* stage, float (&v)[MseGeom<PD>::E]) {
+  constexpr int E = MseGeom<PD>::E;
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int VW = 64 / MseGeom<PD>::P;
+  const int64_t left = p.n - row0;
+  const int rows = left < VW ? (left < 0 ? 0 : (int)left) : VW;
+  const uint64_t a = (uint64_t)(uintptr_t)(p.x + (rows > 0 ? row0 * p.dim : 0));
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+  const int nrec = __builtin_amdgcn_readfirstlane(rows * p.dim * 4);
+  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(uintptr_t)(((uint64_t)hi << 32) | lo), (short)0, nrec, 0x00020000);
+#pragma unroll
+  for (int i = 0; i < VW * PD / 256; i++) {
+    const int c = 64 * i + lane;                          // physical piece
+    const int l = (c & ~7) | ((c & 7) ^ ((c >> 3) & 7));  // the piece it holds
+    const int vec = l / (PD / 4), d = 4 * (l % (PD / 4));
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        r, (void*)(stage + 256 * i), 16,
+        d < p.dim ? (uint32_t)(vec * p.dim + d) * 4u : 0x80000000u, 0, 0, 0);
+  }
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the copies are this wave's own
+  __builtin_amdgcn_wave_barrier();
+#endif
+#pragma unroll
+  for (int i = 0; i < E / 4; i++) {
+    const int l = lane * (E / 4) + i, c = (l & ~7) | ((l & 7) ^ ((l >> 3) & 7));
+    const float4 f = *reinterpret_cast<const float4*>(stage + 4 * c);
+    v[4 * i] = f.x;
+    v[4 * i + 1] = f.y;
+    v[4 * i + 2] = f.z;
+    v[4 * i + 3] = f.w;
+  }
+}
+
 // v holds the row as load_row leaves it
 template <int PD, int BITS, bool RES>
 __device__ __forceinline__ void quantize_row(const MseParams& p, const float* bnd,
@@ -421,7 +466,9 @@ __device__ __forceinline__ void quantize_row(const MseParams& p, const float* bn
   }
 }
 
-template <int PD, int BITS, bool RES>
+// STG: rows come through the LDS stage (its own instantiation: the 32 KB of LDS
+// cost full rows 7% in occupancy where they were only reserved)
+template <int PD, int BITS, bool RES, bool STG = false>
 __global__ __launch_bounds__(kMseThreads) void mse_quantize_kernel(MseParams p) {
   using MG = MseGeom<PD>;
   constexpr int P = MG::P, E = MG::E;
@@ -436,7 +483,13 @@ __global__ __launch_bounds__(kMseThreads) void mse_quantize_kernel(MseParams p) 
   const int lane = threadIdx.x & 63, sub = lane % P;
   const int64_t row = (int64_t)blockIdx.x * MG::VPB + threadIdx.x / P;
   float v[E];
-  load_row<PD>(p, row, sub, v);
+  if constexpr (STG) {
+    __shared__ __attribute__((aligned(16))) float xs[kMseThreads / 64][(64 / P) * PD];
+    load_rows_staged<PD>(p, (int64_t)blockIdx.x * MG::VPB + (threadIdx.x >> 6) * (64 / P), lane,
+                         xs[threadIdx.x >> 6], v);
+  } else {
+    load_row<PD>(p, row, sub, v);
+  }
   quantize_row<PD, BITS, RES>(p, bnd, bins, cen, row, sub, v);
   if constexpr (RES) {
     if (row >= p.n) return;
@@ -858,10 +911,14 @@ template <int PD>
 hipError_t launch_mse(bool quant, int bits, const MseParams& p, hipStream_t st) {
   const dim3 grid((unsigned)((p.n + MseGeom<PD>::VPB - 1) / MseGeom<PD>::VPB));
   const dim3 block(kMseThreads);
+  const bool staged = PD >= 256 && p.dim != PD && (p.dim & 3) == 0;
 #define TQ_MSE_CASE(B)                                                                   \
   case B:                                                                                \
     if (quant && p.rnorm)                                                                \
       hipLaunchKernelGGL((mse_quantize_kernel<PD, B, true>), grid, block, 0, st, p);     \
+    else if (quant && staged)                                                            \
+      hipLaunchKernelGGL((mse_quantize_kernel<PD, B, false, (PD >= 256)>), grid, block, 0, st, \
+                         p);                                                              \
     else if (quant)                                                                      \
       hipLaunchKernelGGL((mse_quantize_kernel<PD, B, false>), grid, block, 0, st, p);    \
     else if (p.add)                                                                      \

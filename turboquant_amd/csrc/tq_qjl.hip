@@ -20,13 +20,16 @@
 // neighbouring tiles, the output blocks of one vector tile first: X is read
 // into one L2 once.
 //
-// MFMA-bound.  Measured at 20,011 vectors of dim 1000: sign(S r) 125 us (126
-// GFLOP issued: 1.0 PFLOP/s; a plain 8192^3 library product reaches 1.23 on
-// this card), z S 85 us; as fp32 library products they took 377 and 357 us,
-// plus 130 us of compares, conversions and sign arithmetic around them.
-// Two workgroups per CU (64 KB of LDS each) hide each other's barrier; the
-// signs of a step are loaded to registers a step ahead and written to LDS
-// behind the copies' own wait (loaded and waited for inside the step: 125 us).
+// Measured at 20,011 vectors of dim 1000: sign(S r) 123 us (126 GFLOP issued:
+// 1.0 PFLOP/s; a plain 8192^3 library product reaches 1.23 on this card), z S
+// 102 us; as fp32 library products they took 377 and 357 us, plus 130 us of
+// compares, conversions and sign arithmetic around them.  What bounds them is
+// the wait per K step (MFMAs fill half of it) and the last round of tiles, so
+// as many workgroups per CU as fit hide each other's barrier: two of the
+// quantize (64 KB of LDS each), three of the dequantize (48 KB, 132 VGPRs; two
+// of them 112 us).  The signs of a step are in registers a step ahead and go
+// to LDS behind the copies' own wait (loaded and waited for inside the step:
+// 125 us).
 #include "tq_qjl.h"
 
 namespace tq {
@@ -84,7 +87,7 @@ __device__ __forceinline__ void z_to_half(uint32_t w, uint32_t& lo, uint32_t& hi
 }
 
 template <bool QUANT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(QUANT ? 2 : 3)))
 void qjl_gemm_kernel(QjlGemmParams p) {
   // quantize: xh, xl, wh, wl; dequantize: z as fp16, wh, wl
   constexpr int kNS = QUANT ? 4 : 3;
@@ -117,11 +120,13 @@ void qjl_gemm_kernel(QjlGemmParams p) {
   const bool zlive = !QUANT && m0 + zr < p.n;
   const bool zvec = !QUANT && (p.dim & 7) == 0;  // rows 8-byte aligned (the entry checks z)
   const int64_t zend = p.n * p.dim;
-  uint32_t zreg[4];
-  auto load_z = [&](int k0) {
+  // four K steps at a time: a thread's pieces of one 128-byte line go out
+  // together (4% at dim 1024 against a step at a time)
+  uint32_t zreg[4][4];
+  auto load_z = [&](int t0) {
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const int k = k0 + zk + 8 * h;
+    for (int i = 0; i < 8; i++) {
+      const int h = i & 1, k = (t0 + i / 2) * kBK + zk + 8 * h;
       uint2 v = {0u, 0u};
       if (zlive && k < p.dim) {
         if (zvec) {
@@ -134,19 +139,19 @@ void qjl_gemm_kernel(QjlGemmParams p) {
             (e < 4 ? v.x : v.y) |= (uint32_t)(uint8_t)zrow[k + e] << (8 * (e & 3));
         }
       }
-      zreg[2 * h] = v.x;
-      zreg[2 * h + 1] = v.y;
+      zreg[i / 2][2 * h] = v.x;
+      zreg[i / 2][2 * h + 1] = v.y;
     }
   };
-  auto store_z = [&](uint8_t* b) {
+  auto store_z = [&](uint8_t* b, const uint32_t* zr4) {
 #pragma unroll
     for (int h = 0; h < 2; h++) {
       u32x4 v;
       uint32_t a, c;
-      z_to_half(zreg[2 * h], a, c);
+      z_to_half(zr4[2 * h], a, c);
       v[0] = a;
       v[1] = c;
-      z_to_half(zreg[2 * h + 1], a, c);
+      z_to_half(zr4[2 * h + 1], a, c);
       v[2] = a;
       v[3] = c;
       *reinterpret_cast<u32x4*>(b + chunk_at(zr, 2 * (threadIdx.x & 1) + h)) = v;
@@ -221,23 +226,26 @@ void qjl_gemm_kernel(QjlGemmParams p) {
   issue(0, buf0);
   if constexpr (!QUANT) {
     load_z(0);
-    store_z(buf0);
-    load_z(kBK);  // (past the last step: zeros)
+    store_z(buf0, zreg[0]);
   }
-  auto iter = [&](int t, uint8_t* cur, uint8_t* nxt) {
+  auto iter = [&](int t, int j, uint8_t* cur, uint8_t* nxt) {  // j = t % 4
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's copies of step t
     __syncthreads();
     if (t + 1 < nk) {
-      // the signs of step t + 1 arrived with the copies just waited for
-      if constexpr (!QUANT) store_z(nxt);
+      // the signs of step t + 1 are in registers: loaded at the latest a step
+      // ago, they arrived with the copies just waited for
+      if constexpr (!QUANT) store_z(nxt, zreg[(j + 1) & 3]);
       issue((t + 1) * kBK, nxt);
-      if constexpr (!QUANT) load_z((t + 2) * kBK);
+      if constexpr (!QUANT)
+        if (j == 2) load_z(t + 2);  // (past the last step: zeros)
     }
     step(cur);
   };
-  for (int t = 0; t < nk; t += 2) {
-    iter(t, buf0, buf1);
-    if (t + 1 < nk) iter(t + 1, buf1, buf0);
+  for (int t = 0; t < nk; t += 4) {
+    iter(t, 0, buf0, buf1);
+    if (t + 1 < nk) iter(t + 1, 1, buf1, buf0);
+    if (t + 2 < nk) iter(t + 2, 2, buf0, buf1);
+    if (t + 3 < nk) iter(t + 3, 3, buf1, buf0);
   }
 
   if constexpr (QUANT) {
