@@ -61,6 +61,18 @@ def test_dequantize_term_against_64_bits(dim, n):
         assert bool(((got - want).abs() <= bound).all()), (got - want).abs().max().item()
 
 
+# either side of the lines between the kernel forms (tiles of 32, 64, 128),
+# ragged in vectors, outputs and K
+FORMS = [(1000, 256), (1000, 257), (1000, 2560), (1000, 2561), (1023, 2700), (1000, 5121),
+         (257, 8193), (513, 3001), (130, 20011), (512, 5000), (1024, 10300)]
+
+
+@pytest.mark.parametrize("dim,n", FORMS)
+def test_every_form_against_64_bits(dim, n):
+    test_quantize_signs_against_64_bits(dim, n)
+    test_dequantize_term_against_64_bits(dim, n)
+
+
 def test_dequantize_paths_agree_around_the_size_rule():
     """One vector fewer than QJL_GEMM_MIN (the torch product) and that many:
     the rows they share are within the roundings of both."""

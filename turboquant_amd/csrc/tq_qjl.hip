@@ -5,7 +5,9 @@
 //
 // Both are C = X W^T with K (= dim) contiguous in X and W, in tiles of 128
 // vectors x 128 outputs per workgroup of four waves (each 64 x 64, 2 x 2
-// blocks of v_mfma_f32_32x32x16_f16), K in steps of 32 through two LDS
+// blocks of v_mfma_f32_32x32x16_f16; 64 x 64 tiles of one block per wave where
+// 128 x 128 ones leave CUs idle, and a split-K kernel for the smallest
+// quantizes: launch_qjl has the rule), K in steps of 32 through two LDS
 // buffers.  fp32 operands enter as fp16 hi + lo halves:
 //  * quantize: X = the unit residual times 4096 (exact; it keeps lo out of the
 //    fp16 subnormals, and a sign does not see it), W = S; three products
@@ -40,9 +42,8 @@ typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kBT = 128;           // tile edge (vectors, outputs)
-constexpr int kBK = 32;            // K step: 64 bytes of a row
-constexpr int kSide = kBT * kBK * 2;  // bytes of one operand half in LDS
+constexpr int kBK = 32;   // K step: 64 bytes of a row
+constexpr int kCus = 256;  // compute units of the card
 
 struct QjlGemmParams {
   const _Float16* xh;   // quantize: residual halves [n][ldk]
@@ -64,12 +65,13 @@ __device__ __forceinline__ int chunk_at(int r, int c) {
 }
 
 #if defined(__HIP_DEVICE_COMPILE__)
+template <int ROWS>
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const _Float16* base, int64_t row,
                                                             int64_t rows, int ldk) {
   const uint64_t a = (uint64_t)(uintptr_t)(base + row * ldk);
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
   const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
-  const int64_t live = rows - row < kBT ? rows - row : kBT;
+  const int64_t live = rows - row < ROWS ? rows - row : ROWS;
   const int nrec = __builtin_amdgcn_readfirstlane((int)live * ldk * 2);
   return __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)(((uint64_t)hi << 32) | lo), (short)0,
                                            nrec, 0x00020000);
@@ -86,9 +88,13 @@ __device__ __forceinline__ void z_to_half(uint32_t w, uint32_t& lo, uint32_t& hi
                                         0x64646464u, u, 0x04030402u)) - b));
 }
 
-template <bool QUANT>
+// BT: the tile's edge, 128 or 64 (vectors, outputs).
+template <bool QUANT, int BT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(QUANT ? 2 : 3)))
 void qjl_gemm_kernel(QjlGemmParams p) {
+  constexpr int kSide = BT * kBK * 2;  // bytes of one operand half in LDS
+  constexpr int WB = BT / 64;          // 32 x 32 blocks per wave and direction
+  constexpr int NC = BT / 64;          // copies per wave and half, 8-sign pieces per thread
   // quantize: xh, xl, wh, wl; dequantize: z as fp16, wh, wl
   constexpr int kNS = QUANT ? 4 : 3;
   __shared__ __attribute__((aligned(16))) uint8_t buf0[kNS * kSide];
@@ -98,35 +104,36 @@ void qjl_gemm_kernel(QjlGemmParams p) {
   const int64_t per = (p.tiles + 7) / 8;
   const int64_t id = (int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
   if ((int64_t)(blockIdx.x >> 3) >= per || id >= p.tiles) return;
-  const int64_t m0 = id / p.ntn * kBT;        // first vector
-  const int n0 = (int)(id % p.ntn) * kBT;     // first output
+  const int64_t m0 = id / p.ntn * BT;        // first vector
+  const int n0 = (int)(id % p.ntn) * BT;     // first output
 
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int hh = lane >> 5, ln = lane & 31;
-  const int wm = 64 * (w & 1), wn = 64 * (w >> 1);  // the wave's vectors / outputs
+  const int wm = BT / 2 * (w & 1), wn = BT / 2 * (w >> 1);  // the wave's vectors / outputs
 
-  // copies: 1 KB = 16 rows of 64 bytes; wave w takes copies w and w + 4 of each
-  // half (8 per half).  Lane l writes row l / 4, physical chunk l % 4.
+  // copies: 1 KB = 16 rows of 64 bytes; wave w takes copies w (and w + 4) of
+  // each half.  Lane l writes row l / 4, physical chunk l % 4.
   const int crow = lane >> 2;
-  uint32_t coff[2];
+  uint32_t coff[NC];
 #pragma unroll
-  for (int i = 0; i < 2; i++) {
+  for (int i = 0; i < NC; i++) {
     const int row = 16 * (w + 4 * i) + crow;
     coff[i] = (uint32_t)(row * p.ldk * 2 + (((lane & 3) ^ ((row >> 1) & 3)) * 16));
   }
-  // dequantize: thread t stages signs of vector t / 2, 16 of a step's 32
-  const int zr = threadIdx.x >> 1, zk = 16 * (threadIdx.x & 1);
+  // dequantize: a thread stages 8 * NC of a step's 32 signs of one vector
+  constexpr int TPV = 4 / NC;  // threads per vector
+  const int zr = threadIdx.x / TPV, zk = 8 * NC * (threadIdx.x % TPV);
   const int8_t* zrow = QUANT ? nullptr : p.z + (m0 + zr < p.n ? m0 + zr : 0) * p.dim;
   const bool zlive = !QUANT && m0 + zr < p.n;
   const bool zvec = !QUANT && (p.dim & 7) == 0;  // rows 8-byte aligned (the entry checks z)
   const int64_t zend = p.n * p.dim;
   // four K steps at a time: a thread's pieces of one 128-byte line go out
   // together (4% at dim 1024 against a step at a time)
-  uint32_t zreg[4][4];
+  uint32_t zreg[4][2 * NC];
   auto load_z = [&](int t0) {
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const int h = i & 1, k = (t0 + i / 2) * kBK + zk + 8 * h;
+    for (int i = 0; i < 4 * NC; i++) {
+      const int h = i % NC, k = (t0 + i / NC) * kBK + zk + 8 * h;
       uint2 v = {0u, 0u};
       if (zlive && k < p.dim) {
         if (zvec) {
@@ -139,13 +146,13 @@ void qjl_gemm_kernel(QjlGemmParams p) {
             (e < 4 ? v.x : v.y) |= (uint32_t)(uint8_t)zrow[k + e] << (8 * (e & 3));
         }
       }
-      zreg[i / 2][2 * h] = v.x;
-      zreg[i / 2][2 * h + 1] = v.y;
+      zreg[i / NC][2 * h] = v.x;
+      zreg[i / NC][2 * h + 1] = v.y;
     }
   };
   auto store_z = [&](uint8_t* b, const uint32_t* zr4) {
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
+    for (int h = 0; h < NC; h++) {
       u32x4 v;
       uint32_t a, c;
       z_to_half(zr4[2 * h], a, c);
@@ -154,34 +161,34 @@ void qjl_gemm_kernel(QjlGemmParams p) {
       z_to_half(zr4[2 * h + 1], a, c);
       v[2] = a;
       v[3] = c;
-      *reinterpret_cast<u32x4*>(b + chunk_at(zr, 2 * (threadIdx.x & 1) + h)) = v;
+      *reinterpret_cast<u32x4*>(b + chunk_at(zr, NC * (threadIdx.x % TPV) + h)) = v;
     }
   };
   auto issue = [&](int k0, uint8_t* b) {
 #if defined(__HIP_DEVICE_COMPILE__)
     auto half = [&](const __amdgpu_buffer_rsrc_t& r, int side) {
 #pragma unroll
-      for (int i = 0; i < 2; i++)
+      for (int i = 0; i < NC; i++)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (void*)(b + side * kSide + 1024 * (w + 4 * i)),
                                                  16, coff[i], k0 * 2, 0, 0);
     };
     if constexpr (QUANT) {
-      half(rows_rsrc(p.xh, m0, p.n, p.ldk), 0);
-      half(rows_rsrc(p.xl, m0, p.n, p.ldk), 1);
+      half(rows_rsrc<BT>(p.xh, m0, p.n, p.ldk), 0);
+      half(rows_rsrc<BT>(p.xl, m0, p.n, p.ldk), 1);
     }
-    half(rows_rsrc(p.wh, n0, p.ldk, p.ldk), kNS - 2);
-    half(rows_rsrc(p.wl, n0, p.ldk, p.ldk), kNS - 1);
+    half(rows_rsrc<BT>(p.wh, n0, p.ldk, p.ldk), kNS - 2);
+    half(rows_rsrc<BT>(p.wl, n0, p.ldk, p.ldk), kNS - 1);
 #else
     (void)k0;
     (void)b;
 #endif
   };
 
-  f32x16 acc[2][2];  // [vector block][output block]
+  f32x16 acc[WB][WB];  // [vector block][output block]
 #pragma unroll
-  for (int i = 0; i < 2; i++)
+  for (int i = 0; i < WB; i++)
 #pragma unroll
-    for (int j = 0; j < 2; j++)
+    for (int j = 0; j < WB; j++)
 #pragma unroll
       for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
 
@@ -197,28 +204,28 @@ void qjl_gemm_kernel(QjlGemmParams p) {
       auto frag = [&](int side, int r) {
         return *reinterpret_cast<const half8_t*>(b + side * kSide + chunk_at(r + ln, 2 * s + hh));
       };
-      half8_t xh[2], xl[2], wh[2], wl[2];
+      half8_t xh[WB], xl[WB], wh[WB], wl[WB];
 #pragma unroll
-      for (int i = 0; i < 2; i++) {
+      for (int i = 0; i < WB; i++) {
         xh[i] = frag(0, wm + 32 * i);
         if constexpr (QUANT) xl[i] = frag(1, wm + 32 * i);
         wh[i] = frag(kNS - 2, wn + 32 * i);
         wl[i] = frag(kNS - 1, wn + 32 * i);
       }
 #pragma unroll
-      for (int i = 0; i < 2; i++)
+      for (int i = 0; i < WB; i++)
 #pragma unroll
-        for (int j = 0; j < 2; j++) acc[i][j] = mma(xh[i], wl[j], acc[i][j]);
+        for (int j = 0; j < WB; j++) acc[i][j] = mma(xh[i], wl[j], acc[i][j]);
       if constexpr (QUANT) {
 #pragma unroll
-        for (int i = 0; i < 2; i++)
+        for (int i = 0; i < WB; i++)
 #pragma unroll
-          for (int j = 0; j < 2; j++) acc[i][j] = mma(xl[i], wh[j], acc[i][j]);
+          for (int j = 0; j < WB; j++) acc[i][j] = mma(xl[i], wh[j], acc[i][j]);
       }
 #pragma unroll
-      for (int i = 0; i < 2; i++)
+      for (int i = 0; i < WB; i++)
 #pragma unroll
-        for (int j = 0; j < 2; j++) acc[i][j] = mma(xh[i], wh[j], acc[i][j]);
+        for (int j = 0; j < WB; j++) acc[i][j] = mma(xh[i], wh[j], acc[i][j]);
     }
   };
 
@@ -249,15 +256,15 @@ void qjl_gemm_kernel(QjlGemmParams p) {
   }
 
   if constexpr (QUANT) {
-    // signs of the tile staged in LDS as bytes ([vector][output], rows of 144
+    // signs of the tile staged in LDS as bytes ([vector][output], rows of BT + 16
     // bytes), then written as runs of a row
-    constexpr int kRS = kBT + 16;
-    static_assert(kBT * kRS <= kNS * kSide, "stage fits");
+    constexpr int kRS = BT + 16;
+    static_assert(BT * kRS <= kNS * kSide, "stage fits");
     __syncthreads();  // the last step's reads
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int i = 0; i < WB; i++)
 #pragma unroll
-      for (int j = 0; j < 2; j++)
+      for (int j = 0; j < WB; j++)
 #pragma unroll
         for (int q = 0; q < 4; q++) {
           uint32_t pk = 0;
@@ -268,27 +275,27 @@ void qjl_gemm_kernel(QjlGemmParams p) {
                                        4 * hh) = pk;
         }
     __syncthreads();
-    const int cols = p.dim - n0 < kBT ? p.dim - n0 : kBT;
+    const int cols = p.dim - n0 < BT ? p.dim - n0 : BT;
     if ((p.dim & 7) == 0) {
 #pragma unroll
-      for (int i = 0; i < 8; i++) {
-        const int r = 16 * i + (threadIdx.x >> 4), c = 8 * (threadIdx.x & 15);
+      for (int i = threadIdx.x; i < BT * BT / 8; i += 256) {
+        const int r = i / (BT / 8), c = 8 * (i % (BT / 8));
         if (m0 + r < p.n && c < cols)
           *reinterpret_cast<uint2*>(p.zout + (m0 + r) * p.dim + n0 + c) =
               *reinterpret_cast<const uint2*>(buf0 + r * kRS + c);
       }
     } else {
-      for (int i = threadIdx.x; i < kBT * kBT; i += 256) {
-        const int r = i / kBT, c = i % kBT;
+      for (int i = threadIdx.x; i < BT * BT; i += 256) {
+        const int r = i / BT, c = i % BT;
         if (m0 + r < p.n && c < cols)
           p.zout[(m0 + r) * p.dim + n0 + c] = (int8_t)buf0[r * kRS + c];
       }
     }
   } else {
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int i = 0; i < WB; i++)
 #pragma unroll
-      for (int j = 0; j < 2; j++) {
+      for (int j = 0; j < WB; j++) {
         const int col = n0 + wn + 32 * j + ln;
         if (col >= p.dim) continue;
 #pragma unroll
@@ -297,6 +304,94 @@ void qjl_gemm_kernel(QjlGemmParams p) {
           if (row < p.n) p.term[row * p.dim + col] = acc[i][j][e];
         }
       }
+  }
+}
+
+// sign(S r) of a small launch: 32 vectors x 32 outputs per workgroup, K split
+// over its waves (wave w takes the runs of 64 elements w, w + waves, ...), the
+// operands straight from memory into registers.  What bounds such a launch is
+// latency: a 128 x 128 tile walks K (dim 1000) in 32 dependent steps of 0.7 us
+// whatever n is, a 64 x 64 tile in 32 of 0.45; here every load of a wave's two
+// runs is in flight at once (the products of 16 vectors 8 us, 23 and 14 in
+// tiles), and up to 16 times as many workgroups fetch.  K is
+// taken in an order of its own, the same in both operands: the 16-byte pieces
+// hh * 64 + 16 i of a run's 128-byte line feed MFMA i, so a lane pair reads
+// whole lines.
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2)))
+void qjl_signs_small_kernel(QjlGemmParams p) {
+  constexpr int kT = 32, kRow = kT + 4;
+  __shared__ __attribute__((aligned(16))) float part[WAVES][kT * kRow];
+  const int nt = (p.dim + kT - 1) / kT;
+  const int64_t m0 = (int64_t)(blockIdx.x / nt) * kT;
+  const int n0 = (int)(blockIdx.x % nt) * kT;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int hh = lane >> 5, ln = lane & 31;
+  f32x16 acc;
+#pragma unroll
+  for (int e = 0; e < 16; e++) acc[e] = 0.0f;
+#if defined(__HIP_DEVICE_COMPILE__)
+  const __amdgpu_buffer_rsrc_t rs[4] = {
+      rows_rsrc<kT>(p.xh, m0, p.n, p.ldk), rows_rsrc<kT>(p.xl, m0, p.n, p.ldk),
+      rows_rsrc<kT>(p.wh, n0, p.ldk, p.ldk), rows_rsrc<kT>(p.wl, n0, p.ldk, p.ldk)};
+  const int runs = (p.dim + 63) / 64;  // (ldk is a multiple of 64, zeros past dim)
+  for (int g = w; g < runs; g += 2 * WAVES) {
+    half8_t f[2][4][4];  // [run][operand][piece]
+#pragma unroll
+    for (int r = 0; r < 2; r++)
+#pragma unroll
+      for (int o = 0; o < 4; o++)
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          // (a second run past K: out of range, zeros)
+          f[r][o][i] = __builtin_bit_cast(
+              half8_t, __builtin_amdgcn_raw_buffer_load_b128(
+                           rs[o],
+                           g + r * WAVES < runs
+                               ? (uint32_t)(ln * p.ldk * 2 + (g + r * WAVES) * 128 + hh * 64 + i * 16)
+                               : 0x80000000u,
+                           0, 0));
+    __builtin_amdgcn_sched_barrier(0);  // all of them in flight before the first wait
+#pragma unroll
+    for (int r = 0; r < 2; r++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[r][3][i], f[r][0][i], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[r][2][i], f[r][1][i], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[r][2][i], f[r][0][i], acc, 0, 0, 0);
+      }
+  }
+#endif
+  // the waves' sums, [vector][output]
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+    *reinterpret_cast<float4*>(&part[w][ln * kRow + 8 * q + 4 * hh]) =
+        float4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+  __syncthreads();
+  for (int t = threadIdx.x; t < kT * kT / 4; t += 64 * WAVES) {
+    const int v = t / (kT / 4), c = 4 * (t % (kT / 4));
+    float4 s = *reinterpret_cast<const float4*>(&part[0][v * kRow + c]);
+#pragma unroll
+    for (int k = 1; k < WAVES; k++) {
+      const float4 a = *reinterpret_cast<const float4*>(&part[k][v * kRow + c]);
+      s.x += a.x;
+      s.y += a.y;
+      s.z += a.z;
+      s.w += a.w;
+    }
+    if (m0 + v >= p.n) continue;
+    int8_t* z = p.zout + (m0 + v) * p.dim + n0 + c;
+    // +1 for >= 0 (sign() with 0 -> +1), else -1
+    const uint32_t pk = (s.x >= 0.0f ? 0x01u : 0xffu) | (s.y >= 0.0f ? 0x0100u : 0xff00u) |
+                        (s.z >= 0.0f ? 0x010000u : 0xff0000u) |
+                        (s.w >= 0.0f ? 0x01000000u : 0xff000000u);
+    if ((p.dim & 7) == 0) {
+      if (n0 + c < p.dim) *reinterpret_cast<uint32_t*>(z) = pk;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        if (n0 + c + e < p.dim) z[e] = (int8_t)(pk >> (8 * e));
+    }
   }
 }
 
@@ -343,14 +438,38 @@ hipError_t launch_qjl(bool quant, const _Float16* xh, const _Float16* xl, const 
   p.n = n;
   p.dim = dim;
   p.ldk = ldk;
-  p.ntn = (dim + kBT - 1) / kBT;
-  p.tiles = (n + kBT - 1) / kBT * p.ntn;
+  // The form by the number of tiles.  Up to one 32 x 32 tile per CU the split-K
+  // kernel: quantize, dim 1000, n = 16 / 256 / 512 16.6 / 19.3 / 29 us against 22.8
+  // / 24 / 26.5 with 64 x 64 tiles and 31.5 / 33.2 / 34 with 128 x 128 (the whole
+  // call; the products alone 8 against 23 us at n = 16).  Then 64 x 64 tiles while
+  // few enough to fill a round or two of the card: 2.5 per CU for the quantize (n
+  // = 2500 41.3 against 43.5, n = 4096 60 against 50; dim 256, n = 8192 19.8
+  // against 22.0), 5 for the dequantize, more of which fit a CU (dim 1000, n =
+  // 2500 31.5 against 43.0, n = 4096 41.3 against 45.8; dim 256, n = 12000 20.8
+  // against 23.6; dim 1000, n = 8192 72 against 61).
+  const int64_t t32 = (n + 31) / 32 * ((dim + 31) / 32);
+  if (quant && t32 <= kCus) {
+    if (dim > 256)
+      hipLaunchKernelGGL((qjl_signs_small_kernel<8>), dim3((unsigned)t32), dim3(512), 0, st, p);
+    else
+      hipLaunchKernelGGL((qjl_signs_small_kernel<4>), dim3((unsigned)t32), dim3(256), 0, st, p);
+    return hipGetLastError();
+  }
+  const int64_t t64 = (n + 63) / 64 * ((dim + 63) / 64);
+  const int bt = t64 <= (quant ? 5 : 10) * kCus / 2 ? 64 : 128;
+  p.ntn = (dim + bt - 1) / bt;
+  p.tiles = (n + bt - 1) / bt * p.ntn;
   const int64_t grid = (p.tiles + 7) / 8 * 8;
   if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-  if (quant)
-    hipLaunchKernelGGL((qjl_gemm_kernel<true>), dim3((unsigned)grid), dim3(256), 0, st, p);
+  const dim3 g((unsigned)grid), wg(256);
+  if (quant && bt == 64)
+    hipLaunchKernelGGL((qjl_gemm_kernel<true, 64>), g, wg, 0, st, p);
+  else if (quant)
+    hipLaunchKernelGGL((qjl_gemm_kernel<true, 128>), g, wg, 0, st, p);
+  else if (bt == 64)
+    hipLaunchKernelGGL((qjl_gemm_kernel<false, 64>), g, wg, 0, st, p);
   else
-    hipLaunchKernelGGL((qjl_gemm_kernel<false>), dim3((unsigned)grid), dim3(256), 0, st, p);
+    hipLaunchKernelGGL((qjl_gemm_kernel<false, 128>), g, wg, 0, st, p);
   return hipGetLastError();
 }
 
