@@ -82,6 +82,14 @@ def test_batch_against_float64(reqs, hq, hkv, hd, dtype):
             assert bool(((got - want).abs() <= tol).all()), (got - want).abs().max().item()
 
 
+@pytest.mark.parametrize("hq,hkv", [(1, 1), (7, 7), (8, 8), (9, 3), (16, 2), (24, 8), (40, 8)])
+def test_head_orders(hq, hkv):
+    """Every head is served once whatever the head count (multiples of 8 are
+    dealt to the XCDs in runs), split keys and merges included."""
+    test_batch_against_float64([(5, 2500), (130, 0)], hq, hkv, 128, torch.float16)
+    test_batch_against_float64([(70, 20)], hq, hkv, 256, torch.bfloat16)
+
+
 @pytest.mark.parametrize("hkv,hd,dtype,aligned", [
     (8, 128, torch.bfloat16, True), (8, 128, torch.float16, False), (3, 64, torch.float32, True),
     (2, 256, torch.bfloat16, False), (2, 96, torch.float16, True), (1, 80, torch.float32, False),
