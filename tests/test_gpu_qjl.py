@@ -40,6 +40,32 @@ def test_quantize_signs_against_64_bits(dim, n):
     assert bool((proj.abs() <= bound)[wrong].all()), proj[wrong].abs().max().item()
 
 
+@pytest.mark.parametrize("dim,n", [(50, 33), (64, 1), (97, 65), (128, 31), (128, 40003)])
+def test_fused_signs_against_64_bits(dim, n):
+    """Up to padded size 128, at row scales whose residual needs other powers of
+    two (down to the clamped norm), with a zero and a NaN row."""
+    bits = 2 + dim % 4
+    print(f"case: fused qjl quantize dim={dim} n={n} bits={bits}", flush=True)
+    q, x, pd, (bnd, cen) = _prod(dim, bits, n)
+    x *= 10.0 ** torch.arange(-9, 16, 4, device="cuda").repeat(n // 7 + 1)[:n, None].float()
+    if n > 2:
+        x[1], x[2, 3] = 0.0, float("nan")
+    args = (x, pd, bits - 1, q.mse.rotation.signs, bnd, cen)
+    packed, norms, resid, rnorm = ops.prod_quantize(*args)
+    sh, sl, _, _ = q.qjl.halves(pd)
+    p2, n2, z, r2 = ops.prod_quantize_qjl(*args, sh, sl)
+    assert torch.equal(p2, packed) and torch.equal(n2.view(torch.int32), norms.view(torch.int32))
+    assert torch.equal(r2.view(torch.int32), rnorm.view(torch.int32))
+    s64, r64 = q.qjl.S.double(), resid.double()
+    proj = r64 @ s64.t()
+    wrong = z != torch.where(proj >= 0, 1, -1)  # (a NaN row: all -1)
+    # as above, and resid itself is rounded to 2^-24; below its norm's 2^-35 a
+    # component is under the quantum of a subnormal lo (2^-24 of rows near 2^10)
+    bound = ((r64.abs() @ s64.abs().t()) * (2.0 ** -20 + 3 * dim * 2.0 ** -24)
+             + s64.abs().sum(1) * 2.0 ** -35)
+    assert bool((proj.abs() <= bound)[wrong].all()), proj[wrong].abs().max().item()
+
+
 @pytest.mark.parametrize("dim,n", SHAPES)
 def test_dequantize_term_against_64_bits(dim, n):
     """z S alone: norms of zero and a weight of 1, with signs and with any

@@ -281,9 +281,12 @@ __device__ __forceinline__ int bin_code(float y, const uint2* bins, int base) {
 // With RES (TurboQuantProd's first stage, reference quantizer.py:137-143) the
 // row also reads its codes back as the dequantize kernel does (centroids,
 // the same ascending-stride FWHT, scale, sign, norm: the same fp32 bits),
-// forms the residual r = x - x_hat over the first dim dims, its norm
-// rn = max(||r||, 1e-8) (stored) and r / rn correctly rounded, left in v
-// (0 beyond dim).  Every lane of the workgroup runs this, live or not (the
+// forms the residual r = x - x_hat over the first dim dims (0 beyond dim) and
+// its norm rn = max(||r||, 1e-8) (stored).  RES 1 leaves r / rn correctly
+// rounded in v.  RES 2, for the fused QJL signs, which no positive factor
+// changes, leaves r itself and returns a power of two s with |r| s < 2^11: r s
+// is exact (the kernels of padded size 256 and up keep RES 1: RES 2 measured 3
+// to 6% slower there).  Every lane of the workgroup runs this, live or not (the
 // lane exchanges need the whole vector group); only live rows store.
 //
 // Rows of a multiple of four dims come as float4 pieces also where dim is not
@@ -368,9 +371,18 @@ __device__ __forceinline__ void load_rows_staged(const MseParams& p, int64_t row
   }
 }
 
+// r s as fp16 hi + lo (r s - hi is exact in fp32)
+__device__ __forceinline__ void residual_halves(const float* r, float s, half8_t& h, half8_t& l) {
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    h[e] = (_Float16)__builtin_fmaf(r[e], s, 0.0f);
+    l[e] = (_Float16)__builtin_fmaf(r[e], s, -(float)h[e]);
+  }
+}
+
 // v holds the row as load_row leaves it
-template <int PD, int BITS, bool RES>
-__device__ __forceinline__ void quantize_row(const MseParams& p, const float* bnd,
+template <int PD, int BITS, int RES>
+__device__ __forceinline__ float quantize_row(const MseParams& p, const float* bnd,
                                              const uint2* bins, const float* cen, int64_t row,
                                              int sub, float (&v)[MseGeom<PD>::E]) {
 #pragma clang fp contract(off)
@@ -380,6 +392,7 @@ __device__ __forceinline__ void quantize_row(const MseParams& p, const float* bn
   constexpr int NB = E / PER;                    // packed bytes per lane
   const bool live = row < p.n;
   const int d0 = sub * E;
+  float scale = 1.0f;
   float xo[RES ? E : 1];
   if constexpr (RES) {
 #pragma unroll
@@ -400,14 +413,17 @@ __device__ __forceinline__ void quantize_row(const MseParams& p, const float* bn
   // <= 1, no overflow; x = 0 gives +-0 as x / n does)
   const float yr = 1.0f / nrm;
   float sgn[E];  // the lane's signs, float4 loads (signs is 16-byte aligned)
+  auto load_signs = [&]() {
 #pragma unroll
-  for (int i = 0; i < E / 4; i++) {
-    const float4 f = reinterpret_cast<const float4*>(p.signs + d0)[i];
-    sgn[4 * i] = f.x;
-    sgn[4 * i + 1] = f.y;
-    sgn[4 * i + 2] = f.z;
-    sgn[4 * i + 3] = f.w;
-  }
+    for (int i = 0; i < E / 4; i++) {
+      const float4 f = reinterpret_cast<const float4*>(p.signs + d0)[i];
+      sgn[4 * i] = f.x;
+      sgn[4 * i + 1] = f.y;
+      sgn[4 * i + 2] = f.z;
+      sgn[4 * i + 3] = f.w;
+    }
+  };
+  load_signs();
 #pragma unroll
   for (int i = 0; i < E; i++) {
     const float q = v[i] * yr;
@@ -432,6 +448,10 @@ __device__ __forceinline__ void quantize_row(const MseParams& p, const float* bn
   else
     encode([&](float y) { return search_code<BITS>(y, bnd); });
   if constexpr (RES) {
+    if constexpr (RES == 2) {  // read again instead of held: E registers
+      asm volatile("" ::: "memory");
+      load_signs();
+    }
     fwht_contig<E, P>(v, sub);
     float rs = 0.0f;
 #pragma unroll
@@ -444,16 +464,20 @@ __device__ __forceinline__ void quantize_row(const MseParams& p, const float* bn
     for (int m = 1; m < P; m <<= 1) rs += lane_xor(rs, m);
     const float rq = sqrtf(rs);
     const float rn = rq < 1e-8f ? 1e-8f : rq;
-    const float ry = 1.0f / rn;
+    if constexpr (RES == 1) {
+      const float ry = 1.0f / rn;
 #pragma unroll
-    for (int i = 0; i < E; i++) {  // r / rn correctly rounded, as x / n above
-      const float q = v[i] * ry;
-      const float r = __builtin_fmaf(-q, rn, v[i]);
-      v[i] = __builtin_fmaf(r, ry, q);
+      for (int i = 0; i < E; i++) {  // r / rn correctly rounded, as x / n above
+        const float q = v[i] * ry;
+        const float r = __builtin_fmaf(-q, rn, v[i]);
+        v[i] = __builtin_fmaf(r, ry, q);
+      }
+    } else {  // rn >= 1e-8 has a biased exponent of 100 or more
+      scale = __uint_as_float((264u - (__float_as_uint(rn) >> 23)) << 23);
     }
     if (live && sub == 0) p.rnorm[row] = rn;
   }
-  if (!live) return;
+  if (!live) return scale;
   if (sub == 0) p.norms[row] = nrm;
   uint8_t* dst = p.packed + row * p.nbytes + sub * NB;
   if constexpr (NB == 1) {
@@ -464,6 +488,7 @@ __device__ __forceinline__ void quantize_row(const MseParams& p, const float* bn
 #pragma unroll
     for (int k = 0; k < NB / 4; k++) reinterpret_cast<uint32_t*>(dst)[k] = word[k];
   }
+  return scale;
 }
 
 // STG: rows come through the LDS stage (its own instantiation: the 32 KB of LDS
@@ -494,16 +519,11 @@ __global__ __launch_bounds__(kMseThreads) void mse_quantize_kernel(MseParams p) 
   if constexpr (RES) {
     if (row >= p.n) return;
     const int d0 = sub * E;
-    if (p.rhi) {  // (v s - hi is exact in fp32)
+    if (p.rhi) {
 #pragma unroll
       for (int c = 0; c < E / 8; c++) {
         half8_t h, l;
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-          const float r = v[8 * c + e] * kQjlScale;
-          h[e] = (_Float16)r;
-          l[e] = (_Float16)(r - (float)h[e]);
-        }
+        residual_halves(v + 8 * c, kQjlScale, h, l);
         *reinterpret_cast<half8_t*>(p.rhi + row * PD + d0 + 8 * c) = h;
         *reinterpret_cast<half8_t*>(p.rlo + row * PD + d0 + 8 * c) = l;
       }
@@ -680,8 +700,15 @@ __global__ __launch_bounds__(kMseThreads) void mse_dequantize_kernel(MseParams p
 //               from an fp32 GEMM's only where that GEMM's own rounding could
 //               flip it);
 //   dequantize: z S = z hi + z lo (z = +-1 exact in fp16).
-// Persistent workgroups: each wave loads its 16-row blocks of S (or S^T) into
-// registers once and then serves batches of 32 vectors.  C^T = S R^T per
+// Persistent workgroups: each wave loads its 16-row blocks of S (or S^T) once
+// and then serves batches of 32 vectors.  Both kernels are bound by the rows'
+// vector instructions (padded size 128: 55 per element of the quantize), so
+// what counts is waves in flight: three per SIMD at 128, for which the quantize
+// keeps S lo in LDS (32 KB, a wave reads only what it wrote), reads the signs
+// twice and takes the next rows while the products run.  150,001 x 128 at 4 bits
+// 48.7 -> 43.5 us, 200,003 x 96 60.4 -> 53.6 and, dequantize, 43.4 -> 37.6 (two
+// waves; signs converted one by one); rows off the float4 pieces want the longer
+// prefetch (100,003 x 97 41.9 -> 44.2).  C^T = S R^T per
 // batch: A = S rows (lane: row l % 16, dims 8 (l / 16) ..), B = the batch's
 // vectors from LDS (lane: vector l % 16, the same dims), D = lane: vector
 // l % 16, outputs 4 (l / 16) + e.
@@ -718,7 +745,8 @@ __device__ __forceinline__ void load_s_frags(const QjlParams& q, int w, int lane
 }
 
 template <int PD, int BITS>
-__global__ __launch_bounds__(kMseThreads) void prod_qjl_quantize_kernel(MseParams p, QjlParams q) {
+__global__ __launch_bounds__(kMseThreads) __attribute__((amdgpu_waves_per_eu(PD == 128 ? 3 : 4)))
+void prod_qjl_quantize_kernel(MseParams p, QjlParams q) {
   using MG = MseGeom<PD>;
   using QG = QjlGeom<PD>;
   constexpr int P = MG::P, E = MG::E, RS = QG::RS;
@@ -733,29 +761,31 @@ __global__ __launch_bounds__(kMseThreads) void prod_qjl_quantize_kernel(MseParam
   if (threadIdx.x >= 64 && threadIdx.x < 128)
     bins[threadIdx.x - 64] = uint2{p.bin_b[threadIdx.x - 64], p.bin_n[threadIdx.x - 64]};
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, sub = lane % P, vl = threadIdx.x / P;
-  half8_t ah[QG::NRB][QG::NKS], al[QG::NRB][QG::NKS];
-  load_s_frags<PD>(q, w, lane, ah, al);
-  float xn[E];  // the next batch's rows, loaded while this batch computes
-  load_row<PD>(p, (int64_t)blockIdx.x * 32 + vl, sub, xn);
+  // S hi in registers; S lo, each wave's own blocks as it reads them, in LDS
+  __shared__ half8_t sl[4][QG::NRB][QG::NKS][64];
+  half8_t ah[QG::NRB][QG::NKS];
+  {
+    half8_t al[QG::NRB][QG::NKS];
+    load_s_frags<PD>(q, w, lane, ah, al);
+#pragma unroll
+    for (int rb = 0; rb < QG::NRB; rb++)
+#pragma unroll
+      for (int ks = 0; ks < QG::NKS; ks++) sl[w][rb][ks][lane] = al[rb][ks];
+  }
+  float v[E];
+  load_row<PD>(p, (int64_t)blockIdx.x * 32 + vl, sub, v);
   __syncthreads();
   for (int64_t bt = blockIdx.x; bt < q.nbatch; bt += gridDim.x) {
-    float v[E];
-#pragma unroll
-    for (int i = 0; i < E; i++) v[i] = xn[i];
-    if (bt + gridDim.x < q.nbatch) load_row<PD>(p, (bt + gridDim.x) * 32 + vl, sub, xn);
-    quantize_row<PD, BITS, true>(p, bnd, bins, cen, bt * 32 + vl, sub, v);
-    // the unit residual as fp16 hi + lo (v - hi is exact in fp32)
+    const float s = quantize_row<PD, BITS, 2>(p, bnd, bins, cen, bt * 32 + vl, sub, v);
 #pragma unroll
     for (int c = 0; c < E / 8; c++) {
       half8_t h, l;
-#pragma unroll
-      for (int e = 0; e < 8; e++) {
-        h[e] = (_Float16)v[8 * c + e];
-        l[e] = (_Float16)(v[8 * c + e] - (float)h[e]);
-      }
+      residual_halves(v + 8 * c, s, h, l);
       *reinterpret_cast<half8_t*>(rh + vl * RS + sub * E + 8 * c) = h;
       *reinterpret_cast<half8_t*>(rl + vl * RS + sub * E + 8 * c) = l;
     }
+    // the next batch's rows come in during the products
+    if (bt + gridDim.x < q.nbatch) load_row<PD>(p, (bt + gridDim.x) * 32 + vl, sub, v);
     __syncthreads();
 #pragma unroll
     for (int cb = 0; cb < 2; cb++) {
@@ -771,7 +801,7 @@ __global__ __launch_bounds__(kMseThreads) void prod_qjl_quantize_kernel(MseParam
         for (int rb = 0; rb < QG::NRB; rb++) {
           acc[rb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[rb][ks], bh, acc[rb], 0, 0, 0);
           acc[rb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[rb][ks], bl, acc[rb], 0, 0, 0);
-          acc[rb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[rb][ks], bh, acc[rb], 0, 0, 0);
+          acc[rb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(sl[w][rb][ks][lane], bh, acc[rb], 0, 0, 0);
         }
       }
       const int64_t vec = bt * 32 + 16 * cb + (lane & 15);
@@ -799,7 +829,8 @@ __global__ __launch_bounds__(kMseThreads) void prod_qjl_quantize_kernel(MseParam
 }
 
 template <int PD, int BITS>
-__global__ __launch_bounds__(kMseThreads) void prod_qjl_dequantize_kernel(MseParams p,
+__global__ __launch_bounds__(kMseThreads) __attribute__((amdgpu_waves_per_eu(PD == 128 ? 3 : 4)))
+void prod_qjl_dequantize_kernel(MseParams p,
                                                                           QjlParams q) {
   using MG = MseGeom<PD>;
   using QG = QjlGeom<PD>;
@@ -859,10 +890,10 @@ __global__ __launch_bounds__(kMseThreads) void prod_qjl_dequantize_kernel(MsePar
       for (int rb = 0; rb < QG::NRB; rb++) acc[rb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int ks = 0; ks < QG::NKS; ks++) {
-        half8_t b;
-#pragma unroll
-        for (int e = 0; e < 8; e++)
-          b[e] = (_Float16)(int8_t)((e < 4 ? zc[cb][ks].x : zc[cb][ks].y) >> (8 * (e & 3)));
+        uint4 zh;
+        z_to_half(zc[cb][ks].x, zh.x, zh.y);
+        z_to_half(zc[cb][ks].y, zh.z, zh.w);
+        const half8_t b = __builtin_bit_cast(half8_t, zh);
 #pragma unroll
         for (int rb = 0; rb < QG::NRB; rb++) {
           acc[rb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[rb][ks], b, acc[rb], 0, 0, 0);
@@ -914,7 +945,7 @@ hipError_t launch_mse(bool quant, int bits, const MseParams& p, hipStream_t st) 
   const bool staged = PD >= 256 && p.dim != PD && (p.dim & 3) == 0;
 #define TQ_MSE_CASE(B)                                                                   \
   case B:                                                                                \
-    if (quant && p.rnorm)                                                                \
+    if (quant && p.rnorm)                                                           \
       hipLaunchKernelGGL((mse_quantize_kernel<PD, B, true>), grid, block, 0, st, p);     \
     else if (quant && staged)                                                            \
       hipLaunchKernelGGL((mse_quantize_kernel<PD, B, false, (PD >= 256)>), grid, block, 0, st, \

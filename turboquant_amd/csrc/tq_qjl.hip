@@ -38,7 +38,6 @@ namespace tq {
 namespace {
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -77,16 +76,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const _Float16* base
                                            nrec, 0x00020000);
 }
 #endif
-
-// four int8 as fp16 (exact: 1024 + (z + 128) - 1152)
-__device__ __forceinline__ void z_to_half(uint32_t w, uint32_t& lo, uint32_t& hi) {
-  const uint32_t u = w ^ 0x80808080u;
-  const half2_t b = {(_Float16)1152.0f, (_Float16)1152.0f};
-  lo = __builtin_bit_cast(uint32_t, (half2_t)(__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(
-                                        0x64646464u, u, 0x04010400u)) - b));
-  hi = __builtin_bit_cast(uint32_t, (half2_t)(__builtin_bit_cast(half2_t, __builtin_amdgcn_perm(
-                                        0x64646464u, u, 0x04030402u)) - b));
-}
 
 // BT: the tile's edge, 128 or 64 (vectors, outputs).
 template <bool QUANT, int BT>
