@@ -64,6 +64,7 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef short v4i16 __attribute__((ext_vector_type(4)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
@@ -117,7 +118,7 @@ struct PrefillBatch {
   int ratio, hd;      // hd <= kD: dims of q and o rows (zero padded to kD here)
   int q_bf16, o_bf16;  // q / o element type (else fp16)
   float c;             // sm_scale * log2(e)
-  _Float16* ws_o;      // [slot][kBM 128][Hq][kD]
+  float* ws_o;         // [slot][kBM 128][Hq][kD]
   float* ws_ml;        // [slot][128][Hq][2]
   PrefillReq reqs[kBatchReqs];
   PrefillItem items[kBatchItems];
@@ -487,21 +488,33 @@ void prefill_kernel(PP p) {
   lsum = sum32(lsum);
   const float inv = lsum > 0.0f ? 1.0f / lsum : 0.0f;
   if (SPLIT || (kBatch && wk.slot >= 0)) {
-    // this split's O / row sum (a convex combination of V rows: fp16 is
-    // safe) and (mc, row sum); a split that held no visible key for a row
-    // leaves mc = -inf, sum 0, O = 0
+    // this split's O / row sum and (mc, row sum); a split that held no visible
+    // key for a row leaves mc = -inf, sum 0, O = 0.  One request: as fp16 (a
+    // convex combination of V rows: safe).  Batch mode splits blocks that one
+    // launch per request left whole, so what was a sum in fp32 stays one: fp32.
     if (qrow < wk.lq) {
       const int64_t r = (kBatch ? (int64_t)wk.slot * kBM + 32 * w + n
                                 : (int64_t)blockIdx.z * wk.lq + qrow) * gridDim.x + head;
-      _Float16* const wo = p.ws_o + r * kD + 4 * hh;
+      if constexpr (kBatch) {
+        float* const wo = p.ws_o + r * kD + 4 * hh;
 #pragma unroll
-      for (int d = 0; d < kD / 32; d++)
+        for (int d = 0; d < kD / 32; d++)
 #pragma unroll
-        for (int jq = 0; jq < 4; jq++) {
-          const uint32_t lo = pack_h2(oacc[d][4 * jq] * inv, oacc[d][4 * jq + 1] * inv);
-          const uint32_t hi = pack_h2(oacc[d][4 * jq + 2] * inv, oacc[d][4 * jq + 3] * inv);
-          *reinterpret_cast<u32x2*>(wo + 32 * d + 8 * jq) = u32x2{lo, hi};
-        }
+          for (int jq = 0; jq < 4; jq++)
+            *reinterpret_cast<f32x4*>(wo + 32 * d + 8 * jq) =
+                f32x4{oacc[d][4 * jq] * inv, oacc[d][4 * jq + 1] * inv, oacc[d][4 * jq + 2] * inv,
+                      oacc[d][4 * jq + 3] * inv};
+      } else {
+        _Float16* const wo = p.ws_o + r * kD + 4 * hh;
+#pragma unroll
+        for (int d = 0; d < kD / 32; d++)
+#pragma unroll
+          for (int jq = 0; jq < 4; jq++) {
+            const uint32_t lo = pack_h2(oacc[d][4 * jq] * inv, oacc[d][4 * jq + 1] * inv);
+            const uint32_t hi = pack_h2(oacc[d][4 * jq + 2] * inv, oacc[d][4 * jq + 3] * inv);
+            *reinterpret_cast<u32x2*>(wo + 32 * d + 8 * jq) = u32x2{lo, hi};
+          }
+      }
       if (hh == 0) *reinterpret_cast<f32x2*>(p.ws_ml + 2 * r) = f32x2{mc, lsum};
     }
     return;
@@ -818,7 +831,7 @@ struct PrefillMerge {
   void* o;
   int64_t o_st, o_sh;
   int hq, hd, o_bf16;
-  const _Float16* ws_o;
+  const float* ws_o;
   const float* ws_ml;
   PrefillGroup groups[kBatchItems];
 };
@@ -841,12 +854,13 @@ __global__ __launch_bounds__(256) void prefill_batch_merge_kernel(PrefillMerge p
 #pragma unroll 4
   for (int z = 0; z < g.nsplit; z++) {
     const f32x2 ml = *reinterpret_cast<const f32x2*>(p.ws_ml + 2 * (v0 + z * zs));
-    const half8_t x = *reinterpret_cast<const half8_t*>(p.ws_o + (v0 + z * zs) * kD + c);
+    const f32x4* const x = reinterpret_cast<const f32x4*>(p.ws_o + (v0 + z * zs) * kD + c);
+    const f32x4 x0 = x[0], x1 = x[1];
     // a split without a visible key for the row has weight 0 (its O is 0)
     const float wgt = ml[0] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml[0] - mx) * ml[1];
     den += wgt;
 #pragma unroll
-    for (int i = 0; i < 8; i++) acc[i] = __builtin_fmaf(wgt, (float)x[i], acc[i]);
+    for (int i = 0; i < 8; i++) acc[i] = __builtin_fmaf(wgt, i < 4 ? x0[i] : x1[i - 4], acc[i]);
   }
   if (c >= p.hd) return;
   const float inv = den > 0.0f ? 1.0f / den : 0.0f;
@@ -1115,7 +1129,7 @@ hipError_t launch_batch(const BatchPlan& bp, int heads, hipStream_t st, PrefillB
 
 // workspace of a plan: O rows, then (max, sum) pairs, of each slot's 128 rows
 int64_t batch_ws_bytes(const BatchPlan& bp, int heads, int head_dim) {
-  return (int64_t)bp.slots * 128 * heads * (head_dim * 2 + 8);
+  return (int64_t)bp.slots * 128 * heads * (head_dim * 4 + 8);
 }
 
 bool batch_sizes_ok(const int32_t* q_lens, const int32_t* kv_lens, int32_t nreq, int32_t heads,
@@ -1252,9 +1266,8 @@ extern "C" int tq_prefill_attention_batch(
         set_error("%s: workspace smaller than tq_prefill_batch_workspace_bytes", what);
         return kEinval;
       }
-      p.ws_o = static_cast<_Float16*>(workspace);
-      p.ws_ml = reinterpret_cast<float*>(p.ws_o + (int64_t)bp.slots * 128 * num_qo_heads *
-                                                      padded_dim);
+      p.ws_o = static_cast<float*>(workspace);
+      p.ws_ml = p.ws_o + (int64_t)bp.slots * 128 * num_qo_heads * padded_dim;
       for (int i = 0; i < n; i++)
         p.reqs[i] = {q_starts[a + i], q_lens[a + i], kv_starts[a + i], kv_lens[a + i],
                      kv_sources[a + i] ? 1 : 0};
