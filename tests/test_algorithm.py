@@ -106,6 +106,19 @@ def test_qjl_unbiased():
     assert abs(np.mean(est) - float(x @ y)) < 0.15
 
 
+@pytest.mark.parametrize("inference,change", [
+    (False, lambda s: s.neg_()), (False, lambda s: s.data.neg_()), (True, lambda s: s.neg_())])
+def test_qjl_halves_follow_writes_to_the_matrix(inference, change):
+    """The operand halves are those of S as it is now, however it was written."""
+    with torch.inference_mode(inference):
+        q = A.QJL(200, device="cpu", seed=3)
+    before = [h.clone() for h in q.halves(256)]
+    with torch.inference_mode(inference):
+        change(q.S)
+    for now, was in zip(q.halves(256), before):
+        assert torch.equal(now, -was)
+
+
 @pytest.mark.parametrize("bits,expected", [(1, 0.36), (2, 0.117), (3, 0.03), (4, 0.009)])
 def test_mse_distortion(bits, expected):
     q = A.TurboQuantMSE(128, bits, device=DEV, seed=42)

@@ -149,6 +149,33 @@ def test_first_call_inside_a_graph():
         assert torch.equal(z, eager)
 
 
+@pytest.mark.parametrize("dim", [100, 400])
+def test_matrix_written_between_calls_captures_and_replays(dim):
+    """A write that torch does not count, a capture right after it, and a
+    graph whose matrix changes before its replays: always today's S."""
+    q, x, _, _ = _prod(dim, 4, 2100)
+    first = [t.clone() for t in q.quantize(x)]
+    xh = q.dequantize(*first)
+    q.qjl.S.data.neg_()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        z = q.quantize(x)[2]
+        back = q.dequantize(*first)
+    want = -first[2]
+    mse = q.mse.dequantize(first[0], first[1])
+    for _ in range(4):
+        z.zero_(), back.zero_()
+        g.replay()
+        assert torch.equal(q.quantize(x)[2], want)
+        torch.cuda.synchronize()
+        assert torch.equal(z, want)
+        # x_mse -+ term, the term's magnitude within a rounding of each sum
+        got = (back - mse) * (1 if torch.equal(want, first[2]) else -1)
+        assert torch.allclose(got, xh - mse, rtol=1e-5, atol=2.0 ** -22 * xh.abs().max().item())
+        q.qjl.S.data.neg_()
+        want = -want
+
+
 @pytest.mark.parametrize("dim", [50, 64, 97, 128, 257, 1000])
 def test_operand_halves(dim):
     q = A.QJL(dim, device="cuda:0", seed=3)

@@ -176,39 +176,23 @@ class QJL:
 
     def halves(self, padded_dim: int):
         """(S_hi, S_lo, S^T_hi, S^T_lo): fp16 halves with S = hi + lo (to 22
-        bits), zero-padded to [padded_dim, padded_dim], for the fused kernels
-        (made once per padded size and device; again when S was replaced or
-        written to)."""
-        made_from = (self.S, None if self.S.is_inference() else self.S._version)
-        kept_of = self.__dict__.get("_halves_of", (None, None))
-        cache = self.__dict__.get("_halves", {})
-        key = (padded_dim, str(self.S.device))
-        if kept_of[0] is not made_from[0] or kept_of[1] != made_from[1]:
-            if cache and self.S.is_cuda:
-                torch.cuda.synchronize(self.S.device)  # kernels on any stream that read the old ones
-            cache = {}
-        if key in cache:
-            return cache[key]
+        bits), zero-padded to [padded_dim, padded_dim], for the fused kernels.
+        Made on every call (a kernel of a few us on a GPU): a write to S can
+        go unseen (through .data, in inference mode, in a replayed graph), so
+        nothing made from an earlier S is kept."""
         if self.S.is_cuda and self.S.dtype == torch.float32:
             from . import ops
-            out = ops.qjl_halves(self.S, padded_dim)
-        else:
-            out = []
-            for m in (self.S, self.S.t()):
-                hi = m.half()
-                lo = (m - hi.float()).half()
-                for h in (hi, lo):
-                    pad = torch.zeros((padded_dim, padded_dim), dtype=torch.float16,
-                                      device=self.S.device)
-                    pad[:self.dim, :self.dim] = h
-                    out.append(pad)
-        if self.S.is_cuda:
-            if torch.cuda.is_current_stream_capturing():
-                return tuple(out)  # they hold values only once the graph runs: not kept
-            # later calls may come from other streams
-            torch.cuda.current_stream(self.S.device).synchronize()
-        self._halves, self._halves_of = {**cache, key: tuple(out)}, made_from
-        return self._halves[key]
+            return ops.qjl_halves(self.S, padded_dim)
+        out = []
+        for m in (self.S, self.S.t()):
+            hi = m.half()
+            lo = (m - hi.float()).half()
+            for h in (hi, lo):
+                pad = torch.zeros((padded_dim, padded_dim), dtype=torch.float16,
+                                  device=self.S.device)
+                pad[:self.dim, :self.dim] = h
+                out.append(pad)
+        return tuple(out)
 
     @torch.no_grad()
     def quantize(self, x: torch.Tensor) -> torch.Tensor:

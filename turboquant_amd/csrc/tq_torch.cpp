@@ -339,6 +339,21 @@ bool halves(const Tensor& t, int64_t padded_dim, c10::Device dev) {
          t.size(1) == padded_dim && t.is_contiguous() && aligned(t, 16);
 }
 
+// ops.qjl_halves
+std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> qjl_halves(const Tensor& s,
+                                                                     int64_t padded_dim) {
+  const c10::Device dev = s.device();
+  if (!is_f32(s, dev) || s.dim() != 2 || s.size(0) != s.size(1) || s.size(0) < 1 ||
+      s.size(0) > padded_dim || padded_dim > 1024)
+    return std::nullopt;
+  const c10::DeviceGuard guard(dev);
+  const Tensor out = at::empty({4, padded_dim, padded_dim}, s.options().dtype(at::kHalf));
+  if (!on(out, dev) || tq_qjl_halves(cptr<float>(s), s.size(0), padded_dim, out.data_ptr(),
+                                     stream_of(dev)) != 0)
+    return std::nullopt;
+  return std::make_tuple(out.select(0, 0), out.select(0, 1), out.select(0, 2), out.select(0, 3));
+}
+
 // ops.prod_quantize_qjl (large: prod_quantize_qjl_ws)
 ProdCodes prod_quantize_qjl(const Tensor& x, int64_t padded_dim, int64_t bits, const Tensor& signs,
                             const std::vector<double>& boundaries,
@@ -452,6 +467,7 @@ PYBIND11_MODULE(_tq_torch, m) {
   m.def("prefill_gather", &prefill_gather, unlocked);
   m.def("mse_quantize", &mse_quantize, unlocked);
   m.def("mse_dequantize", &mse_dequantize, unlocked);
+  m.def("qjl_halves", &qjl_halves, unlocked);
   m.def("prod_quantize_qjl", &prod_quantize_qjl, unlocked);
   m.def("prod_dequantize_qjl", &prod_dequantize_qjl, unlocked);
 }

@@ -509,6 +509,9 @@ def _aligned16(t: torch.Tensor) -> torch.Tensor:
 def qjl_halves(s: torch.Tensor, padded_dim: int):
     """(S hi, S lo, S^T hi, S^T lo): fp16 halves of the QJL matrix s fp32
     [dim, dim], zero-padded to [padded_dim, padded_dim] (tq_qjl_halves)."""
+    r = (_nat or _native()).qjl_halves(s, padded_dim)
+    if r is not None:
+        return r
     _require_gpu(s)
     if s.dtype != torch.float32 or s.dim() != 2 or s.size(0) != s.size(1):
         raise RuntimeError("qjl_halves: S must be a square fp32 matrix")
