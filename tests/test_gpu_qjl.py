@@ -149,6 +149,27 @@ def test_first_call_inside_a_graph():
         assert torch.equal(z, eager)
 
 
+def test_what_the_product_with_s_refuses_is_refused():
+    """Vectors of another length in the same padded size, and a matrix of
+    another shape or type, as the torch product with S refuses them."""
+    q, x, _, _ = _prod(400, 4, 2100)
+    out = q.quantize(x)
+    for other in (300, 399, 500):
+        with pytest.raises(RuntimeError):
+            q.quantize(torch.randn((4, other), device="cuda"))
+    s = q.qjl.S
+    for bad in (s.double(), s.half(), s[:300, :300], s[:, :300], s.cpu()):
+        q.qjl.S = bad
+        with pytest.raises(RuntimeError):
+            q.quantize(x)
+        with pytest.raises(RuntimeError):
+            q.dequantize(*out)
+    small = A.TurboQuantProd(100, 3, device="cuda:0")
+    small.qjl.S = small.qjl.S[:90, :90].contiguous()
+    with pytest.raises(RuntimeError):
+        small.quantize(torch.randn((4, 100), device="cuda"))
+
+
 @pytest.mark.parametrize("dim", [100, 400])
 def test_matrix_written_between_calls_captures_and_replays(dim):
     """A write that torch does not count, a capture right after it, and a

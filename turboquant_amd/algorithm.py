@@ -180,6 +180,9 @@ class QJL:
         Made on every call (a kernel of a few us on a GPU): a write to S can
         go unseen (through .data, in inference mode, in a replayed graph), so
         nothing made from an earlier S is kept."""
+        if tuple(self.S.shape) != (self.dim, self.dim):
+            raise RuntimeError(f"QJL: S must be [{self.dim}, {self.dim}], got "
+                               f"{tuple(self.S.shape)}")
         if self.S.is_cuda and self.S.dtype == torch.float32:
             from . import ops
             return ops.qjl_halves(self.S, padded_dim)
@@ -265,6 +268,14 @@ class TurboQuantProd:
         self.mse = TurboQuantMSE(dim, bit_width - 1, device=device, seed=seed)
         self.qjl = QJL(dim, device=device, seed=seed + 10000)
 
+    def _large_halves(self, dim: int, padded_dim: int):
+        """The operand halves above padded size 128, for vectors of `dim`: what
+        the fp32 product with S refuses is refused."""
+        if dim != self.qjl.dim or self.qjl.S.dtype != torch.float32:
+            raise RuntimeError(f"TurboQuantProd: vectors of {dim} dims do not go with a QJL "
+                               f"matrix {self.qjl.S.dtype} [{self.qjl.dim}, {self.qjl.dim}]")
+        return self.qjl.halves(padded_dim)
+
     @torch.no_grad()
     def quantize(self, x: torch.Tensor):
         """-> (mse_packed, mse_norms, qjl_signs int8 {-1, +1}, residual_norms).
@@ -281,7 +292,7 @@ class TurboQuantProd:
                 sh, sl, _, _ = self.qjl.halves(pd)
                 return ops.prod_quantize_qjl(x, pd, self.mse.bit_width, self.mse.rotation.signs,
                                              bnd, cen, sh, sl)
-            sh, sl, _, _ = self.qjl.halves(pd)
+            sh, sl, _, _ = self._large_halves(x.shape[-1], pd)
             return ops.prod_quantize_qjl_ws(x, pd, self.mse.bit_width, self.mse.rotation.signs,
                                             bnd, cen, sh, sl)
         packed, norms = self.mse.quantize(x)
@@ -301,7 +312,7 @@ class TurboQuantProd:
                                                self.mse.rotation.signs,
                                                self.mse._host_tables()[1], th, tl)
             if qjl_signs.dtype == torch.int8 and mse_norms.numel() >= QJL_GEMM_MIN:
-                _, _, th, tl = self.qjl.halves(pd)
+                _, _, th, tl = self._large_halves(self.dim, pd)
                 return ops.prod_dequantize_qjl_ws(mse_packed, mse_norms, qjl_signs,
                                                   residual_norms, self.dim, pd,
                                                   self.mse.bit_width, self.mse.rotation.signs,
