@@ -26,6 +26,8 @@
 extern "C" {
 #endif
 
+#define TQ_ABI_VERSION 11 /* what tq_abi_version() returns */
+
 typedef struct ihipStream_t* tq_stream_t; /* == hipStream_t */
 
 enum tq_dtype { TQ_F32 = 0, TQ_F16 = 1, TQ_BF16 = 2 };
@@ -404,7 +406,7 @@ int tq_prod_dequantize_qjl(const uint8_t* packed, const float* norms, const int8
                            float* out, tq_stream_t stream);
 
 /*
- * The operand halves of the calls around it from the QJL matrix S fp32
+ * The operand halves of the calls above from the QJL matrix S fp32
  * [dim, dim]: `halves` receives fp16 [4][padded_dim][padded_dim], S hi, S lo,
  * S^T hi, S^T lo (hi + lo = S to 22 bits), zero past dim.  padded_dim a power
  * of two 64..1024.
@@ -415,11 +417,20 @@ int tq_qjl_halves(const float* s, int32_t dim, int32_t padded_dim, void* halves,
 /*
  * The same above padded_dim 128 (256, 512 or 1024), where S no longer fits a
  * wave's registers: the row kernels of tq_prod_quantize / tq_prod_dequantize
- * and the QJL product as a matrix-core kernel of its own.  Operands as above
- * (halves [padded_dim, padded_dim]).  tq_prod_quantize_qjl_ws keeps the unit
- * residual in `workspace` (16-byte aligned, tq_prod_workspace_bytes bytes) as
- * fp16 halves; tq_prod_dequantize_qjl_ws forms z S in the rows of `out`.
+ * and the QJL product as a matrix-core kernel of its own.  tq_qjl_operand
+ * makes its operand from S fp32 [dim, dim]: `halves` receives fp16
+ * [2][padded_dim][padded_dim], hi and lo of S (transposed 0: for the quantize)
+ * or S^T (else: for the dequantize), zero past dim, each row times a power of
+ * two that takes its largest entry to [2^14, 2^15), and `scales` fp32
+ * [padded_dim] the inverses of those powers.  A quantize takes halves of any
+ * positive row scale; the dequantize multiplies output column j by st_scale[j]
+ * (null: unscaled halves, as tq_qjl_halves makes them).
+ * tq_prod_quantize_qjl_ws keeps the unit residual in `workspace` (16-byte
+ * aligned, tq_prod_workspace_bytes bytes) as fp16 halves;
+ * tq_prod_dequantize_qjl_ws forms z S in the rows of `out`.
  */
+int tq_qjl_operand(const float* s, int32_t dim, int32_t padded_dim, int32_t transposed,
+                   void* halves, float* scales, tq_stream_t stream);
 int64_t tq_prod_workspace_bytes(int64_t num_vectors, int32_t padded_dim);
 int tq_prod_quantize_qjl_ws(const float* x, int64_t num_vectors, int32_t dim, int32_t padded_dim,
                             int32_t mse_bit_width, const float* signs, const float* boundaries,
@@ -431,7 +442,7 @@ int tq_prod_dequantize_qjl_ws(const uint8_t* packed, const float* norms, const i
                               const float* residual_norms, int64_t num_vectors, int32_t dim,
                               int32_t padded_dim, int32_t mse_bit_width, const float* signs,
                               const float* centroids, const void* st_hi, const void* st_lo,
-                              float* out, tq_stream_t stream);
+                              const float* st_scale, float* out, tq_stream_t stream);
 
 /*
  * Layer glue of the end-to-end harness, no counterpart in the

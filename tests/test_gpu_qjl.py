@@ -197,6 +197,46 @@ def test_matrix_written_between_calls_captures_and_replays(dim):
         want = -want
 
 
+@pytest.mark.parametrize("dim", [129, 256, 300, 512, 1000, 1023, 1024])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_scaled_operand(dim, transposed):
+    """hi + lo over the row's power of two is S: to half an ulp of a 22-bit
+    number, or, where lo is subnormal, half its quantum 2^-24 (rows reach 2^14
+    at least).  Rows of any magnitude, an empty and an infinite one."""
+    s = torch.randn((dim, dim), generator=torch.Generator("cuda").manual_seed(dim), device="cuda")
+    s *= 10.0 ** torch.linspace(-33, 37, dim, device="cuda")[:, None]
+    s[3] = 0.0
+    s[5, 7] = float("inf")
+    if transposed:
+        s = s.t().contiguous()
+    pd = A.next_power_of_2(dim)
+    hi, lo, scale = ops.qjl_operand(s, pd, transposed)
+    rows = s.double() if not transposed else s.double().t()
+    got = (hi.double() + lo.double()) * scale.double()[:, None]
+    assert (got[dim:] == 0).all() and (got[:, dim:] == 0).all() and (got[3] == 0).all()
+    got, top = got[:dim, :dim], rows.abs().amax(1)
+    fine = torch.isfinite(top)
+    assert not fine[5] and got[5, 7] == float("inf") and torch.isfinite(got[5, :7]).all()
+    bound = rows.abs() * 2.0 ** -22 + (top * 2.0 ** -38)[:, None]
+    assert ((got - rows).abs() <= bound)[fine].all()
+    keep = fine & (top > 0)
+    big = hi[:dim].abs().amax(1).double()[keep]
+    assert (big >= 2.0 ** 14).all() and (big <= 2.0 ** 15).all()
+
+
+@pytest.mark.parametrize("k", [-100, -20, 20, 100])
+def test_matrix_of_another_magnitude(k):
+    """S over fp32's range: signs do not change with a power of two on S, the
+    read-back term changes by it exactly."""
+    q, x, pd, (_, cen) = _prod(700, 4, 2300)
+    packed, norms, z, rn = q.quantize(x)
+    zero, one = torch.zeros_like(norms), torch.ones_like(rn)
+    term = q.dequantize(packed, zero, z, one)
+    q.qjl.S *= 2.0 ** k
+    assert torch.equal(q.quantize(x)[2], z)
+    assert torch.equal(q.dequantize(packed, zero, z, one), term * 2.0 ** k)
+
+
 @pytest.mark.parametrize("dim", [50, 64, 97, 128, 257, 1000])
 def test_operand_halves(dim):
     q = A.QJL(dim, device="cuda:0", seed=3)

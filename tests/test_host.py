@@ -159,6 +159,11 @@ def test_cabi_argument_errors_without_gpu():
     assert rc == -22 and b"head_dim" in lib.tq_last_error()
     # an empty batch is a no-op that succeeds
     assert lib.tq_combine_splits(null, null, 0, 1, 32, 128, null, null, null) == 0
+    # the QJL operand: padded sizes above 128, dim at most that, no null pointers
+    one = ctypes.c_void_p(256)
+    for args in ((one, 100, 128, 0, one, one), (one, 257, 256, 1, one, one),
+                 (null, 200, 256, 0, one, one), (one, 200, 256, 1, one, null)):
+        assert lib.tq_qjl_operand(*args, null) == -22
     # the stream-read diagnostic: null source, size not a multiple of 16
     assert lib.tq_diag_stream_read(null, 16, null, null) == -22
     assert lib.tq_diag_stream_read(ctypes.c_void_p(256), 24, ctypes.c_void_p(256), null) == -22

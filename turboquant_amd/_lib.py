@@ -69,11 +69,12 @@ SIGNATURES = {
     "tq_prod_dequantize_qjl": (_I32, [_P, _P, _P, _P, _I64, _I32, _I32, _I32, _P, _P, _P, _P,
                                       _P, _P]),
     "tq_qjl_halves": (_I32, [_P, _I32, _I32, _P, _P]),
+    "tq_qjl_operand": (_I32, [_P, _I32, _I32, _I32, _P, _P, _P]),
     "tq_prod_workspace_bytes": (_I64, [_I64, _I32]),
     "tq_prod_quantize_qjl_ws": (_I32, [_P, _I64, _I32, _I32, _I32, _P, _P, _P, _P, _P, _P, _P,
                                        _P, _P, _P, _I64, _P]),
     "tq_prod_dequantize_qjl_ws": (_I32, [_P, _P, _P, _P, _I64, _I32, _I32, _I32, _P, _P, _P,
-                                         _P, _P, _P]),
+                                         _P, _P, _P, _P]),
     "tq_diag_mse_bucketize": (_I32, [_I32]),
     "tq_e2e_add_rms_norm": (_I32, [_P, _P, _P, _P, _I64, _I32, _F32, _P]),
     "tq_e2e_qk_norm_rope": (_I32, [_P, _I64, _P, _P, _P, _P, _I64, _P, _I64, _I32, _I32, _I32,
@@ -82,7 +83,7 @@ SIGNATURES = {
     "tq_last_error": (ctypes.c_char_p, []),
     "tq_abi_version": (_I32, []),
 }
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 _lib = None
 

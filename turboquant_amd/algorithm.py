@@ -268,13 +268,16 @@ class TurboQuantProd:
         self.mse = TurboQuantMSE(dim, bit_width - 1, device=device, seed=seed)
         self.qjl = QJL(dim, device=device, seed=seed + 10000)
 
-    def _large_halves(self, dim: int, padded_dim: int):
-        """The operand halves above padded size 128, for vectors of `dim`: what
-        the fp32 product with S refuses is refused."""
-        if dim != self.qjl.dim or self.qjl.S.dtype != torch.float32:
+    def _qjl_operand(self, dim: int, transposed: bool):
+        """(hi, lo, scale) of S or S^T above padded size 128, for vectors of
+        `dim`: what the fp32 product with S refuses is refused.  Made from S
+        on every call, as QJL.halves."""
+        from . import ops
+        s = self.qjl.S
+        if tuple(s.shape) != (dim, dim) or s.dtype != torch.float32:
             raise RuntimeError(f"TurboQuantProd: vectors of {dim} dims do not go with a QJL "
-                               f"matrix {self.qjl.S.dtype} [{self.qjl.dim}, {self.qjl.dim}]")
-        return self.qjl.halves(padded_dim)
+                               f"matrix {s.dtype} {tuple(s.shape)}")
+        return ops.qjl_operand(s, self.mse.rotation.padded_dim, transposed)
 
     @torch.no_grad()
     def quantize(self, x: torch.Tensor):
@@ -292,7 +295,7 @@ class TurboQuantProd:
                 sh, sl, _, _ = self.qjl.halves(pd)
                 return ops.prod_quantize_qjl(x, pd, self.mse.bit_width, self.mse.rotation.signs,
                                              bnd, cen, sh, sl)
-            sh, sl, _, _ = self._large_halves(x.shape[-1], pd)
+            sh, sl, _ = self._qjl_operand(x.shape[-1], False)
             return ops.prod_quantize_qjl_ws(x, pd, self.mse.bit_width, self.mse.rotation.signs,
                                             bnd, cen, sh, sl)
         packed, norms = self.mse.quantize(x)
@@ -312,11 +315,11 @@ class TurboQuantProd:
                                                self.mse.rotation.signs,
                                                self.mse._host_tables()[1], th, tl)
             if qjl_signs.dtype == torch.int8 and mse_norms.numel() >= QJL_GEMM_MIN:
-                _, _, th, tl = self._large_halves(self.dim, pd)
+                th, tl, scale = self._qjl_operand(self.dim, True)
                 return ops.prod_dequantize_qjl_ws(mse_packed, mse_norms, qjl_signs,
                                                   residual_norms, self.dim, pd,
                                                   self.mse.bit_width, self.mse.rotation.signs,
-                                                  self.mse._host_tables()[1], th, tl)
+                                                  self.mse._host_tables()[1], th, tl, scale)
             return ops.prod_dequantize(mse_packed, mse_norms, qjl_signs.float() @ self.qjl.S,
                                        residual_norms, self.dim, self.mse.rotation.padded_dim,
                                        self.mse.bit_width, self.mse.rotation.signs,

@@ -1371,7 +1371,7 @@ extern "C" int tq_prod_quantize_qjl_ws(const float* x, int64_t num_vectors, int3
   if (rc) return rc;
   const hipError_t e = tq::launch_qjl(
       true, pa.rhi, pa.rlo, nullptr, static_cast<const _Float16*>(s_hi),
-      static_cast<const _Float16*>(s_lo), qjl_signs, nullptr, num_vectors, dim, padded_dim,
+      static_cast<const _Float16*>(s_lo), nullptr, qjl_signs, nullptr, num_vectors, dim, padded_dim,
       reinterpret_cast<hipStream_t>(stream));
   if (e != hipSuccess) tq::set_error("%s: launch failed: %s", what, hipGetErrorString(e));
   return (int)e;
@@ -1382,7 +1382,8 @@ extern "C" int tq_prod_dequantize_qjl_ws(const uint8_t* packed, const float* nor
                                          int64_t num_vectors, int32_t dim, int32_t padded_dim,
                                          int32_t mse_bit_width, const float* signs,
                                          const float* centroids, const void* st_hi,
-                                         const void* st_lo, float* out, tq_stream_t stream) {
+                                         const void* st_lo, const float* st_scale, float* out,
+                                         tq_stream_t stream) {
   const char* what = "prod_dequantize_qjl_ws";
   int rc = tq::qjl_ws_check(what, padded_dim, st_hi, st_lo, qjl_signs, num_vectors, dim);
   if (rc || num_vectors == 0) return rc;
@@ -1401,7 +1402,7 @@ extern "C" int tq_prod_dequantize_qjl_ws(const uint8_t* packed, const float* nor
   // z S goes into the output rows, which the dequantize then completes in place
   const hipError_t e = tq::launch_qjl(
       false, nullptr, nullptr, qjl_signs, static_cast<const _Float16*>(st_hi),
-      static_cast<const _Float16*>(st_lo), nullptr, out, num_vectors, dim, padded_dim,
+      static_cast<const _Float16*>(st_lo), st_scale, nullptr, out, num_vectors, dim, padded_dim,
       reinterpret_cast<hipStream_t>(stream));
   if (e != hipSuccess) {
     tq::set_error("%s: launch failed: %s", what, hipGetErrorString(e));

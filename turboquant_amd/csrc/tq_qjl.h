@@ -21,10 +21,11 @@ __device__ __forceinline__ void z_to_half(uint32_t w, uint32_t& lo, uint32_t& hi
 }
 
 // quant: zout = sign(X S^T) from X's halves [n][ldk] and S's halves
-// [ldk][ldk]; else term = z S (fp32 [n][dim]) from S^T's halves.  ldk is a
-// multiple of 128 and >= dim, columns and rows past dim zero.
+// [ldk][ldk]; else term = z S (fp32 [n][dim]) from S^T's halves, column j
+// times wscale[j] (null: 1).  ldk is a multiple of 128 and >= dim, columns and
+// rows past dim zero.
 hipError_t launch_qjl(bool quant, const _Float16* xh, const _Float16* xl, const int8_t* z,
-                      const _Float16* wh, const _Float16* wl, int8_t* zout, float* term, int64_t n,
-                      int dim, int ldk, hipStream_t st);
+                      const _Float16* wh, const _Float16* wl, const float* wscale, int8_t* zout,
+                      float* term, int64_t n, int dim, int ldk, hipStream_t st);
 
 }  // namespace tq

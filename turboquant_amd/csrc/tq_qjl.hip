@@ -14,6 +14,11 @@
 //    hi hi + hi lo + lo hi.  What is dropped is 2^-22 of |S_j| |r|, under the
 //    rounding of an fp32 sum of these terms.
 //  * dequantize: X = z (int8, exact in fp16), W = S^T; two products.
+// Each row of W comes scaled by a power of two that takes its largest entry to
+// [2^14, 2^15) (qjl_operand), so that S has fp32's range here too and lo is
+// normal for every entry down to 2^-17 of its row's largest: without the scale
+// 5% of a Gaussian S (|S| < 0.12) had a lo of fewer bits.  A sign does not see
+// the scale; the dequantize takes it out of the sum, exactly.
 // The halves of one K step feed 12 (8) MFMAs from 8 (6) LDS reads, so the
 // kernels are MFMA-bound where a plain fp16 product of this tile is
 // LDS-bound.  Tiles are copied with direct-to-LDS loads, 16-byte chunks
@@ -50,6 +55,7 @@ struct QjlGemmParams {
   const int8_t* z;      // dequantize: signs [n][dim]
   const _Float16* wh;   // S (quantize) or S^T (dequantize) halves [ldk][ldk]
   const _Float16* wl;
+  const float* wscale;  // dequantize: what the rows of W were divided by [ldk], or null
   int8_t* zout;         // quantize: [n][dim]
   float* term;          // dequantize: [n][dim]
   int64_t n;
@@ -287,10 +293,11 @@ void qjl_gemm_kernel(QjlGemmParams p) {
       for (int j = 0; j < WB; j++) {
         const int col = n0 + wn + 32 * j + ln;
         if (col >= p.dim) continue;
+        const float sc = p.wscale ? p.wscale[col] : 1.0f;
 #pragma unroll
         for (int e = 0; e < 16; e++) {
           const int64_t row = m0 + wm + 32 * i + 8 * (e >> 2) + 4 * hh + (e & 3);
-          if (row < p.n) p.term[row * p.dim + col] = acc[i][j][e];
+          if (row < p.n) p.term[row * p.dim + col] = acc[i][j][e] * sc;
         }
       }
   }
@@ -411,17 +418,89 @@ __global__ __launch_bounds__(256) void split_halves_kernel(const float* __restri
     put(2 * sq + (int64_t)(c0 + i) * pd + r0 + x, tile[x][i]);
 }
 
+// The power of two that takes m (the largest magnitude of a row) to [2^14,
+// 2^15), as far as it and its inverse are normal floats.
+__device__ __forceinline__ float row_scale(float m, float& inv) {
+  const int e = min(253, max(1, 268 - (int)(__float_as_uint(m) >> 23)));
+  inv = __uint_as_float((uint32_t)(254 - e) << 23);
+  return __uint_as_float((uint32_t)e << 23);
+}
+
+__device__ __forceinline__ void put_halves(_Float16* out, int64_t at, int64_t sq, float v) {
+  const _Float16 hi = (_Float16)v;
+  out[at] = hi;
+  // (an infinite entry: lo 0 instead of inf - inf)
+  out[at + sq] = __builtin_isinf((float)hi) ? (_Float16)0.0f : (_Float16)(v - (float)hi);
+}
+
+// W = S as hi + lo [2][pd][pd], rows scaled, zero-padded; one wave per row.
+__global__ __launch_bounds__(256) void operand_rows_kernel(const float* __restrict__ s, int dim,
+                                                           int pd, _Float16* __restrict__ out,
+                                                           float* __restrict__ scales) {
+  const int lane = threadIdx.x & 63, r = 4 * (int)blockIdx.x + (threadIdx.x >> 6);
+  float v[16], m = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    const int c = 64 * i + lane;
+    v[i] = r < dim && c < dim ? s[(int64_t)r * dim + c] : 0.0f;
+    m = fmaxf(m, fabsf(v[i]));
+  }
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) m = fmaxf(m, __shfl_xor(m, d));
+  float inv;
+  const float sc = row_scale(m, inv);
+  if (lane == 0) scales[r] = inv;
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    const int c = 64 * i + lane;
+    if (c < pd) put_halves(out, (int64_t)r * pd + c, (int64_t)pd * pd, v[i] * sc);
+  }
+}
+
+// The same for W = S^T: a workgroup takes 32 columns of S, all their rows in
+// registers (thread: column tid % 32, rows tid / 32 + 32 i), and writes them
+// as rows of W through a 32 x 32 tile.
+__global__ __launch_bounds__(1024) void operand_cols_kernel(const float* __restrict__ s, int dim,
+                                                            int pd, _Float16* __restrict__ out,
+                                                            float* __restrict__ scales) {
+  __shared__ float tile[32][33];
+  const int x = threadIdx.x & 31, y = threadIdx.x >> 5, c0 = 32 * (int)blockIdx.x;
+  float v[32], m = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 32; i++) {
+    const int r = 32 * i + y;
+    v[i] = r < dim && c0 + x < dim ? s[(int64_t)r * dim + c0 + x] : 0.0f;
+    m = fmaxf(m, fabsf(v[i]));
+  }
+  tile[y][x] = m;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 32; k++) m = fmaxf(m, tile[k][x]);
+  float inv;
+  const float sc = row_scale(m, inv);
+  if (y == 0) scales[c0 + x] = inv;
+#pragma unroll
+  for (int i = 0; i < 32; i++) {
+    if (32 * i >= pd) break;  // uniform
+    __syncthreads();
+    tile[x][y] = v[i] * sc;
+    __syncthreads();
+    put_halves(out, (int64_t)(c0 + y) * pd + 32 * i + x, (int64_t)pd * pd, tile[y][x]);
+  }
+}
+
 }  // namespace
 
 hipError_t launch_qjl(bool quant, const _Float16* xh, const _Float16* xl, const int8_t* z,
-                      const _Float16* wh, const _Float16* wl, int8_t* zout, float* term, int64_t n,
-                      int dim, int ldk, hipStream_t st) {
+                      const _Float16* wh, const _Float16* wl, const float* wscale, int8_t* zout,
+                      float* term, int64_t n, int dim, int ldk, hipStream_t st) {
   QjlGemmParams p;
   p.xh = xh;
   p.xl = xl;
   p.z = z;
   p.wh = wh;
   p.wl = wl;
+  p.wscale = wscale;
   p.zout = zout;
   p.term = term;
   p.n = n;
@@ -482,5 +561,31 @@ extern "C" int tq_qjl_halves(const float* s, int32_t dim, int32_t padded_dim, vo
                      static_cast<_Float16*>(halves));
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) set_error("qjl_halves: launch failed: %s", hipGetErrorString(e));
+  return (int)e;
+}
+
+extern "C" int tq_qjl_operand(const float* s, int32_t dim, int32_t padded_dim, int32_t transposed,
+                              void* halves, float* scales, tq_stream_t stream) {
+  using namespace tq;
+  if ((padded_dim != 256 && padded_dim != 512 && padded_dim != 1024) || dim < 1 ||
+      dim > padded_dim) {
+    set_error("qjl_operand: padded_dim %d must be 256, 512 or 1024, dim %d at most that",
+              padded_dim, dim);
+    return kEinval;
+  }
+  if (!s || !halves || !scales) {
+    set_error("qjl_operand: null pointer");
+    return kEinval;
+  }
+  const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  _Float16* const out = static_cast<_Float16*>(halves);
+  if (transposed)
+    hipLaunchKernelGGL(operand_cols_kernel, dim3(padded_dim / 32), dim3(1024), 0, st, s, dim,
+                       padded_dim, out, scales);
+  else
+    hipLaunchKernelGGL(operand_rows_kernel, dim3(padded_dim / 4), dim3(256), 0, st, s, dim,
+                       padded_dim, out, scales);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) set_error("qjl_operand: launch failed: %s", hipGetErrorString(e));
   return (int)e;
 }

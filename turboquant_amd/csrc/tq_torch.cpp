@@ -354,6 +354,23 @@ std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> qjl_halves(const Tenso
   return std::make_tuple(out.select(0, 0), out.select(0, 1), out.select(0, 2), out.select(0, 3));
 }
 
+// ops.qjl_operand
+std::optional<std::tuple<Tensor, Tensor, Tensor>> qjl_operand(const Tensor& s, int64_t padded_dim,
+                                                              bool transposed) {
+  const c10::Device dev = s.device();
+  if (!is_f32(s, dev) || s.dim() != 2 || s.size(0) != s.size(1) || s.size(0) < 1 ||
+      s.size(0) > padded_dim || padded_dim > 1024)
+    return std::nullopt;
+  const c10::DeviceGuard guard(dev);
+  const Tensor out = at::empty({2, padded_dim, padded_dim}, s.options().dtype(at::kHalf));
+  const Tensor scale = at::empty({padded_dim}, s.options());
+  if (!on(out, dev) || !on(scale, dev) ||
+      tq_qjl_operand(cptr<float>(s), s.size(0), padded_dim, transposed, out.data_ptr(),
+                     scale.data_ptr<float>(), stream_of(dev)) != 0)
+    return std::nullopt;
+  return std::make_tuple(out.select(0, 0), out.select(0, 1), scale);
+}
+
 // ops.prod_quantize_qjl (large: prod_quantize_qjl_ws)
 ProdCodes prod_quantize_qjl(const Tensor& x, int64_t padded_dim, int64_t bits, const Tensor& signs,
                             const std::vector<double>& boundaries,
@@ -397,7 +414,8 @@ ProdCodes prod_quantize_qjl(const Tensor& x, int64_t padded_dim, int64_t bits, c
 OptTensor prod_dequantize_qjl(const Tensor& packed, const Tensor& norms, const Tensor& z,
                               const Tensor& rnorm, int64_t dim, int64_t padded_dim, int64_t bits,
                               const Tensor& signs, const std::vector<double>& centroids,
-                              const Tensor& st_hi, const Tensor& st_lo, bool large) {
+                              const Tensor& st_hi, const Tensor& st_lo, bool large,
+                              const OptTensor& st_scale) {
   const c10::Device dev = packed.device();
   if (!codes(packed, norms, padded_dim, bits, dev) || dim < 1 || !is_f32(rnorm, dev) ||
       rnorm.sizes() != norms.sizes() || !on(z, dev) || z.scalar_type() != at::kChar ||
@@ -405,18 +423,27 @@ OptTensor prod_dequantize_qjl(const Tensor& packed, const Tensor& norms, const T
       z.sizes().slice(0, z.dim() - 1) != norms.sizes() || !z.is_contiguous() || !aligned(z, 16) ||
       !is_f32(signs, dev) || signs.numel() < padded_dim || !aligned(signs, 16) ||
       !halves(st_hi, padded_dim, dev) || !halves(st_lo, padded_dim, dev) ||
-      (int64_t)centroids.size() != (1 << bits))
+      (int64_t)centroids.size() != (1 << bits) ||
+      (st_scale.has_value() &&
+       (!large || !is_f32(*st_scale, dev) || st_scale->numel() < padded_dim)))
     return std::nullopt;
   const c10::DeviceGuard guard(dev);
   const Tensor out = at::empty(lead_and(packed, dim), norms.options());
   if (!on(out, dev)) return std::nullopt;
   const auto c = table16(centroids);
-  const auto fn = large ? tq_prod_dequantize_qjl_ws : tq_prod_dequantize_qjl;
-  if (fn(cptr<uint8_t>(packed), cptr<float>(norms),
-         cptr<int8_t>(z), cptr<float>(rnorm), norms.numel(), dim, padded_dim,
-         bits, cptr<float>(signs), c.data(), st_hi.const_data_ptr(),
-         st_lo.const_data_ptr(), out.data_ptr<float>(), stream_of(dev)) != 0)
-    return std::nullopt;
+  const int rc =
+      large ? tq_prod_dequantize_qjl_ws(
+                  cptr<uint8_t>(packed), cptr<float>(norms), cptr<int8_t>(z), cptr<float>(rnorm),
+                  norms.numel(), dim, padded_dim, bits, cptr<float>(signs), c.data(),
+                  st_hi.const_data_ptr(), st_lo.const_data_ptr(),
+                  st_scale.has_value() ? cptr<float>(*st_scale) : nullptr, out.data_ptr<float>(),
+                  stream_of(dev))
+            : tq_prod_dequantize_qjl(
+                  cptr<uint8_t>(packed), cptr<float>(norms), cptr<int8_t>(z), cptr<float>(rnorm),
+                  norms.numel(), dim, padded_dim, bits, cptr<float>(signs), c.data(),
+                  st_hi.const_data_ptr(), st_lo.const_data_ptr(), out.data_ptr<float>(),
+                  stream_of(dev));
+  if (rc != 0) return std::nullopt;
   return out;
 }
 
@@ -460,6 +487,7 @@ TORCH_LIBRARY_IMPL(turboquant_v5, CUDA, m) {
 }
 
 PYBIND11_MODULE(_tq_torch, m) {
+  m.attr("abi_version") = TQ_ABI_VERSION;
   const auto unlocked = py::call_guard<py::gil_scoped_release>();
   m.def("write_cache", &write_cache, unlocked);
   m.def("decode_balanced", &decode_balanced, unlocked);
@@ -468,6 +496,7 @@ PYBIND11_MODULE(_tq_torch, m) {
   m.def("mse_quantize", &mse_quantize, unlocked);
   m.def("mse_dequantize", &mse_dequantize, unlocked);
   m.def("qjl_halves", &qjl_halves, unlocked);
+  m.def("qjl_operand", &qjl_operand, unlocked);
   m.def("prod_quantize_qjl", &prod_quantize_qjl, unlocked);
   m.def("prod_dequantize_qjl", &prod_dequantize_qjl, unlocked);
 }

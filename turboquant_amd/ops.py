@@ -45,6 +45,10 @@ def _native():
         except ImportError as e:
             raise RuntimeError(f"turboquant_amd._tq_torch cannot be loaded ({e}). "
                                "Run `python -m turboquant_amd.build`.") from e
+        abi = getattr(_tq_torch, "abi_version", None)
+        if abi != _lib.ABI_VERSION:  # built against another header
+            raise RuntimeError(f"turboquant_amd._tq_torch ABI {abi} != expected "
+                               f"{_lib.ABI_VERSION}; rebuild it")
         _nat = _tq_torch
     return _nat
 
@@ -525,6 +529,28 @@ def qjl_halves(s: torch.Tensor, padded_dim: int):
     return out.unbind(0)
 
 
+def qjl_operand(s: torch.Tensor, padded_dim: int, transposed: bool):
+    """(hi, lo, scale) of the QJL matrix s fp32 [dim, dim], or of its transpose,
+    for prod_quantize_qjl_ws / prod_dequantize_qjl_ws: fp16 halves [padded_dim,
+    padded_dim] of the rows, each over its power of two scale[row]
+    (tq_qjl_operand)."""
+    r = (_nat or _native()).qjl_operand(s, padded_dim, transposed)
+    if r is not None:
+        return r
+    _require_gpu(s)
+    if s.dtype != torch.float32 or s.dim() != 2 or s.size(0) != s.size(1):
+        raise RuntimeError("qjl_operand: S must be a square fp32 matrix")
+    s = s.contiguous()
+    out = torch.empty((2, padded_dim, padded_dim), dtype=torch.float16, device=s.device)
+    scale = torch.empty((padded_dim,), dtype=torch.float32, device=s.device)
+    lib = _lib.load()
+    with torch.cuda.device(s.device):
+        rc = lib.tq_qjl_operand(s.data_ptr(), s.size(0), int(padded_dim), int(transposed),
+                                out.data_ptr(), scale.data_ptr(), _stream_ptr(s.device))
+    _lib.check(rc, "qjl_operand")
+    return out[0], out[1], scale
+
+
 def mse_quantize(x: torch.Tensor, padded_dim: int, bit_width: int, signs: torch.Tensor,
                  boundaries) -> tuple[torch.Tensor, torch.Tensor]:
     """TurboQuantMSE.quantize on the GPU (tq_mse_quantize): x fp32
@@ -736,19 +762,21 @@ def prod_dequantize_qjl(packed: torch.Tensor, norms: torch.Tensor, qjl_signs: to
 def prod_dequantize_qjl_ws(packed: torch.Tensor, norms: torch.Tensor, qjl_signs: torch.Tensor,
                            residual_norms: torch.Tensor, dim: int, padded_dim: int,
                            mse_bit_width: int, signs: torch.Tensor, centroids,
-                           st_hi: torch.Tensor, st_lo: torch.Tensor) -> torch.Tensor:
+                           st_hi: torch.Tensor, st_lo: torch.Tensor,
+                           st_scale: torch.Tensor | None = None) -> torch.Tensor:
     """prod_dequantize_qjl at padded_dim 256, 512 or 1024
-    (tq_prod_dequantize_qjl_ws)."""
+    (tq_prod_dequantize_qjl_ws); st_scale: fp32 [padded_dim], the row scales
+    of the halves (qjl_operand), none for unscaled ones (qjl_halves)."""
     return _prod_dequantize_qjl(packed, norms, qjl_signs, residual_norms, dim, padded_dim,
-                                mse_bit_width, signs, centroids, st_hi, st_lo, True)
+                                mse_bit_width, signs, centroids, st_hi, st_lo, True, st_scale)
 
 
 def _prod_dequantize_qjl(packed, norms, qjl_signs, residual_norms, dim, padded_dim, mse_bit_width,
-                         signs, centroids, st_hi, st_lo, large: bool):
+                         signs, centroids, st_hi, st_lo, large: bool, st_scale=None):
     centroids = _floats(centroids)
     r = (_nat or _native()).prod_dequantize_qjl(packed, norms, qjl_signs, residual_norms, dim,
                                                 padded_dim, mse_bit_width, signs, centroids, st_hi,
-                                                st_lo, large)
+                                                st_lo, large, st_scale)
     if r is not None:
         return r
     _require_gpu(packed, norms, qjl_signs, residual_norms, signs, st_hi, st_lo)
@@ -765,6 +793,11 @@ def _prod_dequantize_qjl(packed, norms, qjl_signs, residual_norms, dim, padded_d
                 or not t.is_contiguous() or t.data_ptr() % 16:
             raise RuntimeError("prod_dequantize_qjl: S^T halves must be contiguous aligned "
                                "fp16 [padded_dim, padded_dim]")
+    if st_scale is not None:
+        _require_gpu(packed, st_scale)
+        if st_scale.dtype != torch.float32 or st_scale.numel() < padded_dim \
+                or not st_scale.is_contiguous():
+            raise RuntimeError("prod_dequantize_qjl: st_scale must be fp32 [padded_dim]")
     packed = packed.contiguous()
     if packed.data_ptr() % 16:
         packed = packed.clone()
@@ -775,11 +808,15 @@ def _prod_dequantize_qjl(packed, norms, qjl_signs, residual_norms, dim, padded_d
     signs = _aligned16(signs)
     lib = _lib.load()
     with torch.cuda.device(packed.device):
-        fn = lib.tq_prod_dequantize_qjl_ws if large else lib.tq_prod_dequantize_qjl
-        rc = fn(packed.data_ptr(), nf.data_ptr(), z.data_ptr(), rn.data_ptr(), nf.numel(),
+        args = (packed.data_ptr(), nf.data_ptr(), z.data_ptr(), rn.data_ptr(), nf.numel(),
                 int(dim), int(padded_dim), int(mse_bit_width), signs.data_ptr(),
-                _host_f32(centroids), st_hi.data_ptr(), st_lo.data_ptr(), out.data_ptr(),
-                _stream_ptr(packed.device))
+                _host_f32(centroids), st_hi.data_ptr(), st_lo.data_ptr())
+        tail = (out.data_ptr(), _stream_ptr(packed.device))
+        if large:
+            rc = lib.tq_prod_dequantize_qjl_ws(
+                *args, None if st_scale is None else st_scale.data_ptr(), *tail)
+        else:
+            rc = lib.tq_prod_dequantize_qjl(*args, *tail)
     _lib.check(rc, "prod_dequantize_qjl")
     return out
 
