@@ -115,7 +115,8 @@ def test_prod_hip_kernels_against_the_torch_path(dim, bits):
     only the norm's summation order differs); QJL signs against the CPU path
     where the codes agree; the dequantize epilogue against torch's
     x_mse + (z S) * (sqrt(pi/2) / d * gamma) on the same GEMM output, bit
-    for bit."""
+    for bit; the public dequantize, which forms z S on the matrix cores,
+    within the roundings of that product."""
     print(f"case: algorithm Prod HIP dim={dim} bits={bits}", flush=True)
     from turboquant_amd import ops
     g = torch.Generator().manual_seed(dim * 7 + bits)
@@ -192,7 +193,15 @@ def test_prod_hip_kernels_against_the_torch_path(dim, bits):
         print(f"  fused dequantize max |diff| from the fp32 GEMM expression {err:.2e}", flush=True)
         assert torch.allclose(xh, want, rtol=1e-5, atol=1e-5 * want.abs().max().item())
     else:
-        assert torch.equal(xh, want)
+        # z S in the kernel: S as hi + lo (2^-22 of it), the sum of 2 K products
+        # rounded to 2^-24 each; then the weight, the product and the sum
+        w = (qg.qjl.dequant_scale * rg.unsqueeze(-1)).double()
+        mse, s64 = qg.mse.dequantize(pg, ng).double(), qg.qjl.S.double()
+        term64 = (zg.double() @ s64) * w
+        bound = (zg.double().abs() @ s64.abs()) * w * (2.0 ** -22 + (2 * dim + 4) * 2.0 ** -24) \
+            + (mse.abs() + term64.abs()) * 2.0 ** -22
+        err = (xh.double() - (mse + term64)).abs()
+        assert bool((err <= bound).all()), (err - bound).max().item()
     # and against the CPU dequantize of the CPU's own outputs, within GEMM rounding
     xc = qc.dequantize(pc, nc, zc, rc)
     ok = same & (zg.cpu() == zc).all(-1)

@@ -99,14 +99,15 @@ def test_every_form_against_64_bits(dim, n):
     test_dequantize_term_against_64_bits(dim, n)
 
 
-def test_dequantize_paths_agree_around_the_size_rule():
-    """One vector fewer than QJL_GEMM_MIN (the torch product) and that many:
-    the rows they share are within the roundings of both."""
-    q, x, pd, (bnd, cen) = _prod(200, 4, A.QJL_GEMM_MIN)
+@pytest.mark.parametrize("dim", [200, 1000])
+def test_a_vector_has_the_same_bits_in_any_batch(dim):
+    """Alone, in batches that take 64 x 64 tiles and in one that takes 128 x 128
+    tiles: the sum over K runs in the same order in all of them."""
+    q, x, _, _ = _prod(dim, 4, 21001)
     out = q.quantize(x)
-    many, few = q.dequantize(*out), q.dequantize(*[t[:-1] for t in out])
-    assert few.shape[0] == A.QJL_GEMM_MIN - 1
-    assert torch.allclose(many[:-1], few, rtol=1e-5, atol=1e-5 * few.abs().max().item())
+    whole = q.dequantize(*out)
+    for a, b in ((0, 0), (0, 1), (63, 64), (21000, 21001), (7, 72), (100, 2147), (0, 2048)):
+        assert torch.equal(q.dequantize(*[t[a:b].clone() for t in out]), whole[a:b]), (a, b)
 
 
 @pytest.mark.parametrize("dim", [50, 98, 130, 258, 514, 1002, 1023])

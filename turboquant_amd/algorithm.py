@@ -44,15 +44,6 @@ CENTROIDS_N01 = {
 }
 
 
-# Vectors from which TurboQuantProd.dequantize above padded size 128 forms z S
-# with this package's kernel.  The kernel is the faster one at every size (1500
-# vectors of dim 1000: 41 against 63 us; 4096 of 1024: 43 against 88; 20011:
-# 135 against 386) and the nearer one to 64 bits; below the line the product stays
-# torch's fp32 GEMM so that small batches keep equalling torch's expression
-# z.float() @ S bit for bit, which callers compare against.
-QJL_GEMM_MIN = 2048
-
-
 def _levels(bit_width: int) -> list[float]:
     pos = list(CENTROIDS_N01[bit_width])
     return [-c for c in reversed(pos)] + pos
@@ -305,6 +296,9 @@ class TurboQuantProd:
 
     @torch.no_grad()
     def dequantize(self, mse_packed, mse_norms, qjl_signs, residual_norms) -> torch.Tensor:
+        """The inverse of quantize; int8 signs on a GPU take the HIP kernels
+        (tq_prod_dequantize_qjl up to padded size 128, the _ws form above),
+        which give a vector the same bits in a batch of any size."""
         if self.mse._hip(mse_packed) and mse_norms.dtype == torch.float32:
             from . import ops
             pd = self.mse.rotation.padded_dim
@@ -314,7 +308,7 @@ class TurboQuantProd:
                                                self.dim, pd, self.mse.bit_width,
                                                self.mse.rotation.signs,
                                                self.mse._host_tables()[1], th, tl)
-            if qjl_signs.dtype == torch.int8 and mse_norms.numel() >= QJL_GEMM_MIN:
+            if qjl_signs.dtype == torch.int8:
                 th, tl, scale = self._qjl_operand(self.dim, True)
                 return ops.prod_dequantize_qjl_ws(mse_packed, mse_norms, qjl_signs,
                                                   residual_norms, self.dim, pd,
