@@ -224,6 +224,16 @@ void qjl_gemm_kernel(QjlGemmParams p) {
     }
   };
 
+  // the lane's output scales, loaded ahead of the K loop (loaded at its end
+  // 20,011 vectors of dim 1000 take 132 us against 124)
+  float wsc[WB];
+#pragma unroll
+  for (int j = 0; j < WB; j++) wsc[j] = 1.0f;
+  if constexpr (!QUANT)
+    if (p.wscale)
+#pragma unroll
+      for (int j = 0; j < WB; j++) wsc[j] = p.wscale[n0 + wn + 32 * j + ln];  // < ldk
+
   const int nk = (p.dim + kBK - 1) / kBK;
   issue(0, buf0);
   if constexpr (!QUANT) {
@@ -293,11 +303,10 @@ void qjl_gemm_kernel(QjlGemmParams p) {
       for (int j = 0; j < WB; j++) {
         const int col = n0 + wn + 32 * j + ln;
         if (col >= p.dim) continue;
-        const float sc = p.wscale ? p.wscale[col] : 1.0f;
 #pragma unroll
         for (int e = 0; e < 16; e++) {
           const int64_t row = m0 + wm + 32 * i + 8 * (e >> 2) + 4 * hh + (e & 3);
-          if (row < p.n) p.term[row * p.dim + col] = acc[i][j][e] * sc;
+          if (row < p.n) p.term[row * p.dim + col] = acc[i][j][e] * wsc[j];
         }
       }
   }
