@@ -82,6 +82,25 @@ def test_batch_against_float64(reqs, hq, hkv, hd, dtype):
             assert bool(((got - want).abs() <= tol).all()), (got - want).abs().max().item()
 
 
+# more query blocks or shares than one launch's list of items holds: runs of
+# whole blocks (both workgroup shapes), runs of shares, several requests in them
+RUNS = [
+    ([(41217, 0)], 8, 1, 128, torch.float16),
+    ([(41000, 100)], 16, 2, 64, torch.float16),
+    ([(21000, 0)], 2, 1, 128, torch.bfloat16),
+    ([(20600, 1000)], 1, 1, 256, torch.float16),
+    ([(20999, 0)], 2, 1, 64, torch.bfloat16),
+    ([(9000, 0), (700, 5000), (12000, 300), (1, 50), (129, 0)], 1, 1, 128, torch.float16),
+    ([(5000, 60000)], 1, 1, 96, torch.float16),
+    ([(420, 2000)] * 63 + [(1500, 9)], 4, 1, 128, torch.bfloat16),
+]
+
+
+@pytest.mark.parametrize("reqs,hq,hkv,hd,dtype", RUNS)
+def test_runs_against_float64(reqs, hq, hkv, hd, dtype):
+    test_batch_against_float64(reqs, hq, hkv, hd, dtype)
+
+
 @pytest.mark.parametrize("hq,hkv", [(1, 1), (7, 7), (8, 8), (9, 3), (16, 2), (24, 8), (40, 8)])
 def test_head_orders(hq, hkv):
     """Every head is served once whatever the head count (multiples of 8 are

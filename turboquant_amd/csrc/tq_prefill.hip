@@ -95,8 +95,15 @@ struct PrefillParams {
 // Batch mode: the query blocks of several requests in one launch, as a list of
 // work items (a kernel argument, so no device copy of the plan is needed).
 // Item: query block qb (kBM rows) of request req over its key tiles [t0, t1);
-// slot >= 0: the tiles are a share of the block's, O and (max, sum) go to that
-// workspace slot for prefill_batch_merge_kernel.
+// ws_row >= 0: the tiles are a share of the block's, O and (max, sum) of its
+// rows go to the workspace rows from there for prefill_batch_merge_kernel.
+//
+// More items than the list holds (160: a prompt of 40,960 tokens, less where
+// few heads need splits) go as one run of blocks per request, one workgroup row
+// per block and grid z for its shares, which the workgroup works out by itself:
+// still one launch, where lists of 160 one after the other leave the card to
+// drain in between (48,000 tokens at 4 q heads 2.42 -> 2.26 ms, 30,000 at two
+// 0.72 -> 0.49, 60,000 at one 1.83 -> 0.96).
 struct PrefillReq {
   int q0, lq;  // first row in q and o, query rows
   int k0, lk;  // first row in the K / V source, keys
@@ -104,9 +111,36 @@ struct PrefillReq {
 };
 struct PrefillItem {
   uint32_t req_qb;  // req | qb << 6
-  int t0, t1, slot;
+  int t0, t1, ws_row;
+};
+struct PrefillRun {  // the blocks of a request, the last (longest) first
+  int first, req;    // its first workgroup row
+  int ws_row;        // share z of its query row i: workspace row ws_row + z lq + i
 };
 constexpr int kBatchReqs = 64, kBatchItems = 160;
+
+// the shares of a block of `tiles` key tiles, of `unit` each but the last (0:
+// blocks stay whole)
+__host__ __device__ inline int split_shares(int tiles, int unit) {
+  return unit == 0 ? 1 : (tiles + unit - 1) / unit;
+}
+
+// the run of workgroup row y: the last that starts at or before it
+__device__ __forceinline__ PrefillRun find_run(const PrefillRun* runs, int n, int y) {
+  int lo = 0, hi = n - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (runs[mid].first <= y) lo = mid;
+    else hi = mid - 1;
+  }
+  return runs[lo];
+}
+
+// key tiles that any row of query block qb sees
+template <int kBM, int kBN>
+__device__ __forceinline__ int block_tiles(const PrefillReq& rq, int qb) {
+  return (rq.lk - rq.lq + min((qb + 1) * kBM, rq.lq) + kBN - 1) / kBN;
+}
 struct PrefillBatch {
   const void* q;
   const _Float16* k;
@@ -118,10 +152,14 @@ struct PrefillBatch {
   int ratio, hd;      // hd <= kD: dims of q and o rows (zero padded to kD here)
   int q_bf16, o_bf16;  // q / o element type (else fp16)
   float c;             // sm_scale * log2(e)
-  float* ws_o;         // [slot][kBM 128][Hq][kD]
-  float* ws_ml;        // [slot][128][Hq][2]
+  float* ws_o;         // [row][Hq][kD]
+  float* ws_ml;        // [row][Hq][2]
+  int nruns, unit, y0;  // runs (0: items), their split_shares unit, this launch's first row
   PrefillReq reqs[kBatchReqs];
-  PrefillItem items[kBatchItems];
+  union {
+    PrefillItem items[kBatchItems];
+    PrefillRun runs[kBatchReqs];
+  };
 };
 static_assert(sizeof(PrefillBatch) <= 4096, "kernel argument");
 
@@ -156,7 +194,7 @@ __device__ __forceinline__ float sum32(float x) {
 // what one workgroup computes: rows qb kBM .. of a request (query rows from
 // q_row0) over its key tiles [t0, t1)
 struct PrefillWork {
-  int qb, q_row0, lq, lk, t0, t1, slot, hd;
+  int qb, q_row0, lq, lk, t0, t1, ws_row, hd;  // t1 < 0: nothing
   const _Float16* k;
   const _Float16* v;
   int64_t k_st, k_sh, v_st, v_sh;
@@ -169,7 +207,7 @@ __device__ __forceinline__ PrefillWork prefill_work(const PrefillParams& p) {
   r.q_row0 = 0;
   r.lq = p.lq;
   r.lk = p.lk;
-  r.slot = -1;
+  r.ws_row = -1;
   r.hd = 0;
   r.k = p.k;
   r.v = p.v;
@@ -190,16 +228,28 @@ __device__ __forceinline__ PrefillWork prefill_work(const PrefillParams& p) {
 
 template <int kBM, int kBN, bool SPLIT>
 __device__ __forceinline__ PrefillWork prefill_work(const PrefillBatch& p) {
-  const PrefillItem it = p.items[blockIdx.y];
-  const PrefillReq rq = p.reqs[it.req_qb & 63u];
   PrefillWork r;
-  r.qb = (int)(it.req_qb >> 6);
+  PrefillReq rq;
+  if (p.nruns == 0) {
+    const PrefillItem it = p.items[blockIdx.y];
+    rq = p.reqs[it.req_qb & 63u];
+    r.qb = (int)(it.req_qb >> 6);
+    r.t0 = it.t0;
+    r.t1 = it.t1;
+    r.ws_row = it.ws_row;
+  } else {
+    const int y = p.y0 + (int)blockIdx.y, z = (int)blockIdx.z;
+    const PrefillRun run = find_run(p.runs, p.nruns, y);
+    rq = p.reqs[run.req];
+    r.qb = (rq.lq + kBM - 1) / kBM - 1 - (y - run.first);
+    const int tiles = block_tiles<kBM, kBN>(rq, r.qb), ns = split_shares(tiles, p.unit);
+    r.t0 = z * p.unit;
+    r.t1 = z >= ns ? -1 : ns > 1 ? min(tiles, r.t0 + p.unit) : tiles;
+    r.ws_row = ns > 1 ? run.ws_row + z * rq.lq + r.qb * kBM : -1;
+  }
   r.q_row0 = rq.q0;
   r.lq = rq.lq;
   r.lk = rq.lk;
-  r.t0 = it.t0;
-  r.t1 = it.t1;
-  r.slot = it.slot;
   r.hd = p.hd;
   r.k_st = rq.src ? p.k2_st : p.k_st;
   r.k_sh = rq.src ? p.k2_sh : p.k_sh;
@@ -250,6 +300,7 @@ void prefill_kernel(PP p) {
   const int hh = lane >> 5, n = lane & 31;
   const int head = head_of_block(), g = head / p.ratio;
   const PrefillWork wk = prefill_work<kBM, kBN, SPLIT>(p);
+  if (kBatch && wk.t1 < 0) return;
   const int q0 = wk.qb * kBM;
   const int off = wk.lk - wk.lq;
   const int qrow = q0 + 32 * w + n;  // this lane's query row (of its request)
@@ -487,13 +538,13 @@ void prefill_kernel(PP p) {
 
   lsum = sum32(lsum);
   const float inv = lsum > 0.0f ? 1.0f / lsum : 0.0f;
-  if (SPLIT || (kBatch && wk.slot >= 0)) {
+  if (SPLIT || (kBatch && wk.ws_row >= 0)) {
     // this split's O / row sum and (mc, row sum); a split that held no visible
     // key for a row leaves mc = -inf, sum 0, O = 0.  One request: as fp16 (a
     // convex combination of V rows: safe).  Batch mode splits blocks that one
     // launch per request left whole, so what was a sum in fp32 stays one: fp32.
     if (qrow < wk.lq) {
-      const int64_t r = (kBatch ? (int64_t)wk.slot * kBM + 32 * w + n
+      const int64_t r = (kBatch ? (int64_t)wk.ws_row + 32 * w + n
                                 : (int64_t)blockIdx.z * wk.lq + qrow) * gridDim.x + head;
       if constexpr (kBatch) {
         float* const wo = p.ws_o + r * kD + 4 * hh;
@@ -824,7 +875,8 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p, int
 // Merge of the split query blocks of a batch: D / 8 lanes per (row, q head), 8
 // dims (16 bytes) each, the same weights as above.
 struct PrefillGroup {
-  int q_row, slot0;  // the block's first row in o, its first slot
+  int q_row, ws_row;  // the block's first row in o, and in the workspace
+  int stride;         // workspace rows from one share to the next
   uint16_t nsplit, rows;
 };
 struct PrefillMerge {
@@ -833,19 +885,41 @@ struct PrefillMerge {
   int hq, hd, o_bf16;
   const float* ws_o;
   const float* ws_ml;
-  PrefillGroup groups[kBatchItems];
+  int nruns, unit, y0;  // as in PrefillBatch
+  union {
+    PrefillGroup groups[kBatchItems];
+    struct {
+      PrefillReq reqs[kBatchReqs];
+      PrefillRun runs[kBatchReqs];
+    };
+  };
 };
 
 template <int kD>
 __global__ __launch_bounds__(256) void prefill_batch_merge_kernel(PrefillMerge p) {
   constexpr int L = kD / 8, kVecs = 256 / L;
-  const PrefillGroup g = p.groups[blockIdx.y];
+  PrefillGroup g;
+  if (p.nruns == 0) {
+    g = p.groups[blockIdx.y];
+  } else {
+    constexpr int kBM = 128, kBN = 64;  // what splits blocks
+    const int y = p.y0 + (int)blockIdx.y;
+    const PrefillRun run = find_run(p.runs, p.nruns, y);
+    const PrefillReq rq = p.reqs[run.req];
+    const int qb = (rq.lq + kBM - 1) / kBM - 1 - (y - run.first);
+    g.nsplit = (uint16_t)split_shares(block_tiles<kBM, kBN>(rq, qb), p.unit);
+    if (g.nsplit < 2) return;
+    g.q_row = rq.q0 + qb * kBM;
+    g.ws_row = run.ws_row + qb * kBM;
+    g.stride = rq.lq;
+    g.rows = (uint16_t)min(kBM, rq.lq - qb * kBM);
+  }
   const int idx = (int)blockIdx.x * kVecs + (int)threadIdx.x / L;  // row * hq + head
   const int c = 8 * ((int)threadIdx.x % L);
   if (idx >= g.rows * p.hq) return;
   const int row = idx / p.hq, head = idx % p.hq;
-  const int64_t zs = (int64_t)128 * p.hq;  // vectors of one slot
-  const int64_t v0 = g.slot0 * zs + idx;
+  const int64_t zs = (int64_t)g.stride * p.hq;  // vectors from share to share
+  const int64_t v0 = (int64_t)g.ws_row * p.hq + idx;
   float mx = -INFINITY;
   for (int z = 0; z < g.nsplit; z++) mx = fmaxf(mx, p.ws_ml[2 * (v0 + z * zs)]);
   float den = 0.0f, acc[8];
@@ -954,13 +1028,15 @@ PrefillPlan plan_prefill(int q_len, int kv_len, int heads, int head_dim) {
 }
 
 // Plan of one batch of at most kBatchReqs requests: its items (longest first)
-// and the split query blocks.
+// and the split query blocks, or its runs.
 struct BatchPlan {
   int nw = 4;
-  int slots = 0;
+  int ws_rows = 0;
   std::vector<PrefillItem> items;
   std::vector<PrefillGroup> groups;  // q_row: of the request (group_req)
   std::vector<int> group_req;
+  std::vector<PrefillRun> runs;  // not empty: instead of items and groups
+  int unit = 0, shares = 1, rows = 0;  // of the runs: unit, most shares of a block, blocks
 };
 
 struct QueryBlock {
@@ -1026,7 +1102,9 @@ BatchPlan plan_batch(const int32_t* q_lens, const int32_t* kv_lens, int nreq, in
   };
   double best = batch_time(blocks.size(), groups, [&](size_t i) { return blocks[i].tiles; });
   double unit = 1e30;
-  if (!blocks.empty() && blocks.size() <= 4 * groups) {
+  int run_unit = 0;                              // not 0: split in runs, by this unit
+  bool long_list = blocks.size() > kBatchItems;  // a split does not fit the list
+  if (!blocks.empty() && !long_list && blocks.size() <= 4 * groups) {
     const double even = std::max(8.0, total / groups);  // tiles per slot, at least 512 keys
     for (const double f : {1.5, 1.05, 0.8, 0.5}) {
       const double u = std::max(8.0, f * even);
@@ -1038,6 +1116,10 @@ BatchPlan plan_batch(const int32_t* q_lens, const int32_t* kv_lens, int nreq, in
         cost.insert(cost.end(), ns, (double)((b.tiles + ns - 1) / ns));
       }
       if (slots == 0) continue;
+      if (cost.size() > kBatchItems) {
+        long_list = true;
+        continue;
+      }
       std::sort(cost.begin(), cost.end(), [](double x, double y) { return x > y; });
       // the merge: its launch and the slots' rows written and read
       const double t = batch_time(cost.size(), groups, [&](size_t i) { return cost[i]; }) + 2.0 +
@@ -1048,6 +1130,28 @@ BatchPlan plan_batch(const int32_t* q_lens, const int32_t* kv_lens, int nreq, in
       }
     }
   }
+  const int64_t wgs = (int64_t)blocks.size() * heads;
+  if (long_list && wgs < 2 * cus && blocks[0].tiles >= 16) {
+    // splits in runs: as many shares of the longest block as give every CU two
+    // workgroups, each at least 8 tiles; shares of one size start longest
+    // first and the remainders fill in behind them
+    const int most = blocks[0].tiles;
+    const int ns = (int)std::min<int64_t>(((int64_t)(2 * cus) + wgs - 1) / wgs, most / 8);
+    const int u = (most + ns - 1) / ns;
+    int slots = 0, items = 0;
+    for (const QueryBlock& b : blocks) {
+      const int n = split_shares(b.tiles, u);
+      items += n;
+      if (n > 1) slots += n;
+    }
+    // (so many shares that the merge is bound by their bytes, 0.04 us per 128
+    // rows of a head written and read)
+    const double t = std::max(u + 1.0, (total + items) / groups) + 2.0 + 0.6 * slots * heads / 32.0;
+    if (slots > 0 && t < best) {
+      best = t;
+      run_unit = u;
+    }
+  }
   if (head_dim != 256) {
     const std::vector<QueryBlock> wide =
         query_blocks(q_lens, kv_lens, nreq, 256, head_dim == 128 ? 128 : 64);
@@ -1056,21 +1160,35 @@ BatchPlan plan_batch(const int32_t* q_lens, const int32_t* kv_lens, int nreq, in
     if (head_dim == 128 ? t * 3.84 <= best * 2.1 : t * 2.15 <= best * 1.15) {
       bp.nw = 8;
       unit = 1e30;
+      run_unit = 0;
       blocks = wide;
     }
   }
   const int bm = bp.nw == 8 ? 256 : 128;
+  if (run_unit || blocks.size() > kBatchItems) {
+    bp.unit = run_unit;
+    std::vector<int> shares(nreq, 0);  // of a request's longest block, which comes first
+    for (const QueryBlock& b : blocks) {
+      if (shares[b.req]) continue;
+      const int ns = shares[b.req] = split_shares(b.tiles, bp.unit);
+      bp.runs.push_back({bp.rows, b.req, bp.ws_rows});
+      bp.rows += (q_lens[b.req] + bm - 1) / bm;
+      bp.shares = std::max(bp.shares, ns);
+      if (ns > 1) bp.ws_rows += ns * q_lens[b.req];
+    }
+    return bp;
+  }
   for (const QueryBlock& b : blocks) {
     int ns = parts(b.tiles, unit);
     const int per = (b.tiles + ns - 1) / ns;
     ns = (b.tiles + per - 1) / per;
-    const int slot0 = bp.slots;
+    const int row0 = bp.ws_rows;
     for (int z = 0; z < ns; z++)
       bp.items.push_back({(uint32_t)b.req | (uint32_t)b.qb << 6, z * per,
-                          std::min(b.tiles, (z + 1) * per), ns > 1 ? slot0 + z : -1});
+                          std::min(b.tiles, (z + 1) * per), ns > 1 ? row0 + 128 * z : -1});
     if (ns > 1) {
-      bp.slots += ns;
-      bp.groups.push_back({b.qb * bm, slot0, (uint16_t)ns,
+      bp.ws_rows += 128 * ns;
+      bp.groups.push_back({b.qb * bm, row0, 128, (uint16_t)ns,
                            (uint16_t)std::min(bm, q_lens[b.req] - b.qb * bm)});
       bp.group_req.push_back(b.req);
     }
@@ -1081,12 +1199,17 @@ BatchPlan plan_batch(const int32_t* q_lens, const int32_t* kv_lens, int nreq, in
   return bp;
 }
 
+constexpr int kGridRows = 65535;  // workgroup rows of one launch
+
 template <int D>
 hipError_t launch_batch(const BatchPlan& bp, int heads, hipStream_t st, PrefillBatch& p) {
-  for (size_t a = 0; a < bp.items.size(); a += kBatchItems) {
-    const unsigned n = (unsigned)std::min<size_t>(kBatchItems, bp.items.size() - a);
-    std::copy_n(bp.items.begin() + a, n, p.items);
-    const dim3 grid(heads, n);
+  const int nrows = bp.runs.empty() ? (int)bp.items.size() : bp.rows;
+  p.nruns = (int)bp.runs.size();
+  p.unit = bp.unit;
+  if (p.nruns) std::copy(bp.runs.begin(), bp.runs.end(), p.runs);
+  else std::copy(bp.items.begin(), bp.items.end(), p.items);
+  for (p.y0 = 0; p.y0 < nrows; p.y0 += kGridRows) {
+    const dim3 grid(heads, std::min(kGridRows, nrows - p.y0), bp.shares);
     if (bp.nw == 8) {
       if constexpr (D == 64)
         hipLaunchKernelGGL((prefill_rb_kernel<D, 4, 64, 2, 2, PrefillBatch>), grid, dim3(256), 0,
@@ -1101,7 +1224,8 @@ hipError_t launch_batch(const BatchPlan& bp, int heads, hipStream_t st, PrefillB
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  PrefillMerge m;
+  if (bp.ws_rows == 0) return hipSuccess;
+  PrefillMerge m = {};
   m.o = p.o;
   m.o_st = p.o_st;
   m.o_sh = p.o_sh;
@@ -1110,16 +1234,25 @@ hipError_t launch_batch(const BatchPlan& bp, int heads, hipStream_t st, PrefillB
   m.o_bf16 = p.o_bf16;
   m.ws_o = p.ws_o;
   m.ws_ml = p.ws_ml;
-  for (size_t a = 0; a < bp.groups.size(); a += kBatchItems) {
-    const unsigned n = (unsigned)std::min<size_t>(kBatchItems, bp.groups.size() - a);
-    int rows = 0;
-    for (unsigned i = 0; i < n; i++) {
-      m.groups[i] = bp.groups[a + i];
-      m.groups[i].q_row += p.reqs[bp.group_req[a + i]].q0;
+  m.nruns = p.nruns;
+  m.unit = p.unit;
+  int ngroups = bp.rows, rows = 128;
+  if (p.nruns) {
+    std::copy(p.reqs, p.reqs + kBatchReqs, m.reqs);
+    std::copy(bp.runs.begin(), bp.runs.end(), m.runs);
+  } else {
+    ngroups = (int)bp.groups.size();
+    rows = 0;
+    for (int i = 0; i < ngroups; i++) {
+      m.groups[i] = bp.groups[i];
+      m.groups[i].q_row += p.reqs[bp.group_req[i]].q0;
       rows = std::max<int>(rows, m.groups[i].rows);
     }
-    constexpr int kVecs = 256 / (D / 8);
-    hipLaunchKernelGGL((prefill_batch_merge_kernel<D>), dim3((rows * heads + kVecs - 1) / kVecs, n),
+  }
+  constexpr int kVecs = 256 / (D / 8);
+  for (m.y0 = 0; m.y0 < ngroups; m.y0 += kGridRows) {
+    hipLaunchKernelGGL((prefill_batch_merge_kernel<D>),
+                       dim3((rows * heads + kVecs - 1) / kVecs, std::min(kGridRows, ngroups - m.y0)),
                        dim3(256), 0, st, m);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -1127,9 +1260,9 @@ hipError_t launch_batch(const BatchPlan& bp, int heads, hipStream_t st, PrefillB
   return hipSuccess;
 }
 
-// workspace of a plan: O rows, then (max, sum) pairs, of each slot's 128 rows
+// workspace of a plan: O rows, then (max, sum) pairs
 int64_t batch_ws_bytes(const BatchPlan& bp, int heads, int head_dim) {
-  return (int64_t)bp.slots * 128 * heads * (head_dim * 4 + 8);
+  return (int64_t)bp.ws_rows * heads * (head_dim * 4 + 8);
 }
 
 bool batch_sizes_ok(const int32_t* q_lens, const int32_t* kv_lens, int32_t nreq, int32_t heads,
@@ -1235,7 +1368,7 @@ extern "C" int tq_prefill_attention_batch(
     set_error("%s: tensors must be 16-byte aligned", what);
     return kEinval;
   }
-  PrefillBatch p;
+  PrefillBatch p = {};
   p.q = q;
   p.k = static_cast<const _Float16*>(k);
   p.v = static_cast<const _Float16*>(v);
@@ -1267,7 +1400,7 @@ extern "C" int tq_prefill_attention_batch(
         return kEinval;
       }
       p.ws_o = static_cast<float*>(workspace);
-      p.ws_ml = p.ws_o + (int64_t)bp.slots * 128 * num_qo_heads * padded_dim;
+      p.ws_ml = p.ws_o + (int64_t)bp.ws_rows * num_qo_heads * padded_dim;
       for (int i = 0; i < n; i++)
         p.reqs[i] = {q_starts[a + i], q_lens[a + i], kv_starts[a + i], kv_lens[a + i],
                      kv_sources[a + i] ? 1 : 0};
