@@ -170,6 +170,25 @@ def test_cabi_argument_errors_without_gpu():
     assert lib.tq_diag_stream_read(ctypes.c_void_p(256), 0, ctypes.c_void_p(256), null) == 0
 
 
+def test_prefill_batch_workspace_holds_the_rows_of_the_split_blocks():
+    """Shares of a block are as many rows as the block has; whole blocks need
+    none; the query works without a GPU."""
+    lib = _lib.load()
+
+    def need(pairs, heads=32, pd=128):
+        q, kv = ((ctypes.c_int32 * len(pairs))(*c) for c in zip(*pairs))
+        return int(lib.tq_prefill_batch_workspace_bytes(q, kv, len(pairs), heads, pd))
+
+    full = need([(128, 30000)])
+    assert full > 0 and full % (128 * 32 * (128 * 4 + 8)) == 0
+    for rows in (1, 2, 77):
+        assert need([(rows, 30000)]) * 128 == full * rows
+    assert need([(4096, 4096)]) == 0
+    # runs: at one head, shares of the whole prompt at most
+    runs = need([(30000, 30000)], heads=1)
+    assert 0 < runs <= 4 * 30000 * (128 * 4 + 8)
+
+
 def test_missing_library_raises(monkeypatch):
     monkeypatch.setattr(_lib, "_lib", None)
     monkeypatch.setattr(_lib, "LIB_PATH", os.path.join(ROOT, "no_such_dir", "libtq_hip.so"))

@@ -1182,14 +1182,13 @@ BatchPlan plan_batch(const int32_t* q_lens, const int32_t* kv_lens, int nreq, in
     int ns = parts(b.tiles, unit);
     const int per = (b.tiles + ns - 1) / ns;
     ns = (b.tiles + per - 1) / per;
-    const int row0 = bp.ws_rows;
+    const int row0 = bp.ws_rows, rows = std::min(bm, q_lens[b.req] - b.qb * bm);
     for (int z = 0; z < ns; z++)
       bp.items.push_back({(uint32_t)b.req | (uint32_t)b.qb << 6, z * per,
-                          std::min(b.tiles, (z + 1) * per), ns > 1 ? row0 + 128 * z : -1});
+                          std::min(b.tiles, (z + 1) * per), ns > 1 ? row0 + rows * z : -1});
     if (ns > 1) {
-      bp.ws_rows += 128 * ns;
-      bp.groups.push_back({b.qb * bm, row0, 128, (uint16_t)ns,
-                           (uint16_t)std::min(bm, q_lens[b.req] - b.qb * bm)});
+      bp.ws_rows += rows * ns;
+      bp.groups.push_back({b.qb * bm, row0, rows, (uint16_t)ns, (uint16_t)rows});
       bp.group_req.push_back(b.req);
     }
   }
