@@ -145,6 +145,59 @@ def test_gather_against_read_back_and_conversion(hkv, hd, dtype, aligned):
         assert (t[:2] == 7.0).all() and (t[rows:] == 7.0).all()
 
 
+def test_gather_of_more_requests_than_a_launch_takes():
+    """130 requests in one call (64 a launch), against a call for each."""
+    hkv, hd, dev = 2, 64, G.DEV
+    ctxs, fresh = [(7 * i) % 50 for i in range(130)], [(5 * i) % 9 for i in range(130)]
+    c = W.decode_case(5, len(ctxs), [max(1, x) for x in ctxs], hkv, hkv, hd)
+    cache, pd = G.build_cache(c)
+    table, signs = torch.from_numpy(c["block_table"]).to(dev), hadamard_signs(pd, dev)
+    g = torch.Generator("cuda").manual_seed(3)
+    key, value = (torch.randn((sum(fresh), hkv, hd), generator=g, device=dev).to(torch.bfloat16)
+                  for _ in range(2))
+    reqs = [(i, n, sum(fresh[:i]), f, sum(ctxs[:i]) + sum(fresh[:i]))
+            for i, (n, f) in enumerate(zip(ctxs, fresh))]
+    out = [torch.full((sum(ctxs) + sum(fresh), hkv, pd), 7.0, dtype=torch.float16, device=dev)
+           for _ in range(4)]
+    ops.prefill_gather(cache, table, key, value, reqs, hd, pd, signs, *out[:2])
+    for r in reqs:
+        ops.prefill_gather(cache, table, key, value, [r], hd, pd, signs, *out[2:])
+    assert torch.equal(out[0], out[2]) and torch.equal(out[1], out[3])
+    assert not (out[0] == 7.0).all(-1).any()
+
+
+def test_forward_in_passes_of_bounded_rows(monkeypatch):
+    """A step whose gathered rows exceed the bound goes in several passes: the
+    same result.  (Few key tiles, so no block is split in either.)"""
+    from types import SimpleNamespace
+
+    from turboquant_amd import vllm_backend_fused as B
+    hq, hkv, hd, dev = 4, 2, 128, G.DEV
+    reqs = [(40, 100), (3, 300), (130, 0), (2, 17), (60, 250), (1, 90), (200, 30)]
+    lens = [a + b for a, b in reqs]
+    c = W.decode_case(9, len(reqs), lens, hq, hkv, hd)
+    cache, pd = G.build_cache(c)
+    n = sum(r[0] for r in reqs)
+    starts = [sum(r[0] for r in reqs[:i]) for i in range(len(reqs) + 1)]
+    i32 = lambda v, d: torch.tensor(v, dtype=torch.int32, device=d)
+    meta = SimpleNamespace(
+        max_query_len=200, num_actual_tokens=n,
+        block_table=torch.from_numpy(c["block_table"]).to(dev), slot_mapping=None,
+        seq_lens=i32(lens, dev), seq_lens_cpu=i32(lens, "cpu"),
+        query_start_loc=i32(starts, dev), query_start_loc_cpu=i32(starts, "cpu"))
+    g = torch.Generator("cuda").manual_seed(4)
+    for dtype in (torch.float16, torch.bfloat16):
+        q, k, v = (torch.randn((n, h * hd), generator=g, device=dev).to(dtype)
+                   for h in (hq, hkv, hkv))
+        impl = B.TurboQuantFusedImpl(hq, hd, 1.0 / math.sqrt(hd), hkv, None, None, "fp8")
+        run = lambda: impl.forward(None, q, k, v, cache, meta, output=torch.empty_like(q)).clone()
+        monkeypatch.undo()
+        want = run()
+        for rows in (1, 140, 500):  # a request a pass, then several
+            monkeypatch.setattr(B, "GATHER_BYTES", rows * 4 * hkv * pd)
+            assert torch.equal(run(), want), (dtype, rows)
+
+
 def test_batch_refuses_what_it_cannot_read():
     q = torch.zeros((8, 4, 64), dtype=torch.float16, device=G.DEV)
     k = torch.zeros((8, 2, 64), dtype=torch.float16, device=G.DEV)

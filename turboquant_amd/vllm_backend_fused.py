@@ -121,6 +121,11 @@ class TurboQuantBackend(FlashAttentionBackend):
         return None
 
 
+# Gathered K and V of one prefill pass (_attend_chunks): enough requests to
+# fill a launch, and a bound that does not grow with the step or the head size.
+GATHER_BYTES = 1 << 29
+
+
 class TurboQuantMetadataBuilder(FlashAttentionMetadataBuilder):
     pass
 
@@ -332,15 +337,16 @@ class TurboQuantFusedImpl(FlashAttentionImpl):
         in_place = d == pd and rows_ok(key, half[:1]) and rows_ok(value, half[:1]) \
             and min(key.stride(0), value.stride(0)) >= pd
         kv = (key, value) if in_place else (None, None)
+        most = GATHER_BYTES // (4 * hkv * pd)  # rows of K and V
         at = 0
         while at < len(chunks):
-            # the gathered rows of a launch are bounded (1 GB at 8 heads of 128),
-            # one chunk's alone may be more
+            # the requests of a pass: gathered K and V up to GATHER_BYTES, one
+            # request's alone may be more
             reqs, gathers, rows = [], [], 0
             while at < len(chunks):
                 i, a, ql, ctx = chunks[at]
                 if ctx > 0 or not in_place:
-                    if gathers and rows + ctx + ql > 1 << 18:
+                    if gathers and rows + ctx + ql > most:
                         break
                     gathers.append((i, ctx, a, ql, rows))
                     reqs.append((a, ql, rows, ctx + ql, 1))
