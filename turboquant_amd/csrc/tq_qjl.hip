@@ -46,8 +46,7 @@ typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kBK = 32;   // K step: 64 bytes of a row
-constexpr int kCus = 256;  // compute units of the card
+constexpr int kBK = 32;  // K step: 64 bytes of a row
 
 struct QjlGemmParams {
   const _Float16* xh;   // quantize: residual halves [n][ldk]
@@ -527,8 +526,9 @@ hipError_t launch_qjl(bool quant, const _Float16* xh, const _Float16* xl, const 
   // against 22.0), 5 for the dequantize, more of which fit a CU (dim 1000, n =
   // 2500 31.5 against 43.0, n = 4096 41.3 against 45.8; dim 256, n = 12000 20.8
   // against 23.6; dim 1000, n = 8192 72 against 61).
+  const int64_t cus = device_cus() > 0 ? device_cus() : 256;
   const int64_t t32 = (n + 31) / 32 * ((dim + 31) / 32);
-  if (quant && t32 <= kCus) {
+  if (quant && t32 <= cus) {
     if (dim > 256)
       hipLaunchKernelGGL((qjl_signs_small_kernel<8>), dim3((unsigned)t32), dim3(512), 0, st, p);
     else
@@ -536,7 +536,7 @@ hipError_t launch_qjl(bool quant, const _Float16* xh, const _Float16* xl, const 
     return hipGetLastError();
   }
   const int64_t t64 = (n + 63) / 64 * ((dim + 63) / 64);
-  const int bt = t64 <= (quant ? 5 : 10) * kCus / 2 ? 64 : 128;
+  const int bt = t64 <= (quant ? 5 : 10) * cus / 2 ? 64 : 128;
   p.ntn = (dim + bt - 1) / bt;
   p.tiles = (n + bt - 1) / bt * p.ntn;
   const int64_t grid = (p.tiles + 7) / 8 * 8;
