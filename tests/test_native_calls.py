@@ -8,7 +8,7 @@ import torch
 
 from turboquant_amd import _lib, ops
 from turboquant_amd import workloads as W
-from turboquant_amd.geometry import hadamard_signs
+from turboquant_amd.geometry import entry_bytes, hadamard_signs
 
 
 def test_cpu_tensors_are_left_to_the_checks():
@@ -83,3 +83,49 @@ def test_calls_run_on_the_current_stream():
             got = ops.mse_quantize(y, 128, 4, s, b)[0]
         side.synchronize()
         assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
+def test_strided_slots_and_signs_are_read_by_their_strides():
+    """A column of a table of slots, and every other value of a longer table of
+    signs, give what their packed copies give."""
+    g = torch.Generator("cuda").manual_seed(5)
+    hkv, hd, pd, n = 2, 96, 128, 37
+    key, value = (torch.randn((n, hkv, hd), generator=g, device="cuda").half() for _ in range(2))
+    table = torch.randperm(64 * 3, generator=g, device="cuda").to(torch.int32).view(64, 3)
+    slots = table[:n, 1]
+    signs = hadamard_signs(2 * pd, "cuda")[::2]
+    assert not slots.is_contiguous() and not signs.is_contiguous()
+    ops.register_ops()
+    ebs = entry_bytes(hd)[2]
+    caches = [torch.zeros((2, 12, 16, hkv, ebs), dtype=torch.uint8, device="cuda")
+              for _ in range(3)]
+    packed = (signs.contiguous(), slots.contiguous())
+    ops.quantize_write_kv_cache(caches[0], key, value, *packed, hd, pd)
+    ops.quantize_write_kv_cache(caches[1], key, value, signs, slots, hd, pd)
+    torch.ops.turboquant_write.quantize_write_kv_cache(caches[2], key, value, signs, slots, hd, pd)
+    assert torch.equal(caches[0], caches[1]) and torch.equal(caches[0], caches[2])
+    outs = []
+    pages = torch.arange(12, dtype=torch.int32, device="cuda")
+    for s in (packed[0], signs):
+        k, v = (torch.zeros((192, hkv, hd), dtype=torch.float16, device="cuda") for _ in range(2))
+        ops.dequant_paged(caches[0], pages, 192, hkv, hd, pd, s, k, v)
+        gk, gv = (torch.zeros((197, hkv, pd), dtype=torch.float16, device="cuda")
+                  for _ in range(2))
+        ops.prefill_gather(caches[0], pages[None], key, value, [(0, 192, 0, 5, 0)], hd, pd, s, gk,
+                           gv)
+        q = torch.randn((1, 4, pd), generator=torch.Generator("cuda").manual_seed(1),
+                        device="cuda").half()
+        i32 = lambda *x: torch.tensor(x, dtype=torch.int32, device="cuda")
+        o = torch.zeros_like(q)
+        rows = ops.balanced_rows(1, 4, hkv, pd)
+        ops.decode_paged_balanced(q, caches[0], pages, i32(0, 12), i32(192), hkv, hd, pd, 0.1, s,
+                                  o, torch.empty((rows, 4, pd), device="cuda"),
+                                  torch.empty((rows, 4), device="cuda"), i32(0, 0, 0))
+        o2 = torch.zeros_like(q)
+        ops.decode_paged_splitkv(q, caches[0], pages, i32(0, 12), i32(192), hkv, hd, pd, 0.1, s,
+                                 o2, torch.empty((2, 4, pd), device="cuda"),
+                                 torch.empty((2, 4), device="cuda"), 2, 96)
+        outs.append((k, v, gk, gv, o, o2))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)

@@ -82,11 +82,11 @@ bool cache_of(const Tensor& t, c10::Device dev, Cache& c) {
   return true;
 }
 
-// signs fp32 [>= padded_dim], or none
+// signs fp32 [>= padded_dim] contiguous, or none
 bool signs_of(const OptTensor& t, int64_t padded_dim, c10::Device dev, const float*& p) {
   p = nullptr;
   if (!t.has_value() || t->numel() == 0) return true;
-  if (!on(*t, dev) || t->scalar_type() != at::kFloat || t->numel() < padded_dim) return false;
+  if (!is_f32(*t, dev) || t->numel() < padded_dim) return false;
   p = cptr<float>(*t);
   return true;
 }
@@ -98,8 +98,8 @@ bool write_cache(const Tensor& kv_cache, const Tensor& key, const Tensor& value,
   Cache c;
   const float* sp = nullptr;
   if (!cache_of(kv_cache, dev, c) || c.ebs % 16 != 0 || !on(key, dev) || !on(value, dev) ||
-      !on(slots, dev) || slots.scalar_type() != at::kInt || key.dim() != 3 ||
-      value.sizes() != key.sizes() || value.scalar_type() != key.scalar_type() ||
+      !is_i32(slots, dev) || key.dim() != 3 || value.sizes() != key.sizes() ||
+      value.scalar_type() != key.scalar_type() ||
       dtype_code(key.scalar_type()) < 0 || key.size(2) < head_dim || key.stride(2) != 1 ||
       value.stride(2) != 1 || key.size(1) != c.heads || !signs_of(signs, padded_dim, dev, sp) || !sp)
     return false;

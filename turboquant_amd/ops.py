@@ -110,6 +110,8 @@ def quantize_write_kv_cache(kv_cache: torch.Tensor, key: torch.Tensor, value: to
     _, nb, bs, h, _ = kv_cache.shape
     if key.size(1) != h:
         raise RuntimeError(f"key has {key.size(1)} heads, cache has {h}")
+    # the kernel reads both by address
+    signs, slot_mapping = signs.contiguous(), slot_mapping.contiguous()
     lib = _lib.load()
     base = kv_cache.data_ptr()
     slab = nb * bs * h * ebs
@@ -157,6 +159,7 @@ def decode_paged_splitkv(q: torch.Tensor, kv_cache: torch.Tensor, indices: torch
         if signs.dtype != torch.float32 or signs.numel() < pd:
             raise RuntimeError("hadamard_signs must be fp32 [padded_dim]")
         _require_gpu(q, signs)
+        signs = signs.contiguous()
         sp = signs.data_ptr()
     lib = _lib.load()
     base = kv_cache.data_ptr()
@@ -273,6 +276,7 @@ def _decode_balanced(q, kv_cache, indices, indptr, seq_lens, num_kv_heads, head_
         if signs.dtype != torch.float32 or signs.numel() < pd:
             raise RuntimeError("hadamard_signs must be fp32 [padded_dim]")
         _require_gpu(q, signs)
+        signs = signs.contiguous()
         sp = signs.data_ptr()
     lib = _lib.load()
     base = kv_cache.data_ptr()
@@ -411,6 +415,7 @@ def dequant_paged(kv_cache: torch.Tensor, pages: torch.Tensor, num_tokens: int,
         if signs.dtype != torch.float32 or signs.numel() < padded_dim:
             raise RuntimeError("signs must be fp32 [padded_dim]")
         _require_gpu(kv_cache, signs)
+        signs = signs.contiguous()
         sp = signs.data_ptr()
     lib = _lib.load()
     base = kv_cache.data_ptr()
@@ -478,6 +483,7 @@ def prefill_gather(kv_cache: torch.Tensor | None, block_table: torch.Tensor | No
         if signs.dtype != torch.float32 or signs.numel() < padded_dim:
             raise RuntimeError("signs must be fp32 [padded_dim]")
         _require_gpu(key, signs)
+        signs = signs.contiguous()
         sp = signs.data_ptr()
     n = len(requests)
     if n == 0:
