@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define TQ_ABI_VERSION 11 /* what tq_abi_version() returns */
+#define TQ_ABI_VERSION 12 /* what tq_abi_version() returns */
 
 typedef struct ihipStream_t* tq_stream_t; /* == hipStream_t */
 
@@ -406,10 +406,28 @@ int tq_prod_dequantize_qjl(const uint8_t* packed, const float* norms, const int8
                            float* out, tq_stream_t stream);
 
 /*
- * The operand halves of the calls above from the QJL matrix S fp32
- * [dim, dim]: `halves` receives fp16 [4][padded_dim][padded_dim], S hi, S lo,
- * S^T hi, S^T lo (hi + lo = S to 22 bits), zero past dim.  padded_dim a power
- * of two 64..1024.
+ * The same two calls from the QJL matrix itself, s fp32 [dim, dim] row-major
+ * (16-byte aligned) for both: the kernels make its halves (the same bits) as
+ * they load it, so nothing derived from S outlives the call.
+ */
+int tq_prod_quantize_qjl_matrix(const float* x, int64_t num_vectors, int32_t dim,
+                                int32_t padded_dim, int32_t mse_bit_width, const float* signs,
+                                const float* boundaries, const float* centroids, const float* s,
+                                uint8_t* packed, float* norms, int8_t* qjl_signs,
+                                float* residual_norms, tq_stream_t stream);
+int tq_prod_dequantize_qjl_matrix(const uint8_t* packed, const float* norms,
+                                  const int8_t* qjl_signs, const float* residual_norms,
+                                  int64_t num_vectors, int32_t dim, int32_t padded_dim,
+                                  int32_t mse_bit_width, const float* signs,
+                                  const float* centroids, const float* s, float* out,
+                                  tq_stream_t stream);
+
+/*
+ * The operand halves of tq_prod_quantize_qjl / tq_prod_dequantize_qjl from the
+ * QJL matrix S fp32 [dim, dim]: `halves` receives fp16
+ * [4][padded_dim][padded_dim], S hi, S lo, S^T hi, S^T lo (hi + lo = S to 22
+ * bits, to 2^-25 where |S| < 2^-3), zero past dim.  padded_dim a power of two
+ * 64..1024.
  */
 int tq_qjl_halves(const float* s, int32_t dim, int32_t padded_dim, void* halves,
                   tq_stream_t stream);

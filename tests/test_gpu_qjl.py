@@ -66,6 +66,32 @@ def test_fused_signs_against_64_bits(dim, n):
     assert bool((proj.abs() <= bound)[wrong].all()), proj[wrong].abs().max().item()
 
 
+@pytest.mark.parametrize("dim,n", [(33, 5), (50, 33), (64, 1), (66, 40), (97, 65), (100, 31),
+                                   (128, 1), (128, 40003)])
+@pytest.mark.parametrize("scale", [1.0, 1e-6, 1e4])
+def test_matrix_and_its_halves_give_the_same_bits(dim, n, scale):
+    """Up to padded size 128 the kernels split S as they load it: what the calls
+    with halves made beforehand give, also where S is not aligned."""
+    bits = 2 + dim % 4
+    q, x, pd, (bnd, cen) = _prod(dim, bits, n)
+    q.qjl.S *= scale
+    sh, sl, th, tl = q.qjl.halves(pd)
+    args = (x, pd, bits - 1, q.mse.rotation.signs, bnd, cen)
+    want = ops.prod_quantize_qjl(*args, sh, sl)
+    back = (dim, pd, bits - 1, q.mse.rotation.signs, cen)
+    off = torch.empty(dim * dim + 1, device="cuda")[1:].view(dim, dim).copy_(q.qjl.S)
+    for s in (q.qjl.S, off, q.qjl.S.t().contiguous().t()):
+        for a, b in zip(ops.prod_quantize_qjl_matrix(*args, s), want):
+            assert torch.equal(a, b)
+        assert torch.equal(ops.prod_dequantize_qjl_matrix(*want, *back, s),
+                           ops.prod_dequantize_qjl(*want, *back, th, tl))
+    assert torch.equal(q.quantize(x)[2], want[2])
+    with pytest.raises(RuntimeError):
+        ops.prod_quantize_qjl_matrix(*args, q.qjl.S[:-1, :-1].contiguous())
+    with pytest.raises(RuntimeError):
+        ops.prod_dequantize_qjl_matrix(*want, *back, q.qjl.S.double())
+
+
 @pytest.mark.parametrize("dim,n", SHAPES)
 def test_dequantize_term_against_64_bits(dim, n):
     """z S alone: norms of zero and a weight of 1, with signs and with any

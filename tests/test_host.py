@@ -407,6 +407,16 @@ def test_prod_entry_points_refuse_bad_arguments():
     assert b"null pointer" in lib.tq_last_error()
     assert lib.tq_prod_dequantize_qjl(one, one, one, one, 0, 128, 128, 3, one, tab, one, one,
                                       one, null) == 0
+    # from the matrix itself: the same checks
+    assert lib.tq_prod_quantize_qjl_matrix(one, 4, 128, 128, 3, one, tab, tab, null, one, one, one,
+                                           one, null) == -22
+    assert b"null pointer" in lib.tq_last_error()
+    assert lib.tq_prod_dequantize_qjl_matrix(one, one, one, one, 4, 200, 256, 3, one, tab, one, one,
+                                             null) == -22
+    assert b"padded_dim" in lib.tq_last_error()
+    assert lib.tq_prod_dequantize_qjl_matrix(one, one, one, one, 4, 128, 128, 3, one, tab,
+                                             ctypes.c_void_p(24), one, null) == -22
+    assert b"16-byte aligned" in lib.tq_last_error()
     # qjl_signs rows are read and written in 4- and 8-byte pieces: the base
     # must be 8-byte aligned
     odd = ctypes.c_void_p(20)

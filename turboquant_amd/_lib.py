@@ -68,6 +68,10 @@ SIGNATURES = {
                                     _P, _P]),
     "tq_prod_dequantize_qjl": (_I32, [_P, _P, _P, _P, _I64, _I32, _I32, _I32, _P, _P, _P, _P,
                                       _P, _P]),
+    "tq_prod_quantize_qjl_matrix": (_I32, [_P, _I64, _I32, _I32, _I32, _P, _P, _P, _P, _P, _P,
+                                           _P, _P, _P]),
+    "tq_prod_dequantize_qjl_matrix": (_I32, [_P, _P, _P, _P, _I64, _I32, _I32, _I32, _P, _P, _P,
+                                             _P, _P]),
     "tq_qjl_halves": (_I32, [_P, _I32, _I32, _P, _P]),
     "tq_qjl_operand": (_I32, [_P, _I32, _I32, _I32, _P, _P, _P]),
     "tq_prod_workspace_bytes": (_I64, [_I64, _I32]),
@@ -83,7 +87,7 @@ SIGNATURES = {
     "tq_last_error": (ctypes.c_char_p, []),
     "tq_abi_version": (_I32, []),
 }
-ABI_VERSION = 11
+ABI_VERSION = 12
 
 _lib = None
 

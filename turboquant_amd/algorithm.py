@@ -259,6 +259,13 @@ class TurboQuantProd:
         self.mse = TurboQuantMSE(dim, bit_width - 1, device=device, seed=seed)
         self.qjl = QJL(dim, device=device, seed=seed + 10000)
 
+    def _qjl_matrix(self, dim: int):
+        """S where the kernels up to padded size 128 take it as it is (fp32, of
+        the vectors' `dim`), else None: they take its halves."""
+        s = self.qjl.S
+        return s if s.dtype == torch.float32 and tuple(s.shape) == (dim, dim) == (
+            self.dim, self.dim) else None
+
     def _qjl_operand(self, dim: int, transposed: bool):
         """(hi, lo, scale) of S or S^T above padded size 128, for vectors of
         `dim`: what the fp32 product with S refuses is refused.  Made from S
@@ -275,7 +282,7 @@ class TurboQuantProd:
         """-> (mse_packed, mse_norms, qjl_signs int8 {-1, +1}, residual_norms).
         fp32 vectors on a GPU take HIP kernels: up to padded size 128 the
         whole algorithm in one, with the QJL product on the matrix cores
-        (tq_prod_quantize_qjl); above it the MSE stage, its read-back and the
+        (tq_prod_quantize_qjl_matrix); above it the MSE stage, its read-back and the
         unit residual, followed by the QJL product on the matrix cores
         (tq_prod_quantize_qjl_ws)."""
         if x.dtype == torch.float32 and self.mse._hip(x):
@@ -283,9 +290,11 @@ class TurboQuantProd:
             bnd, cen = self.mse._host_tables()
             pd = self.mse.rotation.padded_dim
             if pd <= 128:  # QJL product fused on the matrix cores
-                sh, sl, _, _ = self.qjl.halves(pd)
-                return ops.prod_quantize_qjl(x, pd, self.mse.bit_width, self.mse.rotation.signs,
-                                             bnd, cen, sh, sl)
+                args = (x, pd, self.mse.bit_width, self.mse.rotation.signs, bnd, cen)
+                s = self._qjl_matrix(x.shape[-1])
+                if s is not None:
+                    return ops.prod_quantize_qjl_matrix(*args, s)
+                return ops.prod_quantize_qjl(*args, *self.qjl.halves(pd)[:2])
             sh, sl, _ = self._qjl_operand(x.shape[-1], False)
             return ops.prod_quantize_qjl_ws(x, pd, self.mse.bit_width, self.mse.rotation.signs,
                                             bnd, cen, sh, sl)
@@ -297,17 +306,18 @@ class TurboQuantProd:
     @torch.no_grad()
     def dequantize(self, mse_packed, mse_norms, qjl_signs, residual_norms) -> torch.Tensor:
         """The inverse of quantize; int8 signs on a GPU take the HIP kernels
-        (tq_prod_dequantize_qjl up to padded size 128, the _ws form above),
+        (tq_prod_dequantize_qjl_matrix up to padded size 128, the _ws form above),
         which give a vector the same bits in a batch of any size."""
         if self.mse._hip(mse_packed) and mse_norms.dtype == torch.float32:
             from . import ops
             pd = self.mse.rotation.padded_dim
             if pd <= 128 and qjl_signs.dtype == torch.int8:
-                _, _, th, tl = self.qjl.halves(pd)
-                return ops.prod_dequantize_qjl(mse_packed, mse_norms, qjl_signs, residual_norms,
-                                               self.dim, pd, self.mse.bit_width,
-                                               self.mse.rotation.signs,
-                                               self.mse._host_tables()[1], th, tl)
+                args = (mse_packed, mse_norms, qjl_signs, residual_norms, self.dim, pd,
+                        self.mse.bit_width, self.mse.rotation.signs, self.mse._host_tables()[1])
+                s = self._qjl_matrix(self.dim)
+                if s is not None:
+                    return ops.prod_dequantize_qjl_matrix(*args, s)
+                return ops.prod_dequantize_qjl(*args, *self.qjl.halves(pd)[2:])
             if qjl_signs.dtype == torch.int8:
                 th, tl, scale = self._qjl_operand(self.dim, True)
                 return ops.prod_dequantize_qjl_ws(mse_packed, mse_norms, qjl_signs,

@@ -714,6 +714,7 @@ __global__ __launch_bounds__(kMseThreads) void mse_dequantize_kernel(MseParams p
 // l % 16, outputs 4 (l / 16) + e.
 // --------------------------------------------------------------------------
 struct QjlParams {
+  const float* s;        // S [dim][dim] row-major, or null and its halves:
   const _Float16* s_hi;  // [PD][PD] row-major: quantize S, dequantize S^T
   const _Float16* s_lo;
   int8_t* z;             // quantize out: +-1 [n][dim]
@@ -744,6 +745,46 @@ __device__ __forceinline__ void load_s_frags(const QjlParams& q, int w, int lane
     }
 }
 
+// The same blocks of S (TR: of S^T) from S itself, split as split_halves_kernel
+// does.  A launch loads them once per persistent workgroup, 64 KB at dim 128
+// either way, so this takes the place of the launch that makes the halves where
+// they cannot be kept from one call to the next (quantize and dequantize of 16
+// vectors of dim 128 from Python, one after the other: 16.2 us, 29.1 with halves
+// made in each call; 150,001 vectors 91 and 95.5).
+template <int PD, bool TR>
+__device__ __forceinline__ void split_s_frags(const float* s, int dim, int w, int lane,
+                                              half8_t (&ah)[QjlGeom<PD>::NRB][QjlGeom<PD>::NKS],
+                                              half8_t (&al)[QjlGeom<PD>::NRB][QjlGeom<PD>::NKS]) {
+  using QG = QjlGeom<PD>;
+#pragma unroll
+  for (int rb = 0; rb < QG::NRB; rb++)
+#pragma unroll
+    for (int ks = 0; ks < QG::NKS; ks++) {
+      const int r = 16 * (QG::NRB * w + rb) + (lane & 15), k = 32 * ks + 8 * (lane >> 4);
+      float f[8];
+      if (!TR && (dim & 3) == 0) {  // rows in whole aligned float4 pieces
+#pragma unroll
+        for (int i = 0; i < 8; i += 4) {
+          float4 t = {0.0f, 0.0f, 0.0f, 0.0f};
+          if (r < dim && k + i < dim) t = *reinterpret_cast<const float4*>(s + r * dim + k + i);
+          f[i] = t.x;
+          f[i + 1] = t.y;
+          f[i + 2] = t.z;
+          f[i + 3] = t.w;
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+          f[e] = r < dim && k + e < dim ? s[TR ? (k + e) * dim + r : r * dim + k + e] : 0.0f;
+      }
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        ah[rb][ks][e] = (_Float16)f[e];
+        al[rb][ks][e] = (_Float16)(f[e] - (float)ah[rb][ks][e]);
+      }
+    }
+}
+
 template <int PD, int BITS>
 __global__ __launch_bounds__(kMseThreads) __attribute__((amdgpu_waves_per_eu(PD == 128 ? 3 : 4)))
 void prod_qjl_quantize_kernel(MseParams p, QjlParams q) {
@@ -766,7 +807,8 @@ void prod_qjl_quantize_kernel(MseParams p, QjlParams q) {
   half8_t ah[QG::NRB][QG::NKS];
   {
     half8_t al[QG::NRB][QG::NKS];
-    load_s_frags<PD>(q, w, lane, ah, al);
+    if (q.s) split_s_frags<PD, false>(q.s, p.dim, w, lane, ah, al);
+    else load_s_frags<PD>(q, w, lane, ah, al);
 #pragma unroll
     for (int rb = 0; rb < QG::NRB; rb++)
 #pragma unroll
@@ -841,7 +883,8 @@ void prod_qjl_dequantize_kernel(MseParams p,
   if (threadIdx.x < 16) cen[threadIdx.x] = p.table[threadIdx.x];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, sub = lane % P, vl = threadIdx.x / P;
   half8_t ah[QG::NRB][QG::NKS], al[QG::NRB][QG::NKS];
-  load_s_frags<PD>(q, w, lane, ah, al);  // S^T rows
+  if (q.s) split_s_frags<PD, true>(q.s, p.dim, w, lane, ah, al);  // S^T rows
+  else load_s_frags<PD>(q, w, lane, ah, al);
   // the QJL signs of a batch as B fragments: lane (vector l % 16 of column
   // block cb, dims 32 ks + 8 (l / 16) ..) holds 8 signs, 0 past dim or n
   auto load_z = [&](int64_t bt, uint2 (&zb)[2][QG::NKS]) {
@@ -1112,8 +1155,8 @@ int mse_call(bool quant, const float* x, uint8_t* packed, float* norms, float* o
 // TurboQuantProd with the QJL projections fused (padded size 64 or 128).
 int prod_qjl_call(bool quant, const float* x, uint8_t* packed, float* norms, float* out,
                   int64_t n, int32_t dim, int32_t padded_dim, int32_t bits, const float* signs,
-                  const float* table, const float* centroids, const _Float16* s_hi,
-                  const _Float16* s_lo, int8_t* z, const int8_t* zin, float* rnorm,
+                  const float* table, const float* centroids, const float* s, const void* s_hi,
+                  const void* s_lo, int8_t* z, const int8_t* zin, float* rnorm,
                   const float* gamma, tq_stream_t stream) {
   const char* what = quant ? "prod_quantize_qjl" : "prod_dequantize_qjl";
   if (padded_dim != 64 && padded_dim != 128) {
@@ -1133,16 +1176,17 @@ int prod_qjl_call(bool quant, const float* x, uint8_t* packed, float* norms, flo
     set_error("%s: vector count %lld out of range", what, (long long)n);
     return kEinval;
   }
-  if (!packed || !norms || !signs || !table || !s_hi || !s_lo ||
+  if (!packed || !norms || !signs || !table || (!s && (!s_hi || !s_lo)) ||
       (quant ? (!x || !centroids || !z || !rnorm) : (!out || !zin || !gamma))) {
     set_error("%s: null pointer", what);
     return kEinval;
   }
   if (n == 0) return 0;
   const uintptr_t al = (uintptr_t)(quant ? (const void*)x : (const void*)out) |
-                       (uintptr_t)packed | (uintptr_t)s_hi | (uintptr_t)s_lo | (uintptr_t)signs;
+                       (uintptr_t)packed | (uintptr_t)s | (uintptr_t)s_hi | (uintptr_t)s_lo |
+                       (uintptr_t)signs;
   if ((al & 15) != 0) {
-    set_error("%s: x / out, packed, signs and the S halves must be 16-byte aligned", what);
+    set_error("%s: x / out, packed, signs and S or its halves must be 16-byte aligned", what);
     return kEinval;
   }
   if ((((uintptr_t)z | (uintptr_t)zin) & 7) != 0) {
@@ -1176,8 +1220,9 @@ int prod_qjl_call(bool quant, const float* x, uint8_t* packed, float* norms, flo
   p.bin_base = 0;
   if (quant) build_bins(table, bits, p);
   QjlParams q;
-  q.s_hi = s_hi;
-  q.s_lo = s_lo;
+  q.s = s;
+  q.s_hi = static_cast<const _Float16*>(s_hi);
+  q.s_lo = static_cast<const _Float16*>(s_lo);
   q.z = z;
   q.zin = zin;
   q.nbatch = (n + 31) / 32;
@@ -1285,8 +1330,18 @@ extern "C" int tq_prod_quantize_qjl(const float* x, int64_t num_vectors, int32_t
                                     float* norms, int8_t* qjl_signs, float* residual_norms,
                                     tq_stream_t stream) {
   return tq::prod_qjl_call(true, x, packed, norms, nullptr, num_vectors, dim, padded_dim,
-                           mse_bit_width, signs, boundaries, centroids,
-                           static_cast<const _Float16*>(s_hi), static_cast<const _Float16*>(s_lo),
+                           mse_bit_width, signs, boundaries, centroids, nullptr, s_hi, s_lo,
+                           qjl_signs, nullptr, residual_norms, nullptr, stream);
+}
+
+extern "C" int tq_prod_quantize_qjl_matrix(const float* x, int64_t num_vectors, int32_t dim,
+                                           int32_t padded_dim, int32_t mse_bit_width,
+                                           const float* signs, const float* boundaries,
+                                           const float* centroids, const float* s, uint8_t* packed,
+                                           float* norms, int8_t* qjl_signs, float* residual_norms,
+                                           tq_stream_t stream) {
+  return tq::prod_qjl_call(true, x, packed, norms, nullptr, num_vectors, dim, padded_dim,
+                           mse_bit_width, signs, boundaries, centroids, s, nullptr, nullptr,
                            qjl_signs, nullptr, residual_norms, nullptr, stream);
 }
 
@@ -1298,9 +1353,20 @@ extern "C" int tq_prod_dequantize_qjl(const uint8_t* packed, const float* norms,
                                       const void* st_lo, float* out, tq_stream_t stream) {
   return tq::prod_qjl_call(false, nullptr, const_cast<uint8_t*>(packed),
                            const_cast<float*>(norms), out, num_vectors, dim, padded_dim,
-                           mse_bit_width, signs, centroids, nullptr,
-                           static_cast<const _Float16*>(st_hi), static_cast<const _Float16*>(st_lo),
+                           mse_bit_width, signs, centroids, nullptr, nullptr, st_hi, st_lo,
                            nullptr, qjl_signs, nullptr, residual_norms, stream);
+}
+
+extern "C" int tq_prod_dequantize_qjl_matrix(const uint8_t* packed, const float* norms,
+                                             const int8_t* qjl_signs, const float* residual_norms,
+                                             int64_t num_vectors, int32_t dim, int32_t padded_dim,
+                                             int32_t mse_bit_width, const float* signs,
+                                             const float* centroids, const float* s, float* out,
+                                             tq_stream_t stream) {
+  return tq::prod_qjl_call(false, nullptr, const_cast<uint8_t*>(packed),
+                           const_cast<float*>(norms), out, num_vectors, dim, padded_dim,
+                           mse_bit_width, signs, centroids, nullptr, s, nullptr, nullptr, nullptr,
+                           qjl_signs, nullptr, residual_norms, stream);
 }
 
 namespace tq {

@@ -371,15 +371,23 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> qjl_operand(const Tensor& s, i
   return std::make_tuple(out.select(0, 0), out.select(0, 1), scale);
 }
 
-// ops.prod_quantize_qjl (large: prod_quantize_qjl_ws)
+// the QJL matrix fp32 [dim, dim], or (lo given) its halves
+bool matrix_or_halves(const Tensor& s, const OptTensor& lo, int64_t dim, int64_t padded_dim,
+                      bool large, c10::Device dev) {
+  if (lo.has_value()) return halves(s, padded_dim, dev) && halves(*lo, padded_dim, dev);
+  return !large && is_f32(s, dev) && s.dim() == 2 && s.size(0) == dim && s.size(1) == dim &&
+         aligned(s, 16);
+}
+
+// ops.prod_quantize_qjl (large: prod_quantize_qjl_ws; without s_lo: prod_quantize_qjl_matrix)
 ProdCodes prod_quantize_qjl(const Tensor& x, int64_t padded_dim, int64_t bits, const Tensor& signs,
                             const std::vector<double>& boundaries,
                             const std::vector<double>& centroids, const Tensor& s_hi,
-                            const Tensor& s_lo, bool large) {
+                            const OptTensor& s_lo, bool large) {
   const c10::Device dev = x.device();
   const int64_t per = codes_per_byte(bits);
   if (!vectors(x, dev) || per == 0 || !is_f32(signs, dev) || signs.numel() < padded_dim ||
-      !aligned(signs, 16) || !halves(s_hi, padded_dim, dev) || !halves(s_lo, padded_dim, dev) ||
+      !aligned(signs, 16) || !matrix_or_halves(s_hi, s_lo, x.size(-1), padded_dim, large, dev) ||
       (int64_t)boundaries.size() != (1 << bits) - 1 || (int64_t)centroids.size() != (1 << bits))
     return std::nullopt;
   const int64_t dim = x.size(-1), n = x.numel() / dim;
@@ -398,23 +406,28 @@ ProdCodes prod_quantize_qjl(const Tensor& x, int64_t padded_dim, int64_t bits, c
       large ? tq_prod_quantize_qjl_ws(
                   cptr<float>(x), n, dim, padded_dim, bits,
                   cptr<float>(signs), b.data(), c.data(), s_hi.const_data_ptr(),
-                  s_lo.const_data_ptr(), packed.data_ptr<uint8_t>(), norms.data_ptr<float>(),
+                  s_lo->const_data_ptr(), packed.data_ptr<uint8_t>(), norms.data_ptr<float>(),
                   z.data_ptr<int8_t>(), rnorm.data_ptr<float>(),
                   bytes > 0 ? ws.data_ptr() : nullptr, bytes, stream_of(dev))
-            : tq_prod_quantize_qjl(cptr<float>(x), n, dim, padded_dim, bits,
-                                   cptr<float>(signs), b.data(), c.data(),
-                                   s_hi.const_data_ptr(), s_lo.const_data_ptr(),
-                                   packed.data_ptr<uint8_t>(), norms.data_ptr<float>(),
-                                   z.data_ptr<int8_t>(), rnorm.data_ptr<float>(), stream_of(dev));
+      : s_lo.has_value()
+          ? tq_prod_quantize_qjl(cptr<float>(x), n, dim, padded_dim, bits, cptr<float>(signs),
+                                 b.data(), c.data(), s_hi.const_data_ptr(), s_lo->const_data_ptr(),
+                                 packed.data_ptr<uint8_t>(), norms.data_ptr<float>(),
+                                 z.data_ptr<int8_t>(), rnorm.data_ptr<float>(), stream_of(dev))
+          : tq_prod_quantize_qjl_matrix(
+                cptr<float>(x), n, dim, padded_dim, bits, cptr<float>(signs), b.data(), c.data(),
+                cptr<float>(s_hi), packed.data_ptr<uint8_t>(), norms.data_ptr<float>(),
+                z.data_ptr<int8_t>(), rnorm.data_ptr<float>(), stream_of(dev));
   if (rc != 0) return std::nullopt;
   return std::make_tuple(packed, norms, z, rnorm);
 }
 
-// ops.prod_dequantize_qjl (large: prod_dequantize_qjl_ws)
+// ops.prod_dequantize_qjl (large: prod_dequantize_qjl_ws; without st_lo:
+// prod_dequantize_qjl_matrix, st_hi S itself)
 OptTensor prod_dequantize_qjl(const Tensor& packed, const Tensor& norms, const Tensor& z,
                               const Tensor& rnorm, int64_t dim, int64_t padded_dim, int64_t bits,
                               const Tensor& signs, const std::vector<double>& centroids,
-                              const Tensor& st_hi, const Tensor& st_lo, bool large,
+                              const Tensor& st_hi, const OptTensor& st_lo, bool large,
                               const OptTensor& st_scale) {
   const c10::Device dev = packed.device();
   if (!codes(packed, norms, padded_dim, bits, dev) || dim < 1 || !is_f32(rnorm, dev) ||
@@ -422,7 +435,7 @@ OptTensor prod_dequantize_qjl(const Tensor& packed, const Tensor& norms, const T
       z.dim() != packed.dim() || z.size(-1) != dim ||
       z.sizes().slice(0, z.dim() - 1) != norms.sizes() || !z.is_contiguous() || !aligned(z, 16) ||
       !is_f32(signs, dev) || signs.numel() < padded_dim || !aligned(signs, 16) ||
-      !halves(st_hi, padded_dim, dev) || !halves(st_lo, padded_dim, dev) ||
+      !matrix_or_halves(st_hi, st_lo, dim, padded_dim, large, dev) ||
       (int64_t)centroids.size() != (1 << bits) ||
       (st_scale.has_value() &&
        (!large || !is_f32(*st_scale, dev) || st_scale->numel() < padded_dim)))
@@ -435,14 +448,19 @@ OptTensor prod_dequantize_qjl(const Tensor& packed, const Tensor& norms, const T
       large ? tq_prod_dequantize_qjl_ws(
                   cptr<uint8_t>(packed), cptr<float>(norms), cptr<int8_t>(z), cptr<float>(rnorm),
                   norms.numel(), dim, padded_dim, bits, cptr<float>(signs), c.data(),
-                  st_hi.const_data_ptr(), st_lo.const_data_ptr(),
+                  st_hi.const_data_ptr(), st_lo->const_data_ptr(),
                   st_scale.has_value() ? cptr<float>(*st_scale) : nullptr, out.data_ptr<float>(),
                   stream_of(dev))
-            : tq_prod_dequantize_qjl(
-                  cptr<uint8_t>(packed), cptr<float>(norms), cptr<int8_t>(z), cptr<float>(rnorm),
-                  norms.numel(), dim, padded_dim, bits, cptr<float>(signs), c.data(),
-                  st_hi.const_data_ptr(), st_lo.const_data_ptr(), out.data_ptr<float>(),
-                  stream_of(dev));
+      : st_lo.has_value()
+          ? tq_prod_dequantize_qjl(
+                cptr<uint8_t>(packed), cptr<float>(norms), cptr<int8_t>(z), cptr<float>(rnorm),
+                norms.numel(), dim, padded_dim, bits, cptr<float>(signs), c.data(),
+                st_hi.const_data_ptr(), st_lo->const_data_ptr(), out.data_ptr<float>(),
+                stream_of(dev))
+          : tq_prod_dequantize_qjl_matrix(
+                cptr<uint8_t>(packed), cptr<float>(norms), cptr<int8_t>(z), cptr<float>(rnorm),
+                norms.numel(), dim, padded_dim, bits, cptr<float>(signs), c.data(),
+                cptr<float>(st_hi), out.data_ptr<float>(), stream_of(dev));
   if (rc != 0) return std::nullopt;
   return out;
 }

@@ -701,6 +701,14 @@ def prod_quantize_qjl(x: torch.Tensor, padded_dim: int, mse_bit_width: int,
                               s_lo, False)
 
 
+def prod_quantize_qjl_matrix(x: torch.Tensor, padded_dim: int, mse_bit_width: int,
+                             signs: torch.Tensor, boundaries, centroids, s: torch.Tensor):
+    """prod_quantize_qjl from the QJL matrix itself, fp32 [dim, dim]
+    (tq_prod_quantize_qjl_matrix): nothing made from it to keep or go stale."""
+    return _prod_quantize_qjl(x, padded_dim, mse_bit_width, signs, boundaries, centroids, s, None,
+                              False)
+
+
 def prod_quantize_qjl_ws(x: torch.Tensor, padded_dim: int, mse_bit_width: int,
                          signs: torch.Tensor, boundaries, centroids, s_hi: torch.Tensor,
                          s_lo: torch.Tensor):
@@ -711,6 +719,22 @@ def prod_quantize_qjl_ws(x: torch.Tensor, padded_dim: int, mse_bit_width: int,
                               s_lo, True)
 
 
+def _qjl_operands(hi, lo, dim, padded_dim, what):
+    """The QJL operand as the library takes it: two halves, or (lo None) the
+    matrix itself."""
+    if lo is None:
+        if hi.dtype != torch.float32 or tuple(hi.shape) != (dim, dim):
+            raise RuntimeError(f"{what} must be fp32 [dim, dim]")
+        return (_aligned16(hi),)
+    _require_gpu(hi, lo)
+    for t in (hi, lo):
+        if t.dtype != torch.float16 or tuple(t.shape) != (padded_dim, padded_dim) \
+                or not t.is_contiguous() or t.data_ptr() % 16:
+            raise RuntimeError(f"{what} halves must be contiguous aligned fp16 "
+                               "[padded_dim, padded_dim]")
+    return hi, lo
+
+
 def _prod_quantize_qjl(x, padded_dim, mse_bit_width, signs, boundaries, centroids, s_hi, s_lo,
                        large: bool):
     boundaries, centroids = _floats(boundaries), _floats(centroids)
@@ -718,14 +742,10 @@ def _prod_quantize_qjl(x, padded_dim, mse_bit_width, signs, boundaries, centroid
                                               centroids, s_hi, s_lo, large)
     if r is not None:
         return r
-    _require_gpu(x, signs, s_hi, s_lo)
+    _require_gpu(x, signs, s_hi)
     if x.dtype != torch.float32:
         raise RuntimeError("prod_quantize_qjl: x must be fp32")
-    for t in (s_hi, s_lo):
-        if t.dtype != torch.float16 or tuple(t.shape) != (padded_dim, padded_dim) \
-                or not t.is_contiguous() or t.data_ptr() % 16:
-            raise RuntimeError("prod_quantize_qjl: S halves must be contiguous aligned fp16 "
-                               "[padded_dim, padded_dim]")
+    operand = _qjl_operands(s_hi, s_lo, x.shape[-1], padded_dim, "prod_quantize_qjl: S")
     x = x.contiguous()
     if x.data_ptr() % 16:
         x = x.clone()
@@ -740,7 +760,7 @@ def _prod_quantize_qjl(x, padded_dim, mse_bit_width, signs, boundaries, centroid
     signs = _aligned16(signs)
     lib = _lib.load()
     args = (x.data_ptr(), n, dim, int(padded_dim), int(mse_bit_width), signs.data_ptr(),
-            _host_f32(boundaries), _host_f32(centroids), s_hi.data_ptr(), s_lo.data_ptr(),
+            _host_f32(boundaries), _host_f32(centroids), *(t.data_ptr() for t in operand),
             packed.data_ptr(), norms.data_ptr(), z.data_ptr(), rnorm.data_ptr())
     with torch.cuda.device(x.device):
         if large:
@@ -749,7 +769,8 @@ def _prod_quantize_qjl(x, padded_dim, mse_bit_width, signs, boundaries, centroid
             rc = lib.tq_prod_quantize_qjl_ws(*args, ws.data_ptr(), ws.numel(),
                                              _stream_ptr(x.device))
         else:
-            rc = lib.tq_prod_quantize_qjl(*args, _stream_ptr(x.device))
+            fn = lib.tq_prod_quantize_qjl_matrix if s_lo is None else lib.tq_prod_quantize_qjl
+            rc = fn(*args, _stream_ptr(x.device))
     _lib.check(rc, "prod_quantize_qjl")
     return packed, norms, z, rnorm
 
@@ -763,6 +784,16 @@ def prod_dequantize_qjl(packed: torch.Tensor, norms: torch.Tensor, qjl_signs: to
     halves of S^T."""
     return _prod_dequantize_qjl(packed, norms, qjl_signs, residual_norms, dim, padded_dim,
                                 mse_bit_width, signs, centroids, st_hi, st_lo, False)
+
+
+def prod_dequantize_qjl_matrix(packed: torch.Tensor, norms: torch.Tensor, qjl_signs: torch.Tensor,
+                               residual_norms: torch.Tensor, dim: int, padded_dim: int,
+                               mse_bit_width: int, signs: torch.Tensor, centroids,
+                               s: torch.Tensor) -> torch.Tensor:
+    """prod_dequantize_qjl from the QJL matrix itself, S (not S^T) fp32
+    [dim, dim] (tq_prod_dequantize_qjl_matrix)."""
+    return _prod_dequantize_qjl(packed, norms, qjl_signs, residual_norms, dim, padded_dim,
+                                mse_bit_width, signs, centroids, s, None, False)
 
 
 def prod_dequantize_qjl_ws(packed: torch.Tensor, norms: torch.Tensor, qjl_signs: torch.Tensor,
@@ -785,7 +816,7 @@ def _prod_dequantize_qjl(packed, norms, qjl_signs, residual_norms, dim, padded_d
                                                 st_lo, large, st_scale)
     if r is not None:
         return r
-    _require_gpu(packed, norms, qjl_signs, residual_norms, signs, st_hi, st_lo)
+    _require_gpu(packed, norms, qjl_signs, residual_norms, signs, st_hi)
     per = 2 if mse_bit_width == 3 else 8 // mse_bit_width
     if packed.dtype != torch.uint8 or packed.shape[-1] != padded_dim // per:
         raise RuntimeError("prod_dequantize_qjl: packed must be uint8 [..., padded_dim / per]")
@@ -794,11 +825,8 @@ def _prod_dequantize_qjl(packed, norms, qjl_signs, residual_norms, dim, padded_d
         raise RuntimeError("prod_dequantize_qjl: norms must match packed's leading dims")
     if qjl_signs.dtype != torch.int8 or tuple(qjl_signs.shape) != (*lead, dim):
         raise RuntimeError("prod_dequantize_qjl: qjl_signs must be int8 [..., dim]")
-    for t in (st_hi, st_lo):
-        if t.dtype != torch.float16 or tuple(t.shape) != (padded_dim, padded_dim) \
-                or not t.is_contiguous() or t.data_ptr() % 16:
-            raise RuntimeError("prod_dequantize_qjl: S^T halves must be contiguous aligned "
-                               "fp16 [padded_dim, padded_dim]")
+    operand = _qjl_operands(st_hi, st_lo, dim, padded_dim,
+                                "prod_dequantize_qjl: S" + ("" if st_lo is None else "^T"))
     if st_scale is not None:
         _require_gpu(packed, st_scale)
         if st_scale.dtype != torch.float32 or st_scale.numel() < padded_dim \
@@ -816,13 +844,14 @@ def _prod_dequantize_qjl(packed, norms, qjl_signs, residual_norms, dim, padded_d
     with torch.cuda.device(packed.device):
         args = (packed.data_ptr(), nf.data_ptr(), z.data_ptr(), rn.data_ptr(), nf.numel(),
                 int(dim), int(padded_dim), int(mse_bit_width), signs.data_ptr(),
-                _host_f32(centroids), st_hi.data_ptr(), st_lo.data_ptr())
+                _host_f32(centroids), *(t.data_ptr() for t in operand))
         tail = (out.data_ptr(), _stream_ptr(packed.device))
         if large:
             rc = lib.tq_prod_dequantize_qjl_ws(
                 *args, None if st_scale is None else st_scale.data_ptr(), *tail)
         else:
-            rc = lib.tq_prod_dequantize_qjl(*args, *tail)
+            fn = lib.tq_prod_dequantize_qjl_matrix if st_lo is None else lib.tq_prod_dequantize_qjl
+            rc = fn(*args, *tail)
     _lib.check(rc, "prod_dequantize_qjl")
     return out
 
