@@ -39,7 +39,8 @@
 //  * The requests of a scheduler step run as one launch of work items (batch
 //    mode, tq_prefill_attention_batch): five prompts of 229 .. 1326 tokens at
 //    32 q heads take 52 us where five launches with their key splits and
-//    merges took 125 us, two chunks over 5000-token contexts 138 against 175.
+//    merges took 125 us, chunks of 309 and 867 tokens over 5000 cached 140 against
+//    175.
 //  * Short chunks over long contexts (too few query blocks to fill the
 //    CUs): each query block's tiles are split over several workgroups
 //    (grid z), which leave their normalised O (fp16), reference max and row
@@ -264,10 +265,11 @@ __device__ __forceinline__ PrefillWork prefill_work(const PrefillBatch& p) {
 // head = blockIdx.x the q heads of one kv head land on different XCDs and each
 // of their L2s fetches the same K and V; taken this way an XCD serves
 // consecutive heads, one kv head at 32 / 8.  Where few rows meet many keys that
-// traffic is what bounds the kernel: 256 rows over 32,512 keys 168 -> 147 us, four
-// chunks of 300 over 8,000 with 64 / 8 heads 479 -> 397, six prompts of 1,300 121
-// -> 112, a 32k prompt 7.70 -> 7.67 ms, nothing slower.  Head counts off the 8
-// XCDs keep the plain order (no head order keeps them apart).
+// traffic is what bounds the kernel: 256 rows over 32,512 keys 168 -> 147 us (with
+// fp16 partials then; 150 .. 153 with the fp32 ones of today), four chunks of 300
+// over 8,000 with 64 / 8 heads 479 -> 397, six prompts of 1,300 121 -> 112; a 32k
+// prompt is the same within noise, nothing slower.  Head counts off the 8 XCDs
+// keep the plain order (no head order keeps them apart).
 __device__ __forceinline__ int head_of_block() {
   const int x = blockIdx.x, hq = gridDim.x;
   return (hq & 7) == 0 ? (x & 7) * (hq >> 3) + (x >> 3) : x;

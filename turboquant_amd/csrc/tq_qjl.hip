@@ -15,10 +15,10 @@
 //    rounding of an fp32 sum of these terms.
 //  * dequantize: X = z (int8, exact in fp16), W = S^T; two products.
 // Each row of W comes scaled by a power of two that takes its largest entry to
-// [2^14, 2^15) (qjl_operand), so that S has fp32's range here too and lo is
-// normal for every entry down to 2^-17 of its row's largest: without the scale
-// 5% of a Gaussian S (|S| < 0.12) had a lo of fewer bits.  A sign does not see
-// the scale; the dequantize takes it out of the sum, exactly.
+// [2^14, 2^15) (qjl_operand), so that S has fp32's range here too and hi + lo its
+// 22 bits for every entry down to 2^-17 of its row's largest: without the scale
+// 10% of a Gaussian S (|S| < 2^-3) had a subnormal lo of fewer bits.  A sign does
+// not see the scale; the dequantize takes it out of the sum, exactly.
 // The halves of one K step feed 12 (8) MFMAs from 8 (6) LDS reads, so the
 // kernels are MFMA-bound where a plain fp16 product of this tile is
 // LDS-bound.  Tiles are copied with direct-to-LDS loads, 16-byte chunks
@@ -469,8 +469,8 @@ __global__ __launch_bounds__(256) void operand_rows_kernel(const float* __restri
 // column tid % 32, rows tid / 32 + 32 i, all loads in flight) for their scales
 // and writes every eighth 32 x 32 tile of them as rows of W, through LDS.
 // Eight workgroups read the same strip (out of L2) so that the few strips do
-// not leave most CUs idle: dim 1024 6.3 us
-// with the launch, 9.8 with one workgroup per strip (W = S 3.7 us).
+// not leave most CUs idle: dim 1024 6.3 us with the launch, 9.8 with one
+// workgroup per strip (W = S 3.7 us).
 __global__ __launch_bounds__(1024) void operand_cols_kernel(const float* __restrict__ s, int dim,
                                                             int pd, _Float16* __restrict__ out,
                                                             float* __restrict__ scales) {
@@ -520,7 +520,8 @@ hipError_t launch_qjl(bool quant, const _Float16* xh, const _Float16* xl, const 
   // The form by the number of tiles.  Up to one 32 x 32 tile per CU the split-K
   // kernel: quantize, dim 1000, n = 16 / 256 / 512 16.6 / 19.3 / 29 us against 22.8
   // / 24 / 26.5 with 64 x 64 tiles and 31.5 / 33.2 / 34 with 128 x 128 (the whole
-  // call; the products alone 8 against 23 us at n = 16).  Then 64 x 64 tiles while
+  // call but for the 4 .. 6 us of the operand's launch; the products alone 8
+  // against 23 us at n = 16).  Then 64 x 64 tiles while
   // few enough to fill a round or two of the card: 2.5 per CU for the quantize (n
   // = 2500 41.3 against 43.5, n = 4096 60 against 50; dim 256, n = 8192 19.8
   // against 22.0), 5 for the dequantize, more of which fit a CU (dim 1000, n =

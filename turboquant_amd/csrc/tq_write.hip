@@ -128,8 +128,8 @@ __device__ __forceinline__ float xor_lane(float x) {
 //
 // With 16 lanes per vector a small launch has four times the waves of the
 // fast kernel below and a quarter of the work in each: K and V of 8 tokens x 8
-// heads x 128 take 3.3 us against 4.0 us, 512 tokens 3.8 against 4.3, 1024
-// tokens 5.1 against 4.7 (so up to kSmallWrite vectors).  Above that it serves
+// heads x 128 take 3.5 us against 4.0 us, 512 tokens 4.1 against 4.25, 1024
+// tokens 5.15 against 4.5 (graph replays; so up to kSmallWrite vectors).  Above that it serves
 // the rows that the fast kernel cannot load.
 //
 // sign_first: the signs are flipped before the squares, which leaves a NaN
@@ -343,9 +343,9 @@ __global__ __launch_bounds__(256) void write_kernel(
 //    overflows on finite bf16 or fp32 inputs gives inv = 0, all codes 8.)
 //
 // VALU-bound (about 20 instructions per coordinate): 8192 tokens x 8 heads x
-// 128, K and V, 14.3 us for fp16 (3.0 TB/s), 13.4 for bf16 and 16.8 for fp32
+// 128, K and V, 13.4 us for fp16 (3.2 TB/s), 12.9 for bf16 and 16.6 for fp32
 // rows; in the general kernel, whose bf16 and fp32 loads were single elements,
-// 23.3, 24.2 and 22.2 us.
+// 23.3, 24.2 and 22.2 us (with that kernel's vector loads 23.0, 21.1 and 21.6).
 template <int PD>
 struct FastGeom {
   // 16-byte chunks (8 dims) per lane: 4, and 2 at pd 64, where 4 would leave
